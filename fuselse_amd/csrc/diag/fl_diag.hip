@@ -178,6 +178,8 @@ __device__ __forceinline__ void put_block_record(uint64_t* rec, int64_t i, uint6
 // The forward's row output with a record per row: begin() runs on the row's
 // first thread before its loads, end() once the row's LSE is known.
 struct TimedLseOut {
+    using Map = fl::PackedRows;
+    static constexpr fl::PackedRows map{};
     float* __restrict__ out;
     uint64_t* __restrict__ rec;
     struct Row {

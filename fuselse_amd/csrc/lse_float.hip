@@ -40,9 +40,9 @@ namespace fl {
 // row merges needs a device-scope release per block, which on this GPU writes
 // back the XCD's L2 each time and measured slower than the second launch.)
 // ---------------------------------------------------------------------------
-template <typename T, bool ROBUST, int THREADS, int U>
-__global__ __launch_bounds__(THREADS) void lse_fwd_split_partials(const T* __restrict__ x, int64_t N, int64_t seg,
-                                                                  float2* __restrict__ part) {
+template <typename T, bool ROBUST, int THREADS, int U, typename MAP>
+__global__ __launch_bounds__(THREADS) void lse_fwd_split_partials(const T* __restrict__ x, MAP map, int64_t N,
+                                                                  int64_t seg, float2* __restrict__ part) {
     constexpr int VE = Elem<T>::kVec;
     constexpr int WAVES = THREADS / 64;
     __shared__ float sh_m[WAVES], sh_s[WAVES];
@@ -50,7 +50,7 @@ __global__ __launch_bounds__(THREADS) void lse_fwd_split_partials(const T* __res
     const int S = (int)gridDim.x;
     const int k = (int)blockIdx.x;
     const int64_t row = blockIdx.y;
-    const T* p = x + row * N;
+    const T* p = x + map.offset(row, N);
     const RowSplit sp = split_row(p, N);
     float m = -kInf, s = 0.0f;
     if (k == 0) {
@@ -156,8 +156,8 @@ static void launch_split_merge(const float2* part, OUT out, int64_t B, int S, hi
 template <typename T, bool ROBUST, int THREADS, int U, typename OUT>
 static void launch_split(const T* x, OUT out, int64_t B, int64_t N, const SplitPlan& pl, void* ws, hipStream_t st) {
     float2* part = static_cast<float2*>(ws);
-    lse_fwd_split_partials<T, ROBUST, THREADS, U>
-        <<<dim3((unsigned)pl.S, (unsigned)B), dim3(THREADS), 0, st>>>(x, N, pl.seg, part);
+    lse_fwd_split_partials<T, ROBUST, THREADS, U, typename OUT::Map>
+        <<<dim3((unsigned)pl.S, (unsigned)B), dim3(THREADS), 0, st>>>(x, out.map, N, pl.seg, part);
     launch_split_merge<ROBUST>(part, out, B, (int)pl.S, st);
 }
 
@@ -283,7 +283,7 @@ static void launch_fwd(const T* x, OUT out, int64_t B, int64_t N, hipStream_t st
     if (vecs < 16) {
         // a few vectors per row: 4 lanes per row, one masked batch of 2
         // (22% ahead of the burst loop at 8 vectors)
-        launch_group<T, ROBUST, 4, 2, true, OUT>(x, out, B, N, st);
+        launch_group<T, ROBUST, 4, 2, !OUT::Map::kSliced, OUT>(x, out, B, N, st);
         return;
     }
     // Short rows: LPR lanes per row, about 4 vectors per lane in one burst.
@@ -542,6 +542,75 @@ __global__ __launch_bounds__(64) void lse_bwd_flat(const float* __restrict__ g, 
     Elem<T>::put_vec_buf(ry, l * 16, vals);
 }
 
+// x and grad_x on different 16-byte phases: x starts off the vectors' grid (a
+// view of another matrix) or comes in slices (SlicedRows) whose gradient is
+// packed.  The flat kernel's walk over grad_x, with aligned 16-byte stores; a
+// lane's x vector lies at the same place of its own slice, and is loaded from
+// wherever that is (element-aligned 16-byte loads, plain ones: neighbouring
+// waves share a cache line at each end, and nt loads took 1% more).  A vector
+// that spans two rows, or the matrix's end, goes element by element.  Bound by
+// memory: the gradient of fp32 (8 x 1023, 50257) cut from 8 x 1024 rows moves
+// 3.29 GB in about 525 us; a launch per slice took 6 x 146 + 2 x 65 us, six of
+// them in the scalar kernel below, whose slice and gradient differ in phase.
+template <typename T, typename GR>
+__global__ __launch_bounds__(64) void lse_bwd_flat_shifted(const float* __restrict__ g, const T* __restrict__ x,
+                                                           const float* __restrict__ lse, T* __restrict__ gx,
+                                                           int64_t N, int64_t total, int64_t slice_rows,
+                                                           int64_t slice_skip, GR gr_t, int64_t block0) {
+    constexpr int VE = Elem<T>::kVec;
+    typedef u32x4 __attribute__((aligned(4))) u32x4_a4;
+    typedef u32x4 __attribute__((aligned(2))) u32x4_a2;
+    const int64_t e0 = (block0 + (int64_t)blockIdx.x) * (64 * VE);
+    const int64_t row0 = div_rows(e0, N);
+    const int64_t slice0 = div_rows(row0, slice_rows);
+    const int64_t e = e0 + (int64_t)threadIdx.x * VE;
+    if (e >= total) return;
+    int64_t col = e - row0 * N;
+    int64_t row = row0, slice = slice0;
+    if (N >= 64 * VE) {  // at most one row end, so one slice end, per wave
+        if (col >= N) {
+            row += 1;
+            col -= N;
+            slice += row == (slice0 + 1) * slice_rows;
+        }
+    } else {
+        const uint32_t r = (uint32_t)col / (uint32_t)N;  // col < N + 64 * VE here
+        row += r;
+        col -= (int64_t)r * N;
+        slice = div_rows(row, slice_rows);
+    }
+    const T* xe = x + e + slice * slice_skip;
+    const int64_t left = total - e0;
+    const __amdgpu_buffer_rsrc_t ry = __builtin_amdgcn_make_buffer_rsrc(
+        gx + e0, 0, (left < 64 * VE ? (int)left : 64 * VE) * (int)sizeof(T), 0x00020000);
+    if (col + VE <= N) {
+        const float g0 = g[row];
+        const float lv = lse[row];
+        float v[VE];
+        if constexpr (sizeof(T) == 4)
+            Elem<T>::cvt(*reinterpret_cast<const u32x4_a4*>(xe), v);
+        else
+            Elem<T>::cvt(*reinterpret_cast<const u32x4_a2*>(xe), v);
+        bwd_vals<VE>(gr_t.coef(row, g0), lv, __builtin_fabsf(lv) < 64.0f, v);
+        add_at<GR::kSel, VE>(v, col, gr_t.target(row), g0);
+        Elem<T>::put_vec_buf(ry, (int)threadIdx.x * 16, v);
+        return;
+    }
+    for (int k = 0; k < VE && e + k < total; ++k) {
+        const float g0 = g[row];
+        const float t = bwd_elem(gr_t.coef(row, g0), lse[row], Elem<T>::scalar(xe + k));
+        Elem<T>::put(gx + e + k, t + (GR::kSel && col == gr_t.target(row) ? g0 : 0.0f));
+        if (++col == N) {
+            col = 0;
+            row += 1;
+            if (row == (slice + 1) * slice_rows) {
+                slice += 1;
+                xe += slice_skip;
+            }
+        }
+    }
+}
+
 // Short rows: LPR lanes per row, 256/LPR rows per block, grid-stride.
 template <typename T, int LPR, typename GR, bool BUF>
 __global__ __launch_bounds__(256) void lse_bwd_group_rows(const float* __restrict__ g, const T* __restrict__ x,
@@ -568,18 +637,19 @@ __global__ __launch_bounds__(256) void lse_bwd_group_rows(const float* __restric
     }
 }
 
-// Fallback when x and grad_x differ in 16-byte alignment: scalar grid-stride.
+// Fallback when x and grad_x differ in 16-byte alignment and grad_x is off the
+// vectors' grid: scalar grid-stride.
 template <typename T, typename GR>
 __global__ __launch_bounds__(256) void lse_bwd_scalar(const float* __restrict__ g, const T* __restrict__ x,
                                                       const float* __restrict__ lse, T* __restrict__ gx,
-                                                      int64_t B, int64_t N, GR gr_t) {
+                                                      int64_t B, int64_t N, SlicedRows map, GR gr_t) {
     for (int64_t row = blockIdx.y; row < B; row += gridDim.y) {
         const float g0 = g[row];
         const float gv = gr_t.coef(row, g0);
         const int64_t t = gr_t.target(row);
         const float lv = lse[row];
         for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < N; i += (int64_t)gridDim.x * 256)
-            bwd_one<T, GR>(gx + row * N, x + row * N, i, gv, lv, t, g0);
+            bwd_one<T, GR>(gx + row * N, x + map.offset(row, N), i, gv, lv, t, g0);
     }
 }
 
@@ -658,15 +728,32 @@ static void launch_bwd_vec(const float* g, const T* x, const float* lse, T* gx, 
     }
 }
 
+// x in slices of slice_rows rows, slice_skip elements apart (one slice of B
+// rows: packed), grad_x packed; any alignment of either.
+template <typename T, typename GR>
+static void launch_bwd_shifted(const float* g, const T* x, const float* lse, T* gx, int64_t B, int64_t N,
+                               int64_t slice_rows, int64_t slice_skip, GR gr_t, hipStream_t st) {
+    if (reinterpret_cast<uintptr_t>(gx) & 15u) {
+        int64_t gxdim = (N + 255) / 256;
+        if (gxdim > 1024) gxdim = 1024;
+        int64_t gydim = B < 65535 ? B : 65535;
+        lse_bwd_scalar<T><<<dim3((unsigned)gxdim, (unsigned)gydim), dim3(256), 0, st>>>(
+            g, x, lse, gx, B, N, SlicedRows{slice_rows, slice_skip}, gr_t);
+        return;
+    }
+    constexpr int64_t kPerBlock = 64 * Elem<T>::kVec;
+    for_grid_chunks((B * N + kPerBlock - 1) / kPerBlock, 64, [&](int64_t b0, int64_t nb) {
+        lse_bwd_flat_shifted<T, GR><<<dim3((unsigned)nb), dim3(64), 0, st>>>(g, x, lse, gx, N, B * N, slice_rows,
+                                                                             slice_skip, gr_t, b0);
+    });
+}
+
 template <typename T, typename GR>
 static void launch_bwd(const float* g, const T* x, const float* lse, T* gx, int64_t B, int64_t N, GR gr_t,
                        hipStream_t st) {
     const bool same_align = ((reinterpret_cast<uintptr_t>(x) ^ reinterpret_cast<uintptr_t>(gx)) & 15u) == 0;
     if (!same_align) {
-        int64_t gxdim = (N + 255) / 256;
-        if (gxdim > 1024) gxdim = 1024;
-        int64_t gydim = B < 65535 ? B : 65535;
-        lse_bwd_scalar<T><<<dim3((unsigned)gxdim, (unsigned)gydim), dim3(256), 0, st>>>(g, x, lse, gx, B, N, gr_t);
+        launch_bwd_shifted<T>(g, x, lse, gx, B, N, B, 0, gr_t, st);
         return;
     }
     // buffer stores take 32-bit offsets: rows of 2 GiB or more keep pointer stores
@@ -834,8 +921,20 @@ extern "C" int fl_selective_logsoftmax_f32(const float* x, const int64_t* index,
     FL_CHECK(B >= 0 && N >= 0, "%s: negative shape (B=%lld, N=%lld)", name, (long long)B, (long long)N);
     if (B == 0) return ok();
     FL_CHECK(index != nullptr && logp != nullptr, "%s: NULL pointer argument", name);
-    return fwd_launch<float>(name, x, SelectOut<float>{x, index, logp, lse, N}, B, N, robust, workspace,
+    return fwd_launch<float>(name, x, SelectOut<float>{{}, x, index, logp, lse, N}, B, N, robust, workspace,
                              workspace_bytes, reinterpret_cast<hipStream_t>(stream));
+}
+
+extern "C" int fl_selective_logsoftmax_slices_f32(const float* x, const int64_t* index, float* logp, float* lse,
+                                                  int64_t B, int64_t N, int64_t slice_rows, int64_t slice_skip,
+                                                  int robust, void* workspace, size_t workspace_bytes, void* stream) {
+    const char* name = "fl_selective_logsoftmax_slices_f32";
+    FL_CHECK(B >= 0 && N >= 0, "%s: negative shape (B=%lld, N=%lld)", name, (long long)B, (long long)N);
+    if (B == 0) return ok();
+    FL_CHECK(slice_rows > 0, "%s: slices of %lld rows", name, (long long)slice_rows);
+    FL_CHECK(index != nullptr && logp != nullptr, "%s: NULL pointer argument", name);
+    return fwd_launch<float>(name, x, SelectOut<float, SlicedRows>{{slice_rows, slice_skip}, x, index, logp, lse, N}, B,
+                             N, robust, workspace, workspace_bytes, reinterpret_cast<hipStream_t>(stream));
 }
 
 extern "C" int fl_selective_logsoftmax_bwd_f32(const float* grad, const float* x, const int64_t* index,
@@ -843,4 +942,20 @@ extern "C" int fl_selective_logsoftmax_bwd_f32(const float* grad, const float* x
     const char* name = "fl_selective_logsoftmax_bwd_f32";
     FL_CHECK(index != nullptr || B == 0 || N == 0, "%s: NULL pointer argument", name);
     return bwd_entry<float>(name, grad, x, lse, grad_x, B, N, SelGrad{index}, stream);
+}
+
+extern "C" int fl_selective_logsoftmax_slices_bwd_f32(const float* grad, const float* x, const int64_t* index,
+                                                      const float* lse, float* grad_x, int64_t B, int64_t N,
+                                                      int64_t slice_rows, int64_t slice_skip, void* stream) {
+    const char* name = "fl_selective_logsoftmax_slices_bwd_f32";
+    FL_CHECK(B >= 0 && N >= 0, "%s: negative shape (B=%lld, N=%lld)", name, (long long)B, (long long)N);
+    if (B == 0 || N == 0) return ok();
+    FL_CHECK(slice_rows > 0, "%s: slices of %lld rows", name, (long long)slice_rows);
+    FL_CHECK(grad && x && lse && grad_x && index, "%s: NULL pointer argument", name);
+    FL_CHECK((reinterpret_cast<uintptr_t>(x) % sizeof(float)) == 0 &&
+                 (reinterpret_cast<uintptr_t>(grad_x) % sizeof(float)) == 0,
+             "%s: x / grad_x are not element-aligned", name);
+    launch_bwd_shifted(grad, x, lse, grad_x, B, N, slice_rows, slice_skip, SelGrad{index},
+                       reinterpret_cast<hipStream_t>(stream));
+    return launch_status(name);
 }

@@ -212,7 +212,32 @@ __device__ __forceinline__ int64_t batches(int64_t n) {
 // the lane that later calls end(row, r, lse), so a policy's own loads are in
 // flight during the row's reduction.
 // ---------------------------------------------------------------------------
+// Where a forward's rows lie: row r starts at element offset(r, N) of x.
+// Sliced rows come in runs of `rows` contiguous rows with `skip` further
+// elements between one run's end and the next run's start (a batch whose last
+// positions are cut off, logits[:, :-1]).
+struct PackedRows {
+    static constexpr bool kSliced = false;
+    __device__ __forceinline__ int64_t offset(int64_t row, int64_t N) const { return row * N; }
+    // the runs start on the same 16-byte phase, for elements of E bytes
+    __device__ __forceinline__ bool same_phase(int64_t) const { return true; }
+};
+__device__ __forceinline__ int64_t div_rows(int64_t a, int64_t b) {
+    // a 64-bit division is about 100 instructions; almost every size fits 32
+    return ((uint64_t)a | (uint64_t)b) >> 32 ? a / b : (int64_t)((uint32_t)a / (uint32_t)b);
+}
+struct SlicedRows {
+    static constexpr bool kSliced = true;
+    int64_t rows, skip;
+    __device__ __forceinline__ int64_t offset(int64_t row, int64_t N) const {
+        return row * N + div_rows(row, rows) * skip;
+    }
+    __device__ __forceinline__ bool same_phase(int64_t E) const { return (skip * E) % 16 == 0; }
+};
+
 struct LseOut {
+    using Map = PackedRows;
+    static constexpr PackedRows map{};
     float* __restrict__ out;
     struct Row {};
     __device__ __forceinline__ Row begin(int64_t) const { return {}; }
@@ -223,8 +248,10 @@ struct LseOut {
 // when lse is not NULL.  An index outside [0, N) gives NaN (torch.gather would
 // raise); the special values follow from the robust LSE (a +inf target in a
 // row whose LSE is +inf gives NaN, as torch.log_softmax does).
-template <typename T>
+template <typename T, typename MAP = PackedRows>
 struct SelectOut {
+    using Map = MAP;
+    MAP map;
     const T* __restrict__ x;
     const int64_t* __restrict__ index;
     float* __restrict__ logp;
@@ -235,7 +262,7 @@ struct SelectOut {
     };
     __device__ __forceinline__ Row begin(int64_t row) const {
         const int64_t t = index[row];
-        return {t >= 0 && t < N ? Elem<T>::scalar(x + row * N + t) : __builtin_nanf("")};
+        return {t >= 0 && t < N ? Elem<T>::scalar(x + map.offset(row, N) + t) : __builtin_nanf("")};
     }
     __device__ __forceinline__ void end(int64_t row, Row r, float l) const {
         if (lse) lse[row] = l;
@@ -256,7 +283,7 @@ __global__ __launch_bounds__(THREADS) void lse_fwd_block_rows(const T* __restric
     for (int64_t row = blockIdx.x; row < B; row += gridDim.x) {
         typename OUT::Row orow{};
         if (tid == 0) orow = out.begin(row);
-        const T* p = x + row * N;
+        const T* p = x + out.map.offset(row, N);
         const RowSplit sp = split_row(p, N);
         float m = -kInf, s = 0.0f;
         if (tid < sp.head) fold_scalar<T, ROBUST>(m, s, p + tid);
@@ -295,6 +322,7 @@ __global__ __launch_bounds__(THREADS) void lse_fwd_block_rows(const T* __restric
 // (grid-stride over row groups).
 template <typename T, bool ROBUST, int LPR, int U, bool PIPE, typename OUT>
 __global__ __launch_bounds__(256) void lse_fwd_group_rows(const T* __restrict__ x, OUT out, int64_t B, int64_t N) {
+    static_assert(!(PIPE && OUT::Map::kSliced), "the pipelined loop addresses a wave's rows as one run");
     constexpr int VE = Elem<T>::kVec;
     constexpr int RPW = 64 / LPR;
     constexpr int WAVES = 4;
@@ -314,7 +342,8 @@ __global__ __launch_bounds__(256) void lse_fwd_group_rows(const T* __restrict__ 
     // whole bursts for every lane of the wave: with x 16-byte aligned and rows
     // of whole vectors every body holds N / VE vectors, otherwise at least
     // (N - VE + 1) / VE whatever its alignment
-    const bool whole_rows = (reinterpret_cast<uintptr_t>(x) & 15u) == 0 && (N * E) % 16 == 0;
+    const bool whole_rows =
+        (reinterpret_cast<uintptr_t>(x) & 15u) == 0 && (N * E) % 16 == 0 && out.map.same_phase(E);
     const int64_t nv_lo = whole_rows ? N / VE : (N >= VE - 1 ? (N - VE + 1) / VE : 0);
     const int64_t nfull = nv_lo / ((int64_t)U * LPR);
     for (int64_t base = ((int64_t)blockIdx.x * WAVES + wave) * RPW; base < B; base += step) {
@@ -323,7 +352,7 @@ __global__ __launch_bounds__(256) void lse_fwd_group_rows(const T* __restrict__ 
         if (j == 0 && row < B) orow = out.begin(row);
         float m = -kInf, s = 0.0f;
         if (row < B) {
-            const T* p = x + row * N;
+            const T* p = x + out.map.offset(row, N);
             const RowSplit sp = split_row(p, N);
             for (int64_t h = j; h < sp.head; h += LPR) fold_scalar<T, ROBUST>(m, s, p + h);
             const T* tail = p + sp.head + sp.nvec * VE;

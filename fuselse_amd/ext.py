@@ -241,6 +241,63 @@ def selective_log_softmax_float_backward(grad_output: torch.Tensor, logits: torc
     return grad
 
 
+def _slices_shape(logits: torch.Tensor):
+    """(rows B, N, rows per slice, elements between slices) of 3-D logits whose
+    rows are contiguous within each leading index."""
+    _check(logits.dim() == 3, "logits must be 3D (batch, rows, N)")
+    n0, n1, N = logits.shape
+    _check(n0 >= 1 and n1 >= 1 and N >= 1, "logits must not be empty")
+    skip = logits.stride(0) - n1 * N if n0 > 1 else 0
+    _check(logits.stride(2) == 1 and logits.stride(1) == N, "logits must hold contiguous rows in each slice")
+    return n0 * n1, N, n1, skip
+
+
+def selective_log_softmax_slices_float(logits: torch.Tensor, index: torch.Tensor, robust: bool = True):
+    """selective_log_softmax_float of 3-D fp32 logits (batch, rows, N) whose
+    rows are contiguous within each leading index (logits[:, :-1] of a
+    contiguous tensor), in one launch and without a copy; index int64
+    (batch * rows,).  Returns (logp, lse) of that length."""
+    _check(logits.is_cuda, "logits must be CUDA")
+    _check(index.is_cuda, "index must be CUDA")
+    _check(logits.dtype == torch.float32, "logits must be float32")
+    _check(index.dtype == torch.int64, "index must be int64")
+    B, N, slice_rows, skip = _slices_shape(logits)
+    _check(index.dim() == 1 and index.is_contiguous() and index.size(0) == B,
+           "index must be a contiguous 1D tensor with one entry per row")
+    _check_device(logits, "logits", index=index)
+    logp = torch.empty((B,), dtype=torch.float32, device=logits.device)
+    lse = torch.empty((B,), dtype=torch.float32, device=logits.device)
+    with _on_device(logits):
+        nbytes = _workspace_bytes(B, N, 4)
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=logits.device) if nbytes else None
+        _lib.call("fl_selective_logsoftmax_slices_f32", logits.data_ptr(), index.data_ptr(), logp.data_ptr(),
+                  lse.data_ptr(), B, N, slice_rows, skip, int(robust), ws.data_ptr() if ws is not None else None,
+                  nbytes, _stream(logits))
+    return logp, lse
+
+
+def selective_log_softmax_slices_float_backward(grad_output: torch.Tensor, logits: torch.Tensor, index: torch.Tensor,
+                                                lse: torch.Tensor) -> torch.Tensor:
+    """selective_log_softmax_float_backward for logits in slices: the gradient,
+    contiguous, of logits' shape; grad_output, index and lse (batch * rows,)."""
+    for t, nm in ((grad_output, "grad_output"), (index, "index"), (lse, "lse")):
+        _check(t.is_cuda, f"{nm} must be CUDA")
+        _check(t.is_contiguous() and t.dim() == 1, f"{nm} must be contiguous and 1D")
+    _check(logits.is_cuda, "logits must be CUDA")
+    _check(logits.dtype == torch.float32 and grad_output.dtype == torch.float32 and lse.dtype == torch.float32,
+           "grad_output, logits and lse must be float32")
+    _check(index.dtype == torch.int64, "index must be int64")
+    B, N, slice_rows, skip = _slices_shape(logits)
+    _check(grad_output.size(0) == B and index.size(0) == B and lse.size(0) == B,
+           "grad_output, index and lse must hold one entry per row")
+    _check_device(logits, "logits", grad_output=grad_output, index=index, lse=lse)
+    grad = torch.empty(logits.shape, dtype=torch.float32, device=logits.device)
+    with _on_device(logits):
+        _lib.call("fl_selective_logsoftmax_slices_bwd_f32", grad_output.data_ptr(), logits.data_ptr(),
+                  index.data_ptr(), lse.data_ptr(), grad.data_ptr(), B, N, slice_rows, skip, _stream(logits))
+    return grad
+
+
 def _fwd_half(x: torch.Tensor, dtype: torch.dtype, entry: str, dtype_msg: str, robust: bool,
               keep: bool = False) -> torch.Tensor:
     # fused_fp16_kernel.cu:113-116

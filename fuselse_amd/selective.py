@@ -37,8 +37,17 @@ def _trl_algorithm(logits: torch.Tensor, index: torch.Tensor) -> torch.Tensor:
     return torch.stack(rows)
 
 
-# Most leading slices taken one launch each instead of copying the logits.
+# Most leading slices taken one launch each instead of copying the logits, for
+# an ext without the sliced entries.
 _MAX_SLICES = 64
+
+
+def _is_sliced(x: torch.Tensor) -> bool:
+    """3-D rows contiguous within each leading index but not as a whole (trl
+    takes the logits as logits[:, :-1, :], whose rows skip one row at every
+    leading index)."""
+    return x.dim() == 3 and x.numel() > 0 and x.stride(-1) == 1 and x.stride(1) == x.shape[-1] \
+        and not x.is_contiguous()
 
 
 def _row_slices(x: torch.Tensor):
@@ -58,11 +67,17 @@ def _row_slices(x: torch.Tensor):
 def make_selective_log_softmax(ext, original=None, robust: bool = True):
     fwd = ext.selective_log_softmax_float
     bwd = ext.selective_log_softmax_float_backward
+    fwd_sliced = getattr(ext, "selective_log_softmax_slices_float", None)
+    bwd_sliced = getattr(ext, "selective_log_softmax_slices_float_backward", None)
     fallback = original if original is not None else _trl_algorithm
 
     def forward_rows(logits, idx):
-        """(logp, lse, slices): one launch per contiguous slice of rows (a
-        copy of the logits only when they have none)."""
+        """(logp, lse, slices): one launch for contiguous or sliced rows (one
+        per contiguous slice when the ext has no sliced entries; a copy of the
+        logits only when their rows are neither)."""
+        if fwd_sliced is not None and _is_sliced(logits):
+            logp, lse = fwd_sliced(logits, idx, robust)
+            return logp, lse, [logits]
         slices = _row_slices(logits)
         if slices is None:
             slices = [logits.reshape(-1, logits.shape[-1]).contiguous()]
@@ -93,7 +108,14 @@ def make_selective_log_softmax(ext, original=None, robust: bool = True):
             idx, lse, *slices = ctx.saved_tensors
             g = grad_out.reshape(-1).to(torch.float32).contiguous()
             if len(slices) == 1:
-                return bwd(g, slices[0], idx, lse).reshape(ctx.in_shape), None
+                x = slices[0]
+                if x.dim() == 3:
+                    # logits saved as they came; a saved-tensor hook may have
+                    # given them back in another layout
+                    if _is_sliced(x):
+                        return bwd_sliced(g, x, idx, lse), None
+                    x = x.reshape(-1, x.shape[-1]).contiguous()
+                return bwd(g, x, idx, lse).reshape(ctx.in_shape), None
             grad = torch.empty(ctx.in_shape, dtype=torch.float32, device=lse.device)
             rows = grad.view(-1, ctx.in_shape[-1])
             r0 = 0

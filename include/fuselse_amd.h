@@ -71,6 +71,21 @@ int fl_selective_logsoftmax_bwd_f32(const float* grad, const float* x, const int
                                     float* grad_x, int64_t B, int64_t N, void* stream);
 
 /* ---------------------------------------------------------------------------
+ * The same over logits in slices, in one launch: row r of the B rows starts at
+ * x + r * N + (r / slice_rows) * slice_skip elements, i.e. every slice_rows
+ * contiguous rows are followed by slice_skip elements that are not read
+ * (logits[:, :-1] of a [batch, seq, N] tensor: slice_rows = seq - 1,
+ * slice_skip = N; negative where slices overlap).  index, logp, lse, grad are packed [B], grad_x packed
+ * [B, N].
+ * ------------------------------------------------------------------------- */
+int fl_selective_logsoftmax_slices_f32(const float* x, const int64_t* index, float* logp, float* lse, int64_t B,
+                                       int64_t N, int64_t slice_rows, int64_t slice_skip, int robust,
+                                       void* workspace, size_t workspace_bytes, void* stream);
+int fl_selective_logsoftmax_slices_bwd_f32(const float* grad, const float* x, const int64_t* index,
+                                           const float* lse, float* grad_x, int64_t B, int64_t N,
+                                           int64_t slice_rows, int64_t slice_skip, void* stream);
+
+/* ---------------------------------------------------------------------------
  * Half-precision inputs with fp32 accumulation and fp32 output [B].
  * fl_lse_fwd_f16 replaces batched_logsumexp_fp16 (fuselse/gpu/fused_fp16_kernel.cu:
  * 112-132; kernel :25-110).  fl_lse_fwd_bf16 is the bf16 twin, which the

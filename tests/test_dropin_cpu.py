@@ -304,6 +304,58 @@ def test_selective_takes_trl_slices_without_copying_the_logits():
     assert [c[1] for c in ext.calls] == [(12, 11)]
 
 
+class FakeSlicedExt(FakeSelExt):
+    """FakeSelExt with the sliced entries, which read rows by the address rule
+    the C entries document."""
+
+    @staticmethod
+    def _rows(logits):
+        lt = logits.as_subclass(torch.Tensor)
+        n0, n1, n = lt.shape
+        skip = lt.stride(0) - n1 * n if n0 > 1 else 0
+        at = torch.tensor([r * n + (r // n1) * skip for r in range(n0 * n1)])
+        flat = lt.as_strided((lt.untyped_storage().nbytes() // lt.element_size() - lt.storage_offset(),), (1,))
+        return flat[at[:, None] + torch.arange(n)].as_subclass(FakeCuda)
+
+    def selective_log_softmax_slices_float(self, logits, index, robust=True):
+        assert logits.dim() == 3 and logits.stride(2) == 1 and logits.stride(1) == logits.shape[2]
+        out = self.selective_log_softmax_float(self._rows(logits), index, robust)
+        self.calls[-1] = ("fwd sliced",) + self.calls[-1][1:]
+        return out
+
+    def selective_log_softmax_slices_float_backward(self, g, logits, index, lse):
+        grad = self.selective_log_softmax_float_backward(g, self._rows(logits), index, lse)
+        self.calls[-1] = ("bwd sliced",) + self.calls[-1][1:]
+        return grad.reshape(logits.shape)
+
+
+@pytest.mark.parametrize("cut,sliced", [
+    (lambda t: t[:, :-1], True), (lambda t: t[:, 1:], True), (lambda t: t[::2], True),
+    (lambda t: t[1:, 1:-1], True), (lambda t: t[:1].expand(4, 5, 11), True), (lambda t: t[:, :1], True),
+    (lambda t: t, False), (lambda t: t[:, ::2], False), (lambda t: t[:, :, 1:], False),
+    (lambda t: t.transpose(0, 1), False), (lambda t: t[0], False), (lambda t: t[:1, :-1], False),
+    (lambda t: t[:, None, :-1], False)])
+def test_selective_slices_over_layouts(cut, sliced):
+    """Which layouts take one sliced launch, and that every layout's values and
+    gradients are torch's."""
+    from fuselse_amd.selective import make_selective_log_softmax
+
+    ext = FakeSlicedExt()
+    sls = make_selective_log_softmax(ext)
+    full = torch.randn(4, 5, 11)
+    leaf, ref_leaf = full.clone().requires_grad_(True), full.clone().requires_grad_(True)
+    shape = cut(full).shape
+    index = torch.randint(0, shape[-1], shape[:-1])
+    w = torch.randn(shape[:-1])
+    y = sls(cut(fake(leaf)), fake(index))
+    (y.as_subclass(torch.Tensor) * w).sum().backward()
+    assert [c[0] for c in ext.calls] == (["fwd sliced", "bwd sliced"] if sliced else ["fwd", "bwd"])
+    ref = torch.log_softmax(cut(ref_leaf), -1).gather(-1, index[..., None])[..., 0]
+    (ref * w).sum().backward()
+    torch.testing.assert_close(y.as_subclass(torch.Tensor), ref.detach())
+    torch.testing.assert_close(leaf.grad, ref_leaf.grad)
+
+
 def test_selective_fallbacks_do_not_touch_the_extension():
     from fuselse_amd.selective import make_selective_log_softmax
 

@@ -210,3 +210,54 @@ def test_selective_dropin_on_trl_slice(cuda, Bt, T, V):
         y2 = fuselse_amd.selective_log_softmax(view, torch.from_numpy(idx).to(cuda))
         y3 = fuselse_amd.selective_log_softmax(view.contiguous(), torch.from_numpy(idx).to(cuda))
     torch.testing.assert_close(y2, y3, rtol=1e-6, atol=1e-6)
+
+
+@pytest.mark.parametrize("Bt,T,V,lead,cut", [
+    (3, 5, 1, 1, 0), (2, 7, 3, 0, 1), (5, 4, 61, 0, 1), (3, 9, 255, 1, 1), (4, 3, 256, 0, 1), (3, 6, 257, 0, 1),
+    (2, 5, 1023, 1, 0), (7, 2, 4099, 0, 1), (2, 3, 50257, 0, 1), (2, 2, 128256, 1, 0), (70, 3, 100, 0, 1)])
+def test_selective_slices_in_one_launch(cuda, Bt, T, V, lead, cut):
+    """logits[:, lead:T-cut] through the sliced entries: row lengths around the
+    gradient's 4-element vectors and 256-element waves, slices of every 16-byte
+    phase, a first row off the vectors' grid, more slices than the per-slice
+    path takes.  Targets at row ends land in vectors that span rows."""
+    print(f"case sls slices {Bt}x{T}x{V} lead {lead} cut {cut}", flush=True)
+    ext = _ext()
+    rng = np.random.default_rng(Bt * T + V)
+    x = (rng.standard_normal((Bt, T, V)) * 3).astype(np.float32)
+    view = torch.from_numpy(x).to(cuda)[:, lead:T - cut]
+    rows = np.ascontiguousarray(x[:, lead:T - cut]).reshape(-1, V)
+    B = rows.shape[0]
+    idx = rng.integers(0, V, B)
+    idx[::3], idx[1::3] = V - 1, 0
+    g = rng.standard_normal(B).astype(np.float32)
+    it = torch.from_numpy(idx).to(cuda)
+    logp, lse = ext.selective_log_softmax_slices_float(view, it)
+    _check_fwd(logp.cpu().numpy(), lse.cpu().numpy(), rows, idx)
+    got = ext.selective_log_softmax_slices_float_backward(torch.from_numpy(g).to(cuda), view, it, lse)
+    assert got.shape == view.shape and got.is_contiguous()
+    want = O.selective_logsoftmax_bwd_fp64(g, rows, idx, O.lse_fp64(rows))
+    err = np.abs(got.cpu().numpy().reshape(-1, V) - want)
+    assert (err <= 1e-5 * np.abs(want) + 1e-6 * np.abs(g)[:, None]).all(), err.max()
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f16", "bf16"])
+@pytest.mark.parametrize("B,N", [(5, 3), (9, 50), (4, 513), (3, 2051)])
+def test_backward_of_rows_off_the_gradients_grid(cuda, dtype, B, N):
+    """x one element off the 16-byte grid, its gradient on it: the shifted flat
+    kernel, for every element size (half results are exact to one rounding of
+    the fp32 value, 2^-11 or 2^-8 relative, plus fp16's subnormal step)."""
+    print(f"case bwd shifted {dtype} B={B} N={N}", flush=True)
+    ext = _ext()
+    tdt = {"f32": torch.float32, "f16": torch.float16, "bf16": torch.bfloat16}[dtype]
+    gen = torch.Generator().manual_seed(B + N)
+    xs = (torch.randn(B, N, generator=gen) * 2).to(tdt)
+    g = torch.randn(B, generator=gen)
+    xv = torch.empty(B * N + 1, dtype=tdt, device=cuda)[1:].view(B, N)
+    xv.copy_(xs)
+    lse = torch.logsumexp(xs.double(), -1)
+    lse32 = lse.float().to(cuda)
+    fn = ext.onepass_lse_float_backward if dtype == "f32" else ext.onepass_lse_half_backward
+    got = fn(g.to(cuda), xv, lse32).cpu().double()
+    want = g.double()[:, None] * torch.exp(xs.double() - lse[:, None])
+    rel = {"f32": 1e-5, "f16": 2.0 ** -11 + 1e-5, "bf16": 2.0 ** -8 + 1e-5}[dtype]
+    assert ((got - want).abs() <= rel * want.abs() + (2.0 ** -25 if dtype == "f16" else 1e-30)).all()
