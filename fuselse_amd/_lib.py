@@ -50,6 +50,9 @@ SIGNATURES = {
     "fl_intlse_q10_6": (_int, [_vp, _vp, _vp, _i64, _i64, _vp]),
     "fl_sparse_csr_fwd": (_int, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _int, _vp]),
     "fl_sparse_csr_bwd": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _vp]),
+    "fl_sparse_csr_bwd_workspace_bytes": (ctypes.c_size_t, [_i64, _i64, _i64]),
+    "fl_sparse_csr_bwd_ws": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp,
+                                    ctypes.c_size_t, _vp]),
     "fl_sparse_blocked_fwd": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _int, _vp]),
     "fl_sparse_blocked_bwd": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _int, _vp, _vp,
                                      _i64, _vp, _vp, _vp, _vp]),

@@ -12,12 +12,14 @@
 // Node values are [node][batch] rows, so each edge gathers one contiguous
 // child row.
 //
-// Mapping: one wave per (node, 256-column tile); lane l owns 4 columns (one
-// 16-byte vector when the batch is a multiple of 4 and rows are 16-byte
-// aligned, else 4 strided scalars).  Edge metadata is held one 64-edge window
-// at a time across the lanes and broadcast per edge with readlane; child rows
-// are loaded G = 4 edges at a time into two alternating register buffers, so
-// the next group's loads are in flight while a group folds.
+// Mapping.  CSR layers: csr_fwd_kernel, a wave per run of nodes and tile of 64
+// or 128 columns, its edges one stream.  The block layout (and some Q16.16 CSR
+// layers): sparse_kernel, one wave per (node, tile of 64, 128 or 256 columns);
+// lane l owns 1, 2 or 4 columns (one vector when the batch is a multiple of it
+// and rows are aligned, else strided scalars), edge metadata is held one
+// 64-edge window at a time across the lanes and broadcast per edge with
+// readlane, and child rows are loaded G = 4 edges at a time into two
+// alternating register buffers.
 //
 // fp32: an online (max, scaled sum) per column with one rescale per group.
 // Q16.16: bit-exact with the reference's reduction: ET = 1, 2, 4, 8 chains
@@ -41,8 +43,6 @@ constexpr int kNegInfQ = -0x3fffffff;
 constexpr float kConv = 1.44269504089f * 65536.0f;
 constexpr float kOutScale = 0.69314718056f / 65536.0f;
 constexpr int G = 4;      // edges per load group
-constexpr int P = 4;      // columns per lane, forward kernels
-constexpr int PB = 8;     // columns per lane, backward kernel
 
 __constant__ int kLut[64] = {
        0,  571,  907, 1282, 1634, 1745, 2054, 2592,
@@ -55,75 +55,88 @@ __constant__ int kLut[64] = {
      312,  235,  168,  113,   69,   35,   13,    2,
 };
 
-__device__ __forceinline__ int pair(int a, int b, const int* __restrict__ lut) {
-    const int hi = a > b ? a : b;
-    const int lo = a > b ? b : a;
-    const int sub = (int)((uint32_t)lo - (uint32_t)hi);
-    const uint32_t sh = (uint32_t)(-(sub >> 16));
-    const uint32_t shc = sh < 31u ? sh : 31u;
-    const uint32_t fr = 0x10000u | ((uint32_t)sub & 0xFFFFu);
-    const uint32_t m = fr >> shc;
-    // (fr >> 8) >> shc == m >> 8 (logical shifts compose); byte 1 of m masked
-    // is one instruction on this target
-    const uint32_t off = (m >> 8) & 0xFCu;
-    return (int)((uint32_t)hi + m + (uint32_t)*reinterpret_cast<const int*>(reinterpret_cast<const char*>(lut) + off));
+// Fixed-point values inside the folds are biased by 2^31, as unsigned: the
+// order is the same, and |a - b| is one instruction on unsigned operands.
+constexpr uint32_t kBias = 0x80000000u;
+constexpr uint32_t kNegInfU = (uint32_t)kNegInfQ ^ kBias;
+
+// The reference's pair op, max + M + LUT[(M >> 10) & 63] with
+// M = (2^16 + ((lo - hi) & 0xFFFF)) >> ceil((hi - lo) / 2^16), the shift
+// clamped to 31.  With t = |a - b| + 0xFFFF mod 2^32 (v_sad_u32) the shift is
+// t >> 16, and 2^16 plus the low half of lo - hi is 2^16 plus the complement of
+// t's low half, one bit select.  (Differences within 2^16 of 2^32, which only
+// accumulators wrapped past the int32 limit reach, wrap t to a shift of 0, as
+// the signed 32-bit difference does.)  Seven vector instructions and the table
+// read; max, min, their difference, its halves and a two-instruction table
+// offset took ten: the block layer of 2048 x 32 nodes, 32 edges, batch 512,
+// whose time this is, went from 472 to 424 us.
+__device__ __forceinline__ uint32_t pair(uint32_t a, uint32_t b, const int* __restrict__ lut) {
+    const uint32_t hi = a > b ? a : b;
+    uint32_t t, fr, off;
+    asm("v_sad_u32 %0, %1, %2, %3" : "=v"(t) : "v"(a), "v"(b), "s"(0xFFFFu));
+    const uint32_t th = t >> 16;
+    const uint32_t sh = th < 31u ? th : 31u;
+    asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(fr) : "v"(t), "v"(0x10000u), "s"(0x1FFFFu));
+    const uint32_t m = fr >> sh;
+    // table offset (m >> 8) & 0xFC: byte 1 of m, masked
+    asm("v_and_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_1 src1_sel:DWORD"
+        : "=v"(off)
+        : "v"(m), "s"(0xFCu));
+    return hi + m + (uint32_t)*reinterpret_cast<const int*>(reinterpret_cast<const char*>(lut) + off);
 }
 
-__device__ __forceinline__ int quant(float logit) {
+__device__ __forceinline__ uint32_t quant(float logit) {
     const float r = __builtin_rintf(fmaxf(logit, -20000.0f) * kConv);
     int q;
     asm("v_cvt_i32_f32 %0, %1" : "=v"(q) : "v"(r));
-    return q;
+    return (uint32_t)q ^ kBias;
 }
 
-// The PP columns of lane l in the tile of 64*PP columns starting at b0.  With
-// VEC, lane l holds the 16-byte vectors at b0 + 256*q + 4*l (q < PP/4): each
-// vector load of the wave covers 1 KB of a row, contiguous.  Otherwise lane l
-// holds the scalars b0 + l + 64*i.
-template <bool VEC, int PP>
-struct Cols {
-    static_assert(!VEC || PP % 4 == 0, "vector columns come in fours");
-    __device__ static __forceinline__ bool ok(int64_t b0, int l, int64_t batch, int i) {
-        return VEC ? b0 + 256 * (i / 4) + 4 * l < batch : b0 + l + 64 * i < batch;
+// Vectors of VW floats and their buffer loads.
+template <int VW>
+struct Vec;
+template <>
+struct Vec<4> {
+    typedef f32x4 T;
+    __device__ static __forceinline__ T load(__amdgpu_buffer_rsrc_t r, int off) {
+        return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
     }
-    __device__ static __forceinline__ void load(const float* __restrict__ row, int64_t b0, int l, int64_t batch,
-                                                float (&v)[PP]) {
-        if constexpr (VEC) {
-#pragma unroll
-            for (int q = 0; q < PP / 4; ++q) {
-                const int64_t c = b0 + 256 * q + 4 * l;
-                if (c < batch) {
-                    const f32x4 t = *reinterpret_cast<const f32x4*>(row + c);
-                    v[4 * q] = t.x; v[4 * q + 1] = t.y; v[4 * q + 2] = t.z; v[4 * q + 3] = t.w;
-                } else {
-                    v[4 * q] = v[4 * q + 1] = v[4 * q + 2] = v[4 * q + 3] = 0.0f;
-                }
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < PP; ++i) {
-                const int64_t c = b0 + l + 64 * i;
-                v[i] = c < batch ? row[c] : 0.0f;
-            }
-        }
+};
+template <>
+struct Vec<2> {
+    typedef float T __attribute__((ext_vector_type(2)));
+    __device__ static __forceinline__ T load(__amdgpu_buffer_rsrc_t r, int off) {
+        return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
+    }
+};
+template <>
+struct Vec<1> {
+    typedef float T __attribute__((ext_vector_type(1)));
+    __device__ static __forceinline__ T load(__amdgpu_buffer_rsrc_t r, int off) {
+        return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
+    }
+};
+
+// The PP columns of lane l in the tile of 64*PP columns starting at b0: the
+// vectors of VW columns at b0 + 64*VW*q + VW*l (q < PP/VW), each load of the
+// wave covering 64*VW contiguous columns of a row.  VW > 1 needs the batch and
+// the rows to be whole, aligned vectors, so that none crosses the batch's end.
+template <int VW, int PP>
+struct Cols {
+    static_assert(PP % VW == 0, "columns come in whole vectors");
+    __device__ static __forceinline__ bool ok(int64_t b0, int l, int64_t batch, int i) {
+        return b0 + 64 * VW * (i / VW) + VW * l < batch;
     }
     __device__ static __forceinline__ void store(float* __restrict__ row, int64_t b0, int l, int64_t batch,
                                                  const float (&v)[PP]) {
-        if constexpr (VEC) {
 #pragma unroll
-            for (int q = 0; q < PP / 4; ++q) {
-                const int64_t c = b0 + 256 * q + 4 * l;
-                if (c < batch) {
-                    f32x4 t;
-                    t.x = v[4 * q]; t.y = v[4 * q + 1]; t.z = v[4 * q + 2]; t.w = v[4 * q + 3];
-                    store_stream<f32x4>(t, row + c);
-                }
-            }
-        } else {
+        for (int q = 0; q < PP / VW; ++q) {
+            const int64_t c = b0 + 64 * VW * q + VW * l;
+            if (c < batch) {
+                typename Vec<VW>::T t;
 #pragma unroll
-            for (int i = 0; i < PP; ++i) {
-                const int64_t c = b0 + l + 64 * i;
-                if (c < batch) row[c] = v[i];
+                for (int k = 0; k < VW; ++k) t[k] = v[VW * q + k];
+                store_stream<typename Vec<VW>::T>(t, row + c);
             }
         }
     }
@@ -201,24 +214,20 @@ struct BlockLayout {
 // ---------------------------------------------------------------------------
 // Per-node reductions over one 256-column tile.
 // ---------------------------------------------------------------------------
-// The 16-byte column vectors of lane l (as Cols<true, PP>) from the row
-// segment starting at b0 (`row` points at it), through a buffer resource of
-// `rec` bytes: vectors past the range read as zeros, without a memory access,
-// and the load needs no branch.  The rows are gathered by id, and they take
-// plain loads: with the nontemporal hint (which streamed dense rows read
-// faster) the C5 layer's forward took 3339 us against 3139, its backward
-// 7046 us against 6169.
-template <int PP>
+// The columns of lane l (as Cols<VW, PP>) from the row segment starting at b0
+// (`row` points at it), through a buffer resource of `rec` bytes: columns past
+// the range read as zeros, without a memory access, and the load needs no
+// branch.  The rows are gathered by id, and they take plain loads: with the
+// nontemporal hint (which streamed dense rows read faster) the C5 layer's
+// forward took 3339 us against 3139, its backward 7046 us against 6169.
+template <int VW, int PP>
 __device__ __forceinline__ void load_cols_buf(const float* row, int rec, int l, float (&v)[PP]) {
     const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(row), 0, rec, 0x00020000);
 #pragma unroll
-    for (int q = 0; q < PP / 4; ++q) {
-        const f32x4 t =
-            __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (256 * q + 4 * l) * 4, 0, 0));
-        v[4 * q] = t.x;
-        v[4 * q + 1] = t.y;
-        v[4 * q + 2] = t.z;
-        v[4 * q + 3] = t.w;
+    for (int q = 0; q < PP / VW; ++q) {
+        const typename Vec<VW>::T t = Vec<VW>::load(r, (64 * VW * q + VW * l) * 4);
+#pragma unroll
+        for (int k = 0; k < VW; ++k) v[VW * q + k] = t[k];
     }
 }
 
@@ -229,25 +238,19 @@ __device__ __forceinline__ int cols_bytes(int64_t batch, int64_t b0) {
 }
 
 // Loads the child rows of window edges j .. j + GS - 1 (edges at or past wn
-// are left for the fold to mask).  With VEC every load is issued: each edge's
-// row goes through a buffer resource built from its wave-uniform child id,
-// with an empty range for edges past wn and the range check covering the
-// batch's end, so no load sits behind a branch.  A load behind a branch left
-// the wait-count pass unable to count the loads in flight, and the fold of a
-// group then waited for the next group's loads as well.
-template <int GS, bool VEC, int PP>
+// are left for the fold to mask).  Every load is issued: each edge's row goes
+// through a buffer resource built from its wave-uniform child id, with an
+// empty range for edges past wn and the range check covering the batch's end,
+// so no load sits behind a branch.  A load behind a branch left the wait-count
+// pass unable to count the loads in flight, and the fold of a group then
+// waited for the next group's loads as well.
+template <int GS, int VW, int PP>
 __device__ __forceinline__ void load_group(float (&v)[GS][PP], const EdgeMeta& ew, int j, int wn,
                                            const float* __restrict__ child, int64_t batch, int64_t b0, int l) {
-    if constexpr (VEC) {
-        const int rec = cols_bytes(batch, b0);
+    const int rec = cols_bytes(batch, b0);
 #pragma unroll
-        for (int g = 0; g < GS; ++g)
-            load_cols_buf<PP>(child + bcast64(ew.cid, (j + g) & 63) * batch + b0, j + g < wn ? rec : 0, l, v[g]);
-    } else {
-#pragma unroll
-        for (int g = 0; g < GS; ++g)
-            if (j + g < wn) Cols<VEC, PP>::load(child + bcast64(ew.cid, j + g) * batch, b0, l, batch, v[g]);
-    }
+    for (int g = 0; g < GS; ++g)
+        load_cols_buf<VW, PP>(child + bcast64(ew.cid, (j + g) & 63) * batch + b0, j + g < wn ? rec : 0, l, v[g]);
 }
 
 template <int PP>
@@ -269,9 +272,9 @@ __device__ __forceinline__ void fold_group_f32(const float (&v)[G][PP], const Ed
 // Windows start at multiples of 64 and groups at multiples of G = 4, so for
 // ET <= 4 the chain is g % ET, and for ET = 8 it is C0 + g with C0 = j % 8,
 // 0 or 4: a wave-uniform choice between two static code paths.
-template <int ET, int C0>
+template <int ET, int C0, int P>
 __device__ __forceinline__ void fold_group_q16_at(const float (&v)[G][P], const EdgeMeta& ew, int j, int wn,
-                                                  int (&acc)[ET][P], const int* __restrict__ lut) {
+                                                  uint32_t (&acc)[ET][P], const int* __restrict__ lut) {
 #pragma unroll
     for (int g = 0; g < G; ++g) {
         if (j + g < wn) {
@@ -283,23 +286,23 @@ __device__ __forceinline__ void fold_group_q16_at(const float (&v)[G][P], const 
     }
 }
 
-template <int ET>
+template <int ET, int P>
 __device__ __forceinline__ void fold_group_q16(const float (&v)[G][P], const EdgeMeta& ew, int j, int wn,
-                                               int (&acc)[ET][P], const int* __restrict__ lut) {
+                                               uint32_t (&acc)[ET][P], const int* __restrict__ lut) {
     if constexpr (ET == 8) {
         if (j & 4)
-            fold_group_q16_at<ET, 4>(v, ew, j, wn, acc, lut);
+            fold_group_q16_at<ET, 4, P>(v, ew, j, wn, acc, lut);
         else
-            fold_group_q16_at<ET, 0>(v, ew, j, wn, acc, lut);
+            fold_group_q16_at<ET, 0, P>(v, ew, j, wn, acc, lut);
     } else {
-        fold_group_q16_at<ET, 0>(v, ew, j, wn, acc, lut);
+        fold_group_q16_at<ET, 0, P>(v, ew, j, wn, acc, lut);
     }
 }
 
 // Walks the node's edges in 64-edge windows; groups of GS edges alternate
 // between two register buffers (loads of group g+1 in flight while group g
 // folds).  FOLD(buf, j, wn, ew) folds group starting at window edge j.
-template <int GS, bool VEC, int PP, typename LAYOUT, typename DESC, typename FOLD>
+template <int GS, int VW, int PP, typename LAYOUT, typename DESC, typename FOLD>
 __device__ __forceinline__ void walk_edges(const LAYOUT& L, const DESC& d, const EdgeMeta& first,
                                            const float* __restrict__ child, int64_t batch, int64_t b0, int l,
                                            FOLD fold) {
@@ -308,47 +311,47 @@ __device__ __forceinline__ void walk_edges(const LAYOUT& L, const DESC& d, const
         const int wn = (int)(d.k - w0 < 64 ? d.k - w0 : 64);
         const int ng = (wn + GS - 1) / GS;
         float va[GS][PP], vb[GS][PP];
-        load_group<GS, VEC, PP>(va, ew, 0, wn, child, batch, b0, l);
+        load_group<GS, VW, PP>(va, ew, 0, wn, child, batch, b0, l);
         for (int gi = 0; gi < ng; gi += 2) {
-            // with VEC the prefetch is unconditional (a group past the window
-            // reads empty ranges), keeping every load outside a branch
-            if (VEC || gi + 1 < ng) load_group<GS, VEC, PP>(vb, ew, (gi + 1) * GS, wn, child, batch, b0, l);
+            // the prefetch is unconditional (a group past the window reads
+            // empty ranges), keeping every load outside a branch
+            load_group<GS, VW, PP>(vb, ew, (gi + 1) * GS, wn, child, batch, b0, l);
             fold(va, gi * GS, wn, ew);
             if (gi + 1 >= ng) break;
-            if (VEC || gi + 2 < ng) load_group<GS, VEC, PP>(va, ew, (gi + 2) * GS, wn, child, batch, b0, l);
+            load_group<GS, VW, PP>(va, ew, (gi + 2) * GS, wn, child, batch, b0, l);
             fold(vb, (gi + 1) * GS, wn, ew);
         }
     }
 }
 
-template <bool VEC, typename LAYOUT, typename DESC>
+template <int VW, int P, typename LAYOUT, typename DESC>
 __device__ __forceinline__ void reduce_f32(const LAYOUT& L, const DESC& d, const EdgeMeta& first,
                                            const float* __restrict__ child, int64_t batch, int64_t b0, int l) {
     float m[P], s[P];
 #pragma unroll
     for (int i = 0; i < P; ++i) { m[i] = -kInf; s[i] = 0.0f; }
-    walk_edges<G, VEC, P>(L, d, first, child, batch, b0, l,
+    walk_edges<G, VW, P>(L, d, first, child, batch, b0, l,
                            [&](const float (&v)[G][P], int j, int wn, const EdgeMeta& ew) {
                                fold_group_f32<P>(v, ew, j, wn, m, s);
                            });
     float res[P];
 #pragma unroll
     for (int i = 0; i < P; ++i) res[i] = lse_finish<true>(m[i], s[i]);
-    Cols<VEC, P>::store(L.out_row(d), b0, l, batch, res);
+    Cols<VW, P>::store(L.out_row(d), b0, l, batch, res);
 }
 
-template <int ET, bool VEC, typename LAYOUT, typename DESC>
+template <int ET, int VW, int P, typename LAYOUT, typename DESC>
 __device__ __forceinline__ void reduce_q16_et(const LAYOUT& L, const DESC& d, const EdgeMeta& first,
                                               const float* __restrict__ child, int64_t batch, int64_t b0, int l,
                                               const int* __restrict__ lut) {
-    int acc[ET][P];
+    uint32_t acc[ET][P];
 #pragma unroll
     for (int c = 0; c < ET; ++c)
 #pragma unroll
-        for (int i = 0; i < P; ++i) acc[c][i] = kNegInfQ;
-    walk_edges<G, VEC, P>(L, d, first, child, batch, b0, l,
+        for (int i = 0; i < P; ++i) acc[c][i] = kNegInfU;
+    walk_edges<G, VW, P>(L, d, first, child, batch, b0, l,
                           [&](const float (&v)[G][P], int j, int wn, const EdgeMeta& ew) {
-                              fold_group_q16<ET>(v, ew, j, wn, acc, lut);
+                              fold_group_q16<ET, P>(v, ew, j, wn, acc, lut);
                           });
     float res[P];
 #pragma unroll
@@ -363,23 +366,24 @@ __device__ __forceinline__ void reduce_q16_et(const LAYOUT& L, const DESC& d, co
             for (int c = 0; c < 2; ++c) acc[c][i] = pair(acc[c][i], acc[c + 2][i], lut);
         }
         if constexpr (ET >= 2) acc[0][i] = pair(acc[0][i], acc[1][i], lut);
-        res[i] = acc[0][i] > kNegInfQ ? (float)acc[0][i] * kOutScale : -kInf;
+        const int q = (int)(acc[0][i] ^ kBias);
+        res[i] = q > kNegInfQ ? (float)q * kOutScale : -kInf;
     }
-    Cols<VEC, P>::store(L.out_row(d), b0, l, batch, res);
+    Cols<VW, P>::store(L.out_row(d), b0, l, batch, res);
 }
 
-template <bool VEC, typename LAYOUT, typename DESC>
+template <int VW, int P, typename LAYOUT, typename DESC>
 __device__ __forceinline__ void reduce_q16(const LAYOUT& L, const DESC& d, const EdgeMeta& first,
                                            const float* __restrict__ child, int64_t batch, int64_t b0, int l,
                                            const int* __restrict__ lut) {
     if (d.k <= 8)
-        reduce_q16_et<1, VEC>(L, d, first, child, batch, b0, l, lut);
+        reduce_q16_et<1, VW, P>(L, d, first, child, batch, b0, l, lut);
     else if (d.k <= 16)
-        reduce_q16_et<2, VEC>(L, d, first, child, batch, b0, l, lut);
+        reduce_q16_et<2, VW, P>(L, d, first, child, batch, b0, l, lut);
     else if (d.k <= 32)
-        reduce_q16_et<4, VEC>(L, d, first, child, batch, b0, l, lut);
+        reduce_q16_et<4, VW, P>(L, d, first, child, batch, b0, l, lut);
     else
-        reduce_q16_et<8, VEC>(L, d, first, child, batch, b0, l, lut);
+        reduce_q16_et<8, VW, P>(L, d, first, child, batch, b0, l, lut);
 }
 
 // One single-wave block per (node, 256-column tile) pair, pairs numbered
@@ -389,7 +393,7 @@ __device__ __forceinline__ void reduce_q16(const LAYOUT& L, const DESC& d, const
 // barrier (C5: Q16 4.70 -> 3.79 ms, fp32 3.37 -> 3.32 ms).  One wave needs no
 // barrier for the table: its LDS operations retire in order.  The pair index
 // is block-uniform, so the node's descriptor comes through scalar loads.
-template <bool Q16, bool VEC, typename LAYOUT>
+template <bool Q16, int VW, int P, typename LAYOUT>
 __global__ __launch_bounds__(64) void sparse_kernel(LAYOUT L, const float* __restrict__ child, int64_t batch,
                                                     int64_t items, int64_t tiles, int64_t pair0) {
     __shared__ int lut[64];
@@ -405,25 +409,380 @@ __global__ __launch_bounds__(64) void sparse_kernel(LAYOUT L, const float* __res
     const EdgeMeta first = l < desc.k ? L.meta(desc, l) : EdgeMeta{0, 0.0f};
     const int64_t b0 = (pair - item * tiles) * 64 * P;
     if constexpr (Q16)
-        reduce_q16<VEC>(L, desc, first, child, batch, b0, l, lut);
+        reduce_q16<VW, P>(L, desc, first, child, batch, b0, l, lut);
     else
-        reduce_f32<VEC>(L, desc, first, child, batch, b0, l);
+        reduce_f32<VW, P>(L, desc, first, child, batch, b0, l);
 }
 
+template <bool Q16, int VW, int P, typename LAYOUT>
+static void launch_cols(const LAYOUT& L, const float* child, int64_t items, int64_t batch, hipStream_t st) {
+    const int64_t tiles = (batch + 64 * P - 1) / (64 * P);
+    for_grid_chunks(items * tiles, 64, [&](int64_t p0, int64_t n) {
+        sparse_kernel<Q16, VW, P, LAYOUT><<<dim3((unsigned)n), dim3(64), 0, st>>>(L, child, batch, items, tiles, p0);
+    });
+}
+
+// Columns per lane by the batch (200000 CSR nodes through this kernel, Q16.16,
+// us at 1 / 2 / 4 columns a lane: batch 64 134 / 160 / 242, 100 236 / 164 / 244,
+// 256 437 / 286 / 300, 512 923 / 584 / 531).
 template <bool Q16, typename LAYOUT>
 static void launch(const LAYOUT& L, const float* child, const float* out_any, int64_t items, int64_t batch,
                    hipStream_t st) {
-    const bool vec = (batch % 4 == 0) &&
-                     ((reinterpret_cast<uintptr_t>(child) | reinterpret_cast<uintptr_t>(out_any)) & 15) == 0;
-    const int64_t tile = 64 * P;
-    const int64_t tiles = (batch + tile - 1) / tile;
-    const int64_t pairs = items * tiles;
-    for_grid_chunks(pairs, 64, [&](int64_t p0, int64_t n) {
-        if (vec)
-            sparse_kernel<Q16, true, LAYOUT><<<dim3((unsigned)n), dim3(64), 0, st>>>(L, child, batch, items, tiles, p0);
+    const uintptr_t at = reinterpret_cast<uintptr_t>(child) | reinterpret_cast<uintptr_t>(out_any);
+    if (batch <= 64)
+        launch_cols<Q16, 1, 1>(L, child, items, batch, st);
+    else if (batch <= 128) {
+        if (batch % 2 == 0 && (at & 7) == 0)
+            launch_cols<Q16, 2, 2>(L, child, items, batch, st);
         else
-            sparse_kernel<Q16, false, LAYOUT><<<dim3((unsigned)n), dim3(64), 0, st>>>(L, child, batch, items, tiles, p0);
+            launch_cols<Q16, 1, 2>(L, child, items, batch, st);
+    } else if (batch % 4 == 0 && (at & 15) == 0)
+        launch_cols<Q16, 4, 4>(L, child, items, batch, st);
+    else
+        launch_cols<Q16, 1, 4>(L, child, items, batch, st);
+}
+
+// ---------------------------------------------------------------------------
+// CSR forward: one wave per run of `npw` consecutive nodes and tile of 64 or
+// 128 columns, walking the run's edges as one stream of groups of up to G edges
+// (a group never spans two nodes).  The next group's rows are in flight while
+// a group folds, across node boundaries too, and the group after that has its
+// edge ids and weights on the way through scalar loads, so a node costs no
+// round trips of its own: with a wave per node, each paid three in a row
+// (offsets, ids, rows).  The tiles go one after the other over all runs, so
+// that at any time the gathers stay within one column slice of the children,
+// of which the 256 MB Infinity Cache holds a part: a 1M-row, 512-column layer
+// gathers 7.3 TB/s from random rows in slices where it took 5.9 in whole rows.
+// The layer (8.0M edges, fan-in k^-2 on [2, 256]) went from 3140 to 2554 us in
+// fp32 and to 2595 in Q16.16 (wave per node and 256-column tile, tile-fastest
+// -> this); the gathers alone, with the same stores, take 2354.
+// ---------------------------------------------------------------------------
+// Scalar loads of 4 consecutive words through a buffer resource: words past
+// its range read as 0.
+typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));
+__device__ u32x4v s_buffer_load4(u32x4v rsrc, int32_t off, int32_t aux) __asm("llvm.amdgcn.s.buffer.load.v4i32");
+
+// Group j.. of a run's node: `left` edges of the node from the run's edge e on,
+// of which the group takes the first G.  All of it wave-uniform, in 32-bit
+// scalars (64-bit compares and carried booleans would move to vector
+// registers).  k: the node's edges.
+struct Group {
+    int32_t e, node, left, first, k;
+};
+
+// Lane i holds the edge at which the run's node i starts, counted from the
+// run's first; lanes at and past the run's node count hold the run's end.
+struct Run {
+    int32_t at;
+    __device__ __forceinline__ int32_t start(int node) const { return __builtin_amdgcn_readlane(at, node); }
+    __device__ __forceinline__ Group next(const Group& g) const {
+        const int32_t last = g.left <= G;
+        const int32_t e = g.e + (last ? g.left : G), node = g.node + last;
+        const int32_t left = start(node + 1) - e;
+        return {e, node, left, last, last ? left : g.k};
+    }
+};
+
+// Ids and weights of a group's edges; entries past the group's are those of
+// following edges, or 0, and are masked by `left`.
+struct GroupMeta {
+    u32x4v cid, lw;
+};
+static_assert(G == 4, "a group's ids are one 4-word scalar load");
+
+__device__ __forceinline__ u32x4v words_rsrc(const void* p, int64_t words) {
+    const uint64_t a = reinterpret_cast<uintptr_t>(p);
+    return {(uint32_t)a, (uint32_t)(a >> 32) & 0xFFFFu, words < 0x1FFFFFFF ? (uint32_t)words * 4u : 0x7FFFFFFCu,
+            0x00020000u};
+}
+
+// Folds K edges into (m, s) of each column (FIRST: from nothing).  Where every
+// column's new maximum is finite and below 2^24 the rescale and the
+// exponentials need no special cases (a -inf term is exp2(-inf) = 0, a NaN
+// stays NaN); other lanes take lse_fold's robust forms, on the same values.
+template <int K, bool FIRST, int P>
+__device__ __forceinline__ void fold_edges_f32(const float (&v)[G][P], const float (&lw)[G], float (&m)[P],
+                                               float (&s)[P]) {
+    float t[P][K], mn[P], top = 0.0f;
+#pragma unroll
+    for (int i = 0; i < P; ++i) {
+#pragma unroll
+        for (int g = 0; g < K; ++g) t[i][g] = v[g][i] + lw[g];
+        float cm = t[i][0];
+#pragma unroll
+        for (int g = 1; g < K; ++g) cm = fmaxf(cm, t[i][g]);
+        mn[i] = FIRST ? cm : fmaxf(m[i], cm);
+        top = fmaxf(top, __builtin_fabsf(mn[i]));
+    }
+    if (top < 0x1p24f) {
+#pragma unroll
+        for (int i = 0; i < P; ++i) {
+            const float nb = -mn[i] * kLog2e;
+            float acc = 0.0f;
+#pragma unroll
+            for (int g = 0; g < K; ++g) acc += lse_exp_fused(t[i][g], nb);
+            s[i] = FIRST ? acc : s[i] * fexp2((m[i] - mn[i]) * kLog2e) + acc;
+            m[i] = mn[i];
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < P; ++i) {
+            if (FIRST) {
+                m[i] = -kInf;
+                s[i] = 0.0f;
+            }
+            lse_fold<true, K>(m[i], s[i], t[i]);
+        }
+    }
+}
+
+template <int P>
+__device__ __forceinline__ void fold_f32(const float (&v)[G][P], const GroupMeta& em, const Group& g, float (&m)[P],
+                                         float (&s)[P]) {
+    float lw[G];
+#pragma unroll
+    for (int k = 0; k < G; ++k) lw[k] = __builtin_bit_cast(float, k < g.left ? (uint32_t)em.lw[k] : 0xFF800000u);
+    if (g.first) {
+        if (g.left <= 2)
+            fold_edges_f32<2, true, P>(v, lw, m, s);
+        else
+            fold_edges_f32<G, true, P>(v, lw, m, s);
+    } else {
+        fold_edges_f32<G, false, P>(v, lw, m, s);
+    }
+}
+
+// The folds over a node's groups: begin() at its first group, add() per group,
+// end() after its last.
+template <int P>
+struct FoldF32 {
+    float m[P], s[P];
+    __device__ __forceinline__ void add(const float (&v)[G][P], const GroupMeta& em, const Group& g) {
+        fold_f32<P>(v, em, g, m, s);
+    }
+    __device__ __forceinline__ void end(const Group&, float (&res)[P]) const {
+#pragma unroll
+        for (int i = 0; i < P; ++i) res[i] = lse_finish<true>(m[i], s[i]);
+    }
+};
+
+// The edge-thread tree of reduce_q16_et over a node's groups; chains by the
+// node's fan-in.  A group starts at a multiple of G of its node's edges, so
+// with 8 chains its first edge belongs to chain 0 or 4.
+template <int P>
+struct FoldQ16 {
+    uint32_t acc[8][P];
+    const int* lut;
+    template <int ET, int C0>
+    __device__ __forceinline__ void chains(const float (&v)[G][P], const GroupMeta& em, const Group& g) {
+#pragma unroll
+        for (int e = 0; e < G; ++e) {
+            if (e < g.left) {
+                const uint32_t w = em.lw[e];
+#pragma unroll
+                for (int i = 0; i < P; ++i)
+                    acc[(C0 + e) % ET][i] =
+                        pair(acc[(C0 + e) % ET][i], quant(__builtin_bit_cast(float, w) + v[e][i]), lut);
+            }
+        }
+    }
+    __device__ __forceinline__ void add(const float (&v)[G][P], const GroupMeta& em, const Group& g) {
+        if (g.first) {
+#pragma unroll
+            for (int c = 0; c < 8; ++c)
+#pragma unroll
+                for (int i = 0; i < P; ++i) acc[c][i] = kNegInfU;
+        }
+        if (g.k <= 8)
+            chains<1, 0>(v, em, g);
+        else if (g.k <= 16)
+            chains<2, 0>(v, em, g);
+        else if (g.k <= 32)
+            chains<4, 0>(v, em, g);
+        else if ((g.k - g.left) & 4)
+            chains<8, 4>(v, em, g);
+        else
+            chains<8, 0>(v, em, g);
+    }
+    // xor butterfly over the chains, distances 4, 2, 1 as far as there are chains
+    __device__ __forceinline__ void end(const Group& g, float (&res)[P]) {
+        if (g.k > 32) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+#pragma unroll
+                for (int i = 0; i < P; ++i) acc[c][i] = pair(acc[c][i], acc[c + 4][i], lut);
+        }
+        if (g.k > 16) {
+#pragma unroll
+            for (int c = 0; c < 2; ++c)
+#pragma unroll
+                for (int i = 0; i < P; ++i) acc[c][i] = pair(acc[c][i], acc[c + 2][i], lut);
+        }
+        if (g.k > 8) {
+#pragma unroll
+            for (int i = 0; i < P; ++i) acc[0][i] = pair(acc[0][i], acc[1][i], lut);
+        }
+#pragma unroll
+        for (int i = 0; i < P; ++i) {
+            const int q = (int)(acc[0][i] ^ kBias);
+            res[i] = q > kNegInfQ ? (float)q * kOutScale : -kInf;
+        }
+    }
+};
+
+// Edges of a run that the stream's 32-bit edge numbers and byte offsets hold;
+// a run of more walks its nodes one by one with 64-bit ones (walk_edges).
+constexpr int64_t kRunEdges = 1 << 20;
+
+template <bool Q16, int P>
+struct FoldPick {
+    typedef FoldF32<P> T;
+};
+template <int P>
+struct FoldPick<true, P> {
+    typedef FoldQ16<P> T;
+};
+template <bool Q16, int P>
+using FoldOf = typename FoldPick<Q16, P>::T;
+
+template <bool Q16, int VW, int P>
+__global__ __launch_bounds__(64) void csr_fwd_kernel(const float* __restrict__ child, const int64_t* __restrict__ off,
+                                                     const int32_t* __restrict__ cids, const float* __restrict__ logp,
+                                                     float* __restrict__ out, int64_t batch, int64_t nodes,
+                                                     int npw, int64_t unit0) {
+    __shared__ int lut[64];
+    FoldOf<Q16, P> state;
+    if constexpr (Q16) {
+        // one wave needs no barrier for the table: its LDS operations retire in order
+        lut[threadIdx.x] = kLut[threadIdx.x];
+        __builtin_amdgcn_wave_barrier();
+        state.lut = lut;
+    }
+    const int l = lane_id();
+    const int64_t unit = unit0 + blockIdx.x;
+    const int64_t runs = (nodes + npw - 1) / npw;
+    const int64_t tile = unit / runs;
+    const int64_t n0 = (unit - tile * runs) * npw;
+    const int64_t b0 = tile * 64 * P;
+    const int nn = (int)(nodes - n0 < npw ? nodes - n0 : npw);
+    const int64_t at = off[n0 + (l < nn ? l : nn)];
+    const int64_t e0 = uniform64(at);
+    if (bcast64(at, nn) - e0 > kRunEdges) {
+        const CsrLayout L{off, cids, logp, out, batch};
+        for (int n = 0; n < nn; ++n) {
+            const CsrDesc d = L.node(n0 + n);
+            const EdgeMeta first = l < d.k ? L.meta(d, l) : EdgeMeta{0, 0.0f};
+            if constexpr (Q16)
+                reduce_q16<VW, P>(L, d, first, child, batch, b0, l, lut);
+            else
+                reduce_f32<VW, P>(L, d, first, child, batch, b0, l);
+        }
+        return;
+    }
+    const Run run{(int32_t)(at - e0)};
+    const int32_t edges = run.start(nn);
+    const int64_t nnz = uniform64(off[nodes]);
+    const u32x4v rc = words_rsrc(cids + e0, nnz - e0), rl = words_rsrc(logp + e0, nnz - e0);
+    const float* child_b0 = child + b0;
+    const uint32_t row_bytes = (uint32_t)batch * 4u;
+    const int rec = cols_bytes(batch, b0);
+    const auto load_meta = [&](const Group& g) {
+        return GroupMeta{s_buffer_load4(rc, g.e * 4, 0), s_buffer_load4(rl, g.e * 4, 0)};
+    };
+    const auto load_rows = [&](float (&v)[G][P], const GroupMeta& em, const Group& g) {
+#pragma unroll
+        for (int k = 0; k < G; ++k)
+            load_cols_buf<VW, P>(reinterpret_cast<const float*>(reinterpret_cast<const char*>(child_b0) +
+                                                                (uint64_t)em.cid[k] * row_bytes),
+                                 k < g.left ? rec : 0, l, v[k]);
+    };
+    const auto fold = [&](const float (&v)[G][P], const GroupMeta& em, const Group& g) {
+        state.add(v, em, g);
+        if (g.left <= G && g.node < nn) {
+            float res[P];
+            state.end(g, res);
+            Cols<VW, P>::store(out + (n0 + g.node) * batch, b0, l, batch, res);
+        }
+    };
+    // ga, gb: the groups whose rows are in va, vb; the second one's ids (mb)
+    // are loaded while the first one's rows are awaited.  Groups past the run
+    // load nothing and store nothing: with an exit after the first fold the
+    // compiler sinks the ids' loads below it, next to their use.
+    float va[G][P], vb[G][P];
+    Group ga = {0, 0, run.start(1), 1, run.start(1)};
+    GroupMeta ma = load_meta(ga);
+    load_rows(va, ma, ga);
+    Group gb = run.next(ga);
+    GroupMeta mb = load_meta(gb);
+    while (true) {
+        load_rows(vb, mb, gb);
+        const Group gc = run.next(gb);
+        const GroupMeta mc = load_meta(gc);
+        fold(va, ma, ga);
+        load_rows(va, mc, gc);
+        const Group gd = run.next(gc);
+        const GroupMeta md = load_meta(gd);
+        fold(vb, mb, gb);
+        if (gc.node >= nn) return;
+        ga = gc;
+        ma = mc;
+        gb = gd;
+        mb = md;
+    }
+}
+
+// Nodes per run, by the (node, column tile) pairs of the launch: longer runs
+// spare more of the wave starts, shorter ones keep a small layer's waves many
+// and its largest nodes apart (MI355X, fan-in k^-2 on [2, 256], us at 1 / 2 /
+// 4 / 8 / 16 nodes a run: 2000 x 512 columns 26.5 / 28.0 / 28.9 / 30.5 / 34.0,
+// 20000 x 512 79.7 / 66.8 / 69.9 / 80.0 / 85.6, 200000 x 512 565 / 509 / 497 /
+// 506 / 514, 1M x 512 3325 / 2748 / 2619 / 2554 / 2576).
+static int run_nodes(int64_t pairs) {
+    return pairs < 40000 ? 1 : pairs < 160000 ? 2 : pairs < 1000000 ? 4 : 8;
+}
+
+template <bool Q16, int VW, int P>
+static void launch_csr_cols(const CsrLayout& L, const float* child, int64_t nodes, int npw, hipStream_t st) {
+    const int64_t tiles = (L.batch + 64 * P - 1) / (64 * P);
+    for_grid_chunks((nodes + npw - 1) / npw * tiles, 64, [&](int64_t u0, int64_t n) {
+        csr_fwd_kernel<Q16, VW, P><<<dim3((unsigned)n), dim3(64), 0, st>>>(child, L.offsets, L.cids, L.logp, L.out,
+                                                                          L.batch, nodes, npw, u0);
     });
+}
+
+// Whether the batch's rows cut into 128-column slices without loss: whole
+// 128-byte lines (a slice of a row that starts inside a line reads one more)
+// and at most a tenth of the last slice's lanes idle over all of them.
+static bool slices_fit(int64_t batch) { return batch % 32 == 0 && batch * 10 >= (batch + 127) / 128 * 128 * 9; }
+
+// Columns per lane: 1 up to a batch of 64, else 2 (200000 nodes, fp32, us, 1 / 2
+// columns a lane: batch 64 99 / 105, 100 182 / 142, 512 515 / 497; 4 columns
+// 140, 152, 519).  Large layers whose rows do not cut into such slices take
+// tiles of 256 columns, in fp32 through the stream (us, 128 / 256 columns: 1M x
+// 200 1304 / 1143, 500000 x 500 1482 / 1349, 50000 x 130 76 / 66, but 20000 x
+// 300 58 / 66), in Q16.16 with a wave per node and tile (200000 x 500: 618 in
+// slices, 595 through the stream, whose 8 chains of 4 columns leave it four
+// waves per SIMD).
+template <bool Q16>
+static void launch_csr(const CsrLayout& L, const float* child, int64_t nodes, hipStream_t st) {
+    const uintptr_t at = reinterpret_cast<uintptr_t>(child) | reinterpret_cast<uintptr_t>(L.out);
+    const int64_t batch = L.batch;
+    if (batch <= 64) {
+        launch_csr_cols<Q16, 1, 1>(L, child, nodes, run_nodes(nodes), st);
+        return;
+    }
+    if (batch > 128 && batch % 4 == 0 && (at & 15) == 0 && nodes >= 40000 && !slices_fit(batch)) {
+        if constexpr (Q16)
+            launch_cols<true, 4, 4>(L, child, nodes, batch, st);
+        else
+            launch_csr_cols<false, 4, 4>(L, child, nodes, batch <= 256 ? 2 : 1, st);
+        return;
+    }
+    const int npw = run_nodes(nodes * ((batch + 127) / 128));
+    if (batch % 2 == 0 && (at & 7) == 0)
+        launch_csr_cols<Q16, 2, 2>(L, child, nodes, npw, st);
+    else
+        launch_csr_cols<Q16, 1, 2>(L, child, nodes, npw, st);
 }
 
 // ---------------------------------------------------------------------------
@@ -435,20 +794,28 @@ static void launch(const LAYOUT& L, const float* child, const float* out_any, in
 // A term whose out[n_e, b] is -inf is 0: nothing flows through a node of
 // probability 0 (torch's autograd of logsumexp would give NaN there).
 // The kernel walks the transposed structure (CSC: for child c the edges that
-// point at it, each with its parent node): one wave per child row, every
-// 512-column tile of the batch in turn.  Each child row and each edge belongs
-// to one wave.  grad_child is accumulated in registers and written once.
-// grad_lw[e] is stored by the first column tile and, for batches over 512
-// columns, increased by the later tiles with a no-return atomic add; all of
-// these come from lane 0 of the one wave that owns edge e, in tile order, and
-// same-address accesses of one lane are performed in program order, so the
-// summation order is fixed and the result deterministic.
+// point at it, each with its parent node) the way csr_fwd_kernel walks the
+// nodes: a wave per run of children and column tile, tile-slowest, the two
+// parent rows of each of a group's edges in flight while a group folds.
+// grad_child is accumulated in registers and written once.
+//
+// The edges' weights and batch sums are scattered 4-byte accesses, once per
+// column tile.  So with several tiles csr_bwd_weights gathers the weights into
+// the walk's order first, each tile stores its sums in that order, coalesced,
+// in a workspace, and csr_bwd_sums adds the tiles' sums in tile order and
+// scatters them.  DIRECT, a single tile, takes them where they are and spares
+// two launches.  The summation order is fixed either way.  The 1M-child,
+// 8.0M-edge layer at batch 512 went from 6160 to 5316 us (two gathered rows an
+// edge, 33 GB; a wave per child over whole rows -> this); 200000 x 64 columns,
+// DIRECT, from 265 to 169.
 // ---------------------------------------------------------------------------
-struct ParentMeta {
-    int64_t node;
-    int64_t edge;
-    float lw;
-};
+// g * exp(t - o), or 0 where o is -inf or the place is not one of the batch's.
+// (The product is taken before the select: inside it the compiler branches
+// around the exponential, and waits for every load in flight there.)
+__device__ __forceinline__ float flow(float g, float t, float o, bool ok) {
+    const float x = g * fexp2((t - o) * kLog2e);
+    return ok && o != -kInf ? x : 0.0f;
+}
 
 __device__ __forceinline__ float wave_sum(float v) {
     v += reduce_partner<1>(v);
@@ -460,39 +827,243 @@ __device__ __forceinline__ float wave_sum(float v) {
     return v;
 }
 
+// Sums of four values over the wave: lane l ends with value l % 4's.
+__device__ __forceinline__ float wave_sum4(const float (&v)[4], int l) {
+    const bool odd = l & 1, hi = l & 2;
+    const float a = (odd ? v[1] : v[0]) + reduce_partner<1>(odd ? v[0] : v[1]);
+    const float b = (odd ? v[3] : v[2]) + reduce_partner<1>(odd ? v[2] : v[3]);
+    float s = (hi ? b : a) + reduce_partner<2>(hi ? a : b);
+    // row rotations by 4 and 8: the other quads of the row, lane for lane
+    s += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, s), 0x124, 0xF, 0xF, false));
+    s += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, s), 0x128, 0xF, 0xF, false));
+    s += reduce_partner<16>(s);
+    return s + reduce_partner<32>(s);
+}
+
+__global__ __launch_bounds__(256) void csr_bwd_weights(const float* __restrict__ logp,
+                                                       const int32_t* __restrict__ edges, float* __restrict__ lwc,
+                                                       int64_t nnz, int64_t block0) {
+    const int64_t k = (block0 + blockIdx.x) * 256 + threadIdx.x;
+    if (k < nnz) lwc[k] = logp[edges[k]];
+}
+
+__global__ __launch_bounds__(256) void csr_bwd_sums(const float* __restrict__ part, const int32_t* __restrict__ edges,
+                                                    float* __restrict__ glogp, int64_t nnz, int64_t tiles,
+                                                    int64_t block0) {
+    const int64_t k = (block0 + blockIdx.x) * 256 + threadIdx.x;
+    if (k >= nnz) return;
+    float s = part[k];
+    for (int64_t t = 1; t < tiles; ++t) s += part[t * nnz + k];
+    glogp[edges[k]] = s;
+}
+
+template <bool DIRECT, int VW, int P>
+__global__ __launch_bounds__(64) void csr_bwd_kernel(const float* __restrict__ child, const float* __restrict__ out,
+                                                     const float* __restrict__ gout, const float* __restrict__ logp,
+                                                     const int64_t* __restrict__ csc_off,
+                                                     const int32_t* __restrict__ csc_edge,
+                                                     const int32_t* __restrict__ csc_node,
+                                                     float* __restrict__ gchild, float* __restrict__ glogp,
+                                                     int64_t children, int64_t batch, int npw, int64_t tiles,
+                                                     int64_t unit0) {
+    // logp, glogp: by edge id with DIRECT, else in the walk's order (glogp: one
+    // such array per tile)
+    const int l = lane_id();
+    const int64_t unit = unit0 + blockIdx.x;
+    const int64_t runs = (children + npw - 1) / npw;
+    const int64_t tile = DIRECT ? 0 : unit / runs;
+    const int64_t n0 = (unit - tile * runs) * npw;
+    const int nn = (int)(children - n0 < npw ? children - n0 : npw);
+    const int64_t at = csc_off[n0 + (l < nn ? l : nn)];
+    const int64_t nnz = uniform64(csc_off[children]);
+    const int64_t e0 = uniform64(at);
+    const bool streamed = bcast64(at, nn) - e0 <= kRunEdges;
+    const int64_t b0 = tile * 64 * P;
+    const int rec = cols_bytes(batch, b0);
+    const float* child_b0 = child + b0;
+    const float* gout_b0 = gout + b0;
+    const float* out_b0 = out + b0;
+    const uint64_t row_bytes = (uint64_t)batch * 4u;
+    bool lane_ok[P];
+#pragma unroll
+    for (int i = 0; i < P; ++i) lane_ok[i] = Cols<VW, P>::ok(b0, l, batch, i);
+    float cv[P], acc[P];
+    if (streamed) {
+        const Run run{(int32_t)(at - e0)};
+        const u32x4v rn = words_rsrc(csc_node + e0, nnz - e0);
+        const u32x4v rw = DIRECT ? words_rsrc(csc_edge + e0, nnz - e0) : words_rsrc(logp + e0, nnz - e0);
+        // ids: the parents; w: the weights, or with DIRECT the edge ids
+        struct Meta {
+            u32x4v ids, w;
+        };
+        const auto load_meta = [&](const Group& g) {
+            return Meta{s_buffer_load4(rn, g.e * 4, 0), s_buffer_load4(rw, g.e * 4, 0)};
+        };
+        struct Rows {
+            float x[P], g[G][P], o[G][P], lw[G];
+        };
+        const auto load_rows = [&](Rows& v, const Meta& em, const Group& g) {
+            load_cols_buf<VW, P>(child_b0 + (n0 + (g.node < nn ? g.node : 0)) * batch,
+                                 g.first && g.node < nn ? rec : 0, l, v.x);
+#pragma unroll
+            for (int k = 0; k < G; ++k) {
+                const uint64_t row = (uint64_t)em.ids[k] * row_bytes;
+                const int r = k < g.left ? rec : 0;
+                load_cols_buf<VW, P>(reinterpret_cast<const float*>(reinterpret_cast<const char*>(gout_b0) + row), r,
+                                     l, v.g[k]);
+                load_cols_buf<VW, P>(reinterpret_cast<const float*>(reinterpret_cast<const char*>(out_b0) + row), r,
+                                     l, v.o[k]);
+            }
+            if constexpr (DIRECT) {
+#pragma unroll
+                for (int k = 0; k < G; ++k)
+                    v.lw[k] = logp[k < g.left ? (uint32_t)em.w[k] : 0u];
+            } else {
+#pragma unroll
+                for (int k = 0; k < G; ++k) v.lw[k] = __builtin_bit_cast(float, (uint32_t)em.w[k]);
+            }
+        };
+        const auto fold = [&](const Rows& v, const Meta& em, const Group& g) {
+            if (g.first) {
+#pragma unroll
+                for (int i = 0; i < P; ++i) {
+                    cv[i] = v.x[i];
+                    acc[i] = 0.0f;
+                }
+            }
+            float t[G];
+#pragma unroll
+            for (int k = 0; k < G; ++k) {
+                t[k] = 0.0f;
+#pragma unroll
+                for (int i = 0; i < P; ++i) {
+                    const float x = flow(v.g[k][i], v.lw[k] + cv[i], v.o[k][i], lane_ok[i] && k < g.left);
+                    acc[i] += x;
+                    t[k] += x;
+                }
+            }
+            const float s = wave_sum4(t, l);
+            if constexpr (DIRECT) {
+                const uint32_t lo = l & 1 ? em.w[1] : em.w[0], hi = l & 1 ? em.w[3] : em.w[2];
+                float* dst = glogp + (l & 2 ? hi : lo);
+                if (l < 4 && l < g.left) *dst = s;
+            } else {
+                if (l < 4 && l < g.left) glogp[tile * nnz + e0 + g.e + l] = s;
+            }
+            if (g.left <= G && g.node < nn) Cols<VW, P>::store(gchild + (n0 + g.node) * batch, b0, l, batch, acc);
+        };
+        Rows va, vb;
+        Group ga = {0, 0, run.start(1), 1, 0};
+        Meta ma = load_meta(ga);
+        load_rows(va, ma, ga);
+        Group gb = run.next(ga);
+        Meta mb = load_meta(gb);
+        while (true) {
+            load_rows(vb, mb, gb);
+            const Group gc = run.next(gb);
+            const Meta mc = load_meta(gc);
+            fold(va, ma, ga);
+            load_rows(va, mc, gc);
+            const Group gd = run.next(gc);
+            const Meta md = load_meta(gd);
+            fold(vb, mb, gb);
+            if (gc.node >= nn) break;
+            ga = gc;
+            ma = mc;
+            gb = gd;
+            mb = md;
+        }
+    } else {  // too many edges for the stream's 32-bit edge numbers: one at a time
+        for (int c = 0; c < nn; ++c) {
+            load_cols_buf<VW, P>(child_b0 + (n0 + c) * batch, rec, l, cv);
+#pragma unroll
+            for (int i = 0; i < P; ++i) acc[i] = 0.0f;
+            for (int64_t k = bcast64(at, c); k < bcast64(at, c + 1); ++k) {
+                float g[P], o[P], t = 0.0f;
+                const int64_t row = (int64_t)csc_node[k] * batch, e = csc_edge[k];
+                load_cols_buf<VW, P>(gout_b0 + row, rec, l, g);
+                load_cols_buf<VW, P>(out_b0 + row, rec, l, o);
+                const float lw = logp[DIRECT ? e : k];
+#pragma unroll
+                for (int i = 0; i < P; ++i) {
+                    const float x = flow(g[i], lw + cv[i], o[i], lane_ok[i]);
+                    acc[i] += x;
+                    t += x;
+                }
+                t = wave_sum(t);
+                if (l == 0) glogp[DIRECT ? e : tile * nnz + k] = t;
+            }
+            Cols<VW, P>::store(gchild + (n0 + c) * batch, b0, l, batch, acc);
+        }
+    }
+}
+
+template <bool DIRECT, int VW, int P>
+static void launch_csr_bwd_cols(const float* child, const float* out, const float* gout, const float* logp,
+                                const int64_t* off, const int32_t* edge, const int32_t* node, float* gchild,
+                                float* glogp, int64_t children, int64_t batch, hipStream_t st) {
+    const int64_t tiles = (batch + 64 * P - 1) / (64 * P);
+    const int npw = run_nodes(DIRECT ? children : children * tiles);
+    const int64_t runs = (children + npw - 1) / npw;
+    for_grid_chunks(DIRECT ? runs : runs * tiles, 64, [&](int64_t u0, int64_t n) {
+        csr_bwd_kernel<DIRECT, VW, P><<<dim3((unsigned)n), dim3(64), 0, st>>>(
+            child, out, gout, logp, off, edge, node, gchild, glogp, children, batch, npw, tiles, u0);
+    });
+}
+
+// Columns of a tile of the backward at this batch (200000 children, us, tiles
+// of 64 / 128 / 256 columns: batch 64 169 / 181 / 245, 128 281 / 264 / 273, 512
+// 970 / 973 / 1039; 1M children, batch 512 5285 / 5316 / 5175 at their best run
+// lengths).
+static int64_t bwd_tile_cols(int64_t batch) { return batch <= 64 ? 64 : 128; }
+
+template <bool DIRECT>
+static void launch_csr_bwd(const float* child, const float* out, const float* gout, const float* logp,
+                           const int64_t* off, const int32_t* edge, const int32_t* node, float* gchild, float* glogp,
+                           int64_t children, int64_t batch, hipStream_t st) {
+    const uintptr_t at = reinterpret_cast<uintptr_t>(child) | reinterpret_cast<uintptr_t>(out) |
+                         reinterpret_cast<uintptr_t>(gout) | reinterpret_cast<uintptr_t>(gchild);
+    if (bwd_tile_cols(batch) == 64)
+        launch_csr_bwd_cols<DIRECT, 1, 1>(child, out, gout, logp, off, edge, node, gchild, glogp, children, batch, st);
+    else if (batch % 2 == 0 && (at & 7) == 0)
+        launch_csr_bwd_cols<DIRECT, 2, 2>(child, out, gout, logp, off, edge, node, gchild, glogp, children, batch, st);
+    else
+        launch_csr_bwd_cols<DIRECT, 1, 2>(child, out, gout, logp, off, edge, node, gchild, glogp, children, batch, st);
+}
+
+// Several column tiles without a workspace: one wave per child row (four to a
+// block), every 512-column tile in turn, its parents' rows one edge ahead.  The
+// first tile stores an edge's sum and the later ones add to it with a no-return
+// atomic, all from lane 0 of the wave that owns the edge, in tile order.
+struct ParentMeta {
+    int64_t node;
+    int64_t edge;
+    float lw;
+};
+
+constexpr int PB = 8;  // columns per lane
 // Parent edges per load group (two rows each), and columns per lane: 8 columns
 // and single-edge groups measured 7.2 ms on the 1M-node C5 layer, against
 // 7.8 ms for 4 columns and two-edge groups; the forward keeps 4 columns (8
 // measured 3.8 ms against 3.45 ms).
 constexpr int GB = 1;
 
-template <bool VEC>
+template <int VW>
 __device__ __forceinline__ void load_parents(float (&gv)[GB][PB], float (&ov)[GB][PB], const ParentMeta& pw, int j,
                                              int wn, const float* __restrict__ gout, const float* __restrict__ out,
                                              int64_t batch, int64_t b0, int l) {
-    if constexpr (VEC) {
-        // every load issued, as in load_group: parents past wn read empty ranges
-        const int rec = cols_bytes(batch, b0);
+    // every load issued, as in load_group: parents past wn read empty ranges
+    const int rec = cols_bytes(batch, b0);
 #pragma unroll
-        for (int g = 0; g < GB; ++g) {
-            const int64_t n = bcast64(pw.node, (j + g) & 63);
-            const int r = j + g < wn ? rec : 0;
-            load_cols_buf<PB>(gout + n * batch + b0, r, l, gv[g]);
-            load_cols_buf<PB>(out + n * batch + b0, r, l, ov[g]);
-        }
-    } else {
-#pragma unroll
-        for (int g = 0; g < GB; ++g) {
-            if (j + g < wn) {
-                const int64_t n = bcast64(pw.node, j + g);
-                Cols<VEC, PB>::load(gout + n * batch, b0, l, batch, gv[g]);
-                Cols<VEC, PB>::load(out + n * batch, b0, l, batch, ov[g]);
-            }
-        }
+    for (int g = 0; g < GB; ++g) {
+        const int64_t n = bcast64(pw.node, (j + g) & 63);
+        const int r = j + g < wn ? rec : 0;
+        load_cols_buf<VW, PB>(gout + n * batch + b0, r, l, gv[g]);
+        load_cols_buf<VW, PB>(out + n * batch + b0, r, l, ov[g]);
     }
 }
 
-template <bool VEC>
+template <int VW>
 __device__ __forceinline__ void flow_group(const float (&gv)[GB][PB], const float (&ov)[GB][PB], const ParentMeta& pw,
                                            int j, int wn, const float (&cv)[PB], float (&acc)[PB], bool first_tile,
                                            float* __restrict__ glogp, int64_t batch, int64_t b0, int l) {
@@ -503,8 +1074,7 @@ __device__ __forceinline__ void flow_group(const float (&gv)[GB][PB], const floa
             float tsum = 0.0f;
 #pragma unroll
             for (int i = 0; i < PB; ++i) {
-                const bool live = Cols<VEC, PB>::ok(b0, l, batch, i) && ov[g][i] != -kInf;
-                const float t = live ? gv[g][i] * fexp2((lw + cv[i] - ov[g][i]) * kLog2e) : 0.0f;
+                const float t = flow(gv[g][i], lw + cv[i], ov[g][i], Cols<VW, PB>::ok(b0, l, batch, i));
                 acc[i] += t;
                 tsum += t;
             }
@@ -523,8 +1093,8 @@ __device__ __forceinline__ void flow_group(const float (&gv)[GB][PB], const floa
     }
 }
 
-template <bool VEC, int WPB>
-__global__ __launch_bounds__(64 * WPB) void csr_bwd_kernel(const float* __restrict__ child, const float* __restrict__ out,
+template <int VW>
+__global__ __launch_bounds__(256) void csr_bwd_rows_kernel(const float* __restrict__ child, const float* __restrict__ out,
                                                       const float* __restrict__ gout, const float* __restrict__ logp,
                                                       const int64_t* __restrict__ csc_off,
                                                       const int32_t* __restrict__ csc_edge,
@@ -533,16 +1103,13 @@ __global__ __launch_bounds__(64 * WPB) void csr_bwd_kernel(const float* __restri
                                                       int64_t children, int64_t batch, int64_t block0) {
     const int l = lane_id();
     const int64_t c =
-        (block0 + (int64_t)blockIdx.x) * WPB + (WPB > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0);
+        (block0 + (int64_t)blockIdx.x) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (c >= children) return;
     const int64_t p0 = uniform64(csc_off[c]);
     const int64_t k = uniform64(csc_off[c + 1]) - p0;
     for (int64_t b0 = 0; b0 < batch; b0 += 64 * PB) {
         float cv[PB], acc[PB];
-        if constexpr (VEC)
-            load_cols_buf<PB>(child + c * batch + b0, cols_bytes(batch, b0), l, cv);
-        else
-            Cols<VEC, PB>::load(child + c * batch, b0, l, batch, cv);
+        load_cols_buf<VW, PB>(child + c * batch + b0, cols_bytes(batch, b0), l, cv);
 #pragma unroll
         for (int i = 0; i < PB; ++i) acc[i] = 0.0f;
         for (int64_t w0 = 0; w0 < k; w0 += 64) {
@@ -554,18 +1121,43 @@ __global__ __launch_bounds__(64 * WPB) void csr_bwd_kernel(const float* __restri
             const int wn = (int)(k - w0 < 64 ? k - w0 : 64);
             const int ng = (wn + GB - 1) / GB;
             float ga[GB][PB], oa[GB][PB], gb[GB][PB], ob[GB][PB];
-            load_parents<VEC>(ga, oa, pw, 0, wn, gout, out, batch, b0, l);
+            load_parents<VW>(ga, oa, pw, 0, wn, gout, out, batch, b0, l);
             int gi = 0;
             for (; gi + 1 < ng; gi += 2) {
-                load_parents<VEC>(gb, ob, pw, (gi + 1) * GB, wn, gout, out, batch, b0, l);
-                flow_group<VEC>(ga, oa, pw, gi * GB, wn, cv, acc, b0 == 0, glogp, batch, b0, l);
-                if (VEC || gi + 2 < ng) load_parents<VEC>(ga, oa, pw, (gi + 2) * GB, wn, gout, out, batch, b0, l);
-                flow_group<VEC>(gb, ob, pw, (gi + 1) * GB, wn, cv, acc, b0 == 0, glogp, batch, b0, l);
+                load_parents<VW>(gb, ob, pw, (gi + 1) * GB, wn, gout, out, batch, b0, l);
+                flow_group<VW>(ga, oa, pw, gi * GB, wn, cv, acc, b0 == 0, glogp, batch, b0, l);
+                load_parents<VW>(ga, oa, pw, (gi + 2) * GB, wn, gout, out, batch, b0, l);
+                flow_group<VW>(gb, ob, pw, (gi + 1) * GB, wn, cv, acc, b0 == 0, glogp, batch, b0, l);
             }
-            if (gi < ng) flow_group<VEC>(ga, oa, pw, gi * GB, wn, cv, acc, b0 == 0, glogp, batch, b0, l);
+            if (gi < ng) flow_group<VW>(ga, oa, pw, gi * GB, wn, cv, acc, b0 == 0, glogp, batch, b0, l);
         }
-        Cols<VEC, PB>::store(gchild + c * batch, b0, l, batch, acc);
+        Cols<VW, PB>::store(gchild + c * batch, b0, l, batch, acc);
     }
+}
+
+static void launch_csr_bwd_rows(const float* child, const float* out, const float* gout, const float* logp,
+                                const int64_t* off, const int32_t* edge, const int32_t* node, float* gchild,
+                                float* glogp, int64_t children, int64_t batch, hipStream_t st) {
+    const uintptr_t at = reinterpret_cast<uintptr_t>(child) | reinterpret_cast<uintptr_t>(out) |
+                         reinterpret_cast<uintptr_t>(gout) | reinterpret_cast<uintptr_t>(gchild);
+    for_grid_chunks((children + 3) / 4, 256, [&](int64_t b0, int64_t nb) {
+        if (batch % 4 == 0 && (at & 15) == 0)
+            csr_bwd_rows_kernel<4><<<dim3((unsigned)nb), dim3(256), 0, st>>>(child, out, gout, logp, off, edge, node,
+                                                                            gchild, glogp, children, batch, b0);
+        else
+            csr_bwd_rows_kernel<1><<<dim3((unsigned)nb), dim3(256), 0, st>>>(child, out, gout, logp, off, edge, node,
+                                                                            gchild, glogp, children, batch, b0);
+    });
+}
+
+// Without a workspace.
+static void launch_csr_bwd_plain(const float* child, const float* out, const float* gout, const float* logp,
+                                 const int64_t* off, const int32_t* edge, const int32_t* node, float* gchild,
+                                 float* glogp, int64_t children, int64_t batch, hipStream_t st) {
+    if (batch <= bwd_tile_cols(batch))
+        launch_csr_bwd<true>(child, out, gout, logp, off, edge, node, gchild, glogp, children, batch, st);
+    else
+        launch_csr_bwd_rows(child, out, gout, logp, off, edge, node, gchild, glogp, children, batch, st);
 }
 
 }  // namespace sparse
@@ -583,19 +1175,55 @@ extern "C" int fl_sparse_csr_bwd(const float* child, const float* out, const flo
     FL_CHECK(child && out && grad_out && logparams && csc_offsets && csc_edges && csc_nodes && grad_child &&
                  grad_logparams,
              "%s: NULL pointer argument", name);
-    const bool vec = (batch % 4 == 0) && ((reinterpret_cast<uintptr_t>(child) | reinterpret_cast<uintptr_t>(out) |
-                                           reinterpret_cast<uintptr_t>(grad_out) |
-                                           reinterpret_cast<uintptr_t>(grad_child)) & 15) == 0;
+    sparse::launch_csr_bwd_plain(child, out, grad_out, logparams, csc_offsets, csc_edges, csc_nodes, grad_child,
+                                 grad_logparams, num_children, batch, reinterpret_cast<hipStream_t>(stream));
+    return launch_status(name);
+}
+
+// The workspace form is for slices that fit (slices_fit; 500000 x 400 took 2540
+// us in them against 2099 in whole rows) of layers of at least 64000 (child,
+// column tile) pairs: it pays two more launches (us, workspace / none: 2000 x
+// 512 20 / 13, 12000 x 512 58 / 53, 20000 x 512 89 / 97, 50000 x 512 227 / 265).
+extern "C" size_t fl_sparse_csr_bwd_workspace_bytes(int64_t num_children, int64_t nnz, int64_t batch) {
+    if (nnz <= 0 || batch <= 0) return 0;
+    const int64_t cols = sparse::bwd_tile_cols(batch);
+    const int64_t tiles = (batch + cols - 1) / cols;
+    if (tiles < 2 || num_children * tiles < 64000 || !sparse::slices_fit(batch)) return 0;
+    return (size_t)nnz * (size_t)(tiles + 1) * sizeof(float);
+}
+
+extern "C" int fl_sparse_csr_bwd_ws(const float* child, const float* out, const float* grad_out,
+                                    const float* logparams, const int64_t* csc_offsets, const int32_t* csc_edges,
+                                    const int32_t* csc_nodes, float* grad_child, float* grad_logparams,
+                                    int64_t num_children, int64_t nnz, int64_t batch, void* workspace,
+                                    size_t workspace_bytes, void* stream) {
+    const char* name = "fl_sparse_csr_bwd_ws";
+    FL_CHECK(num_children >= 0 && nnz >= 0 && batch >= 0, "%s: negative size", name);
+    if (num_children == 0 || batch == 0) return ok();
+    FL_CHECK(child && out && grad_out && logparams && csc_offsets && csc_edges && csc_nodes && grad_child &&
+                 grad_logparams,
+             "%s: NULL pointer argument", name);
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    for_grid_chunks((num_children + 3) / 4, 256, [&](int64_t b0, int64_t nb) {
-        if (vec)
-            sparse::csr_bwd_kernel<true, 4><<<dim3((unsigned)nb), dim3(256), 0, st>>>(
-                child, out, grad_out, logparams, csc_offsets, csc_edges, csc_nodes, grad_child, grad_logparams,
-                num_children, batch, b0);
-        else
-            sparse::csr_bwd_kernel<false, 4><<<dim3((unsigned)nb), dim3(256), 0, st>>>(
-                child, out, grad_out, logparams, csc_offsets, csc_edges, csc_nodes, grad_child, grad_logparams,
-                num_children, batch, b0);
+    const size_t need = fl_sparse_csr_bwd_workspace_bytes(num_children, nnz, batch);
+    if (need == 0) {
+        sparse::launch_csr_bwd_plain(child, out, grad_out, logparams, csc_offsets, csc_edges, csc_nodes, grad_child,
+                                     grad_logparams, num_children, batch, st);
+        return launch_status(name);
+    }
+    FL_CHECK(workspace != nullptr && workspace_bytes >= need, "%s: workspace of %llu bytes, %llu needed", name,
+             (unsigned long long)workspace_bytes, (unsigned long long)need);
+    FL_CHECK((reinterpret_cast<uintptr_t>(workspace) & 3u) == 0, "%s: workspace is not 4-byte aligned", name);
+    const int64_t cols = sparse::bwd_tile_cols(batch);
+    const int64_t tiles = (batch + cols - 1) / cols;
+    float* lwc = static_cast<float*>(workspace);
+    float* part = lwc + nnz;
+    for_grid_chunks((nnz + 255) / 256, 256, [&](int64_t b0, int64_t nb) {
+        sparse::csr_bwd_weights<<<dim3((unsigned)nb), dim3(256), 0, st>>>(logparams, csc_edges, lwc, nnz, b0);
+    });
+    sparse::launch_csr_bwd<false>(child, out, grad_out, lwc, csc_offsets, csc_edges, csc_nodes, grad_child, part,
+                                  num_children, batch, st);
+    for_grid_chunks((nnz + 255) / 256, 256, [&](int64_t b0, int64_t nb) {
+        sparse::csr_bwd_sums<<<dim3((unsigned)nb), dim3(256), 0, st>>>(part, csc_edges, grad_logparams, nnz, tiles, b0);
     });
     return launch_status(name);
 }
@@ -610,9 +1238,9 @@ extern "C" int fl_sparse_csr_fwd(const float* child, const int64_t* offsets, con
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     const sparse::CsrLayout L{offsets, child_ids, logparams, out, batch};
     if (q16)
-        sparse::launch<true>(L, child, out, num_nodes, batch, st);
+        sparse::launch_csr<true>(L, child, num_nodes, st);
     else
-        sparse::launch<false>(L, child, out, num_nodes, batch, st);
+        sparse::launch_csr<false>(L, child, num_nodes, st);
     return launch_status(name);
 }
 

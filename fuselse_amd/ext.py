@@ -600,10 +600,7 @@ def sparse_blocked_backward(node_flows, element_flows, node_mars, element_mars, 
         logp = (w if params_are_log else torch.log(torch.clamp_min(w, 1e-45))).contiguous()
         grad_el = torch.empty_like(element_mars)
         grad_lp = torch.empty_like(logp)
-        with _on_device(element_mars):
-            _lib.call("fl_sparse_csr_bwd", element_mars.data_ptr(), node_mars.data_ptr(), node_flows.data_ptr(),
-                      logp.data_ptr(), csc_off.data_ptr(), csc_edge.data_ptr(), csc_node.data_ptr(), grad_el.data_ptr(),
-                      grad_lp.data_ptr(), num_el, batch, _stream(element_mars))
+        _launch_csr_bwd(element_mars, node_mars, node_flows, logp, csc_off, csc_edge, csc_node, grad_el, grad_lp)
         element_flows.add_(grad_el)
         param_flows.view(-1).index_add_(0, q, grad_lp)
         return None
@@ -699,8 +696,19 @@ def sparse_csr_backward(child, out, grad_out, offsets, child_ids, logparams, csc
     if child_ids.numel() == 0:
         grad_child.zero_()
         return grad_child, grad_logp
-    with _on_device(child):
-        _lib.call("fl_sparse_csr_bwd", child.data_ptr(), out.data_ptr(), grad_out.data_ptr(), logparams.data_ptr(),
-                  csc_off.data_ptr(), csc_edge.data_ptr(), csc_node.data_ptr(), grad_child.data_ptr(),
-                  grad_logp.data_ptr(), num_children, batch, _stream(child))
+    _launch_csr_bwd(child, out, grad_out, logparams, csc_off, csc_edge, csc_node, grad_child, grad_logp)
     return grad_child, grad_logp
+
+
+def _launch_csr_bwd(child, out, grad_out, logparams, csc_off, csc_edge, csc_node, grad_child, grad_logp):
+    num_children, batch = child.shape
+    nnz = csc_edge.numel()
+    with _on_device(child):
+        nbytes = _lib.load().fl_sparse_csr_bwd_workspace_bytes(num_children, nnz, batch)
+        # the weights and sums in the walk's order; stream-ordered reuse by
+        # torch's caching allocator keeps it valid until the kernels have run
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=child.device) if nbytes else None
+        _lib.call("fl_sparse_csr_bwd_ws", child.data_ptr(), out.data_ptr(), grad_out.data_ptr(), logparams.data_ptr(),
+                  csc_off.data_ptr(), csc_edge.data_ptr(), csc_node.data_ptr(), grad_child.data_ptr(),
+                  grad_logp.data_ptr(), num_children, nnz, batch, ws.data_ptr() if ws is not None else None, nbytes,
+                  _stream(child))

@@ -231,13 +231,28 @@ int fl_sparse_blocked_fwd(float* node_mars, const float* element_mars, const flo
  * [num_children, batch]; out, grad_out: fp32 [num_nodes, batch]; both
  * gradients are written (not accumulated).  Deterministic: one wave owns each
  * child row and each edge.  grad_child is written once; grad_logparams[e] is
- * stored by the first 512-column tile of the batch and, when batch > 512,
- * increased by the later tiles with atomic adds from that same wave in tile
- * order, so the summation order is fixed.
+ * stored by the first column tile of the batch (64 columns up to a batch of 64,
+ * else 128) and increased by the later tiles with atomic adds from that same
+ * wave in tile order, so the summation order is fixed.
  * ------------------------------------------------------------------------- */
 int fl_sparse_csr_bwd(const float* child, const float* out, const float* grad_out, const float* logparams,
                       const int64_t* csc_offsets, const int32_t* csc_edges, const int32_t* csc_nodes,
                       float* grad_child, float* grad_logparams, int64_t num_children, int64_t batch, void* stream);
+
+/* ---------------------------------------------------------------------------
+ * The same with a caller workspace of
+ * fl_sparse_csr_bwd_workspace_bytes(num_children, nnz, batch) bytes (0: none needed, NULL
+ * will do), 4-byte aligned, any contents: the edges' weights and batch sums
+ * then pass through it in the walk's order instead of being gathered and
+ * scattered once per column tile, and the tiles go one after the other over
+ * all children.  nnz is csc_offsets[num_children].  Deterministic; the sum of
+ * an edge over the batch adds the tiles' sums in tile order.
+ * ------------------------------------------------------------------------- */
+size_t fl_sparse_csr_bwd_workspace_bytes(int64_t num_children, int64_t nnz, int64_t batch);
+int fl_sparse_csr_bwd_ws(const float* child, const float* out, const float* grad_out, const float* logparams,
+                         const int64_t* csc_offsets, const int32_t* csc_edges, const int32_t* csc_nodes,
+                         float* grad_child, float* grad_logparams, int64_t num_children, int64_t nnz,
+                         int64_t batch, void* workspace, size_t workspace_bytes, void* stream);
 
 /* ---------------------------------------------------------------------------
  * Block-layout backward ("flows") of fl_sparse_blocked_fwd in fp32 (the

@@ -682,3 +682,134 @@ def test_blocked_layer_autograd_two_layers(cuda, bs1, bs2):
     np.testing.assert_allclose(y, yt.detach().numpy(), rtol=1e-5, atol=1e-5)
     for got, want in ((gx, xt.grad), (g1, w1t.grad), (g2, w2t.grad)):
         np.testing.assert_allclose(got, want.numpy(), rtol=1e-4, atol=1e-5)
+
+
+def _csr_fp64_torch(child, off, cids, lp):
+    """The CSR sum layer in float64 with torch's scatter operations, for layers
+    the per-node oracle is too slow for (finite inputs, no empty nodes)."""
+    nodes, width = off.numel() - 1, child.shape[1]
+    parent = torch.repeat_interleave(torch.arange(nodes, device=child.device), off.diff())
+    t = lp.double()[:, None] + child.double()[cids.long()]
+    top = torch.full((nodes, width), float("-inf"), dtype=torch.float64, device=child.device)
+    top.scatter_reduce_(0, parent[:, None].expand(-1, width), t, "amax")
+    total = torch.zeros_like(top).index_add_(0, parent, torch.exp(t - top[parent]))
+    return top + torch.log(total), parent, t
+
+
+@pytest.mark.parametrize("nodes,batch", [(61, 1), (61, 63), (61, 64), (61, 65), (61, 127), (61, 128), (61, 129),
+                                         (61, 256), (61, 510), (40001, 3), (20001, 130), (160003, 1), (40001, 200),
+                                         (40001, 132)])
+def test_csr_forward_runs(cuda, nodes, batch):
+    """The streamed forward around its column tiles (64, 128, 256 columns, odd
+    batches), run lengths of 1, 2 and 4 nodes and a run cut short, with empty
+    nodes at the run's start, middle and end, groups of every remainder and
+    every chain count of the Q16.16 tree."""
+    print(f"case csr runs {nodes}x{batch}", flush=True)
+    rng = np.random.default_rng(nodes + batch)
+    fan = O.powerlaw_fanin(nodes, seed=batch)
+    fan[:20] = [0, 1, 2, 3, 4, 5, 0, 0, 8, 9, 256, 16, 17, 32, 33, 36, 40, 63, 64, 65]
+    fan[-3:] = [0, 1, 0]
+    off, cids, lp = _csr(rng, nodes, 300, fanin=fan)
+    child = np.log(rng.random((300, batch)) + 1e-12).astype(np.float32)
+    ch, offd, cid, lpd = _to(cuda, child, off, cids, lp)
+    ext = _ext()
+    got = ext.sparse_csr_forward(ch, offd, cid, lpd).cpu().numpy()
+    np.testing.assert_allclose(got, O.sparse_csr_fp64(child, off, cids, lp), rtol=1e-5, atol=1e-6)
+    gq = ext.sparse_csr_forward(ch, offd, cid, lpd, q16=True).cpu().numpy()
+    np.testing.assert_array_equal(gq.view(np.int32), O.sparse_q16_csr(child, off, cids, lp).view(np.int32))
+
+
+@pytest.mark.parametrize("batch", [5, 130])
+def test_csr_forward_special_values(cuda, batch):
+    """-inf, +inf, NaN and magnitudes past the fused exponent's range, in a
+    node's first group and in later ones."""
+    print(f"case csr special {batch}", flush=True)
+    rng = np.random.default_rng(batch)
+    nodes, nch = 200, 24
+    off, cids, lp = _csr(rng, nodes, nch, fanin=rng.integers(1, 14, nodes))
+    child = (rng.standard_normal((nch, batch)) * 3).astype(np.float32)
+    child[0] = -np.inf
+    child[1, ::2] = np.inf
+    child[2, ::3] = np.nan
+    child[3] = 3e7
+    child[4, 1::2] = -3e7
+    lp[::11] = -np.inf
+    ch, offd, cid, lpd = _to(cuda, child, off, cids, lp)
+    got = _ext().sparse_csr_forward(ch, offd, cid, lpd).cpu().numpy()
+    np.testing.assert_allclose(got, O.sparse_csr_fp64(child, off, cids, lp), rtol=1e-5, atol=1e-6)
+
+
+def test_csr_q16_saturated_pairs(cuda):
+    """Logits around the int32 limit (22713.2 saturates) and around the clamp
+    at -20000, so that differences reach 2^32 and a maximum plus its correction
+    passes 2^31: every bit as in the reference's 32-bit arithmetic."""
+    rng = np.random.default_rng(9)
+    nodes, nch, batch = 300, 64, 70
+    off, cids, _ = _csr(rng, nodes, nch, fanin=rng.integers(1, 40, nodes))
+    lp = np.zeros(off[-1], np.float32)
+    child = rng.choice(np.float32([22713.3, 22713.2, 22713.1, 22713, 22702, 22701.5, 22690, 0, -20000, -3e4, -np.inf,
+                                   np.inf, -11356, -11355.9]), (nch, batch)).astype(np.float32)
+    ch, offd, cid, lpd = _to(cuda, child, off, cids, lp)
+    gq = _ext().sparse_csr_forward(ch, offd, cid, lpd, q16=True).cpu().numpy()
+    np.testing.assert_array_equal(gq.view(np.int32), O.sparse_q16_csr(child, off, cids, lp).view(np.int32))
+
+
+@pytest.mark.parametrize("nodes,children,batch", [(300, 61, 1), (300, 61, 64), (300, 61, 65), (300, 61, 128),
+                                                  (30000, 40001, 3), (20000, 16100, 512), (20000, 22000, 384)])
+def test_csr_backward_runs(cuda, nodes, children, batch):
+    """The streamed backward: one tile (weights and sums by edge id) and, from
+    64000 (child, tile) pairs, several tiles through the workspace; children
+    without edges; twice the same bits.  A sum's error is bounded by 1e-5 of
+    its terms' magnitudes."""
+    print(f"case csr bwd runs {nodes} {children} {batch}", flush=True)
+    rng = np.random.default_rng(children + batch)
+    off, cids, lp = _csr(rng, nodes, children, fanin=np.maximum(O.powerlaw_fanin(nodes, seed=batch), 1))
+    cids[cids % 50 == 7] = 0  # some children without edges, one with many
+    ch, offd, cid, lpd = _to(cuda, np.log(rng.random((children, batch)) + 1e-12).astype(np.float32), off, cids, lp)
+    ext = _ext()
+    gen = torch.Generator(device=cuda)
+    gen.manual_seed(3)
+    out = ext.sparse_csr_forward(ch, offd, cid, lpd)
+    gout = torch.randn(nodes, batch, device=cuda, generator=gen)
+    csc = ext.sparse_csr_transpose(offd, cid, children)
+    gc, gl = ext.sparse_csr_backward(ch, out, gout, offd, cid, lpd, csc)
+    gc2, gl2 = ext.sparse_csr_backward(ch, out, gout, offd, cid, lpd, csc)
+    assert torch.equal(gc, gc2) and torch.equal(gl, gl2)
+    out64, parent, t = _csr_fp64_torch(ch, offd, cid, lpd)
+    term = torch.exp(t - out64[parent]) * gout.double()[parent]
+    assert ((gl.double() - term.sum(1)).abs() <= 1e-5 * term.abs().sum(1) + 1e-30).all()
+    want = torch.zeros(children, batch, dtype=torch.float64, device=cuda)
+    size = want.clone().index_add_(0, cid.long(), term.abs())
+    want.index_add_(0, cid.long(), term)
+    assert ((gc.double() - want).abs() <= 1e-5 * size + 1e-30).all()
+
+
+@pytest.mark.parametrize("batch", [3, 130])
+def test_csr_runs_past_the_streams_edges(cuda, batch):
+    """A node, and a child, of more edges than the stream's 32-bit edge numbers
+    are for (2^20 a run), between ordinary ones."""
+    print(f"case csr long run {batch}", flush=True)
+    big = (1 << 20) + 7
+    fan = np.array([3, big, 0, 9], np.int64)
+    rng = np.random.default_rng(batch)
+    off, cids, lp = _csr(rng, 4, 50, fanin=fan)
+    child = np.log(rng.random((50, batch)) + 1e-12).astype(np.float32)
+    ch, offd, cid, lpd = _to(cuda, child, off, cids, lp)
+    ext = _ext()
+    got = ext.sparse_csr_forward(ch, offd, cid, lpd).cpu().numpy()
+    np.testing.assert_allclose(got, O.sparse_csr_fp64(child, off, cids, lp), rtol=1e-5, atol=1e-6)
+    gq = ext.sparse_csr_forward(ch, offd, cid, lpd, q16=True).cpu().numpy()
+    np.testing.assert_array_equal(gq.view(np.int32), O.sparse_q16_csr(child, off, cids, lp).view(np.int32))
+    if batch > 128:
+        return
+    # one edge to each of `big` nodes from child 1, and a few more
+    off = torch.arange(big + 2, device=cuda)
+    cid = torch.ones(big + 1, dtype=torch.int32, device=cuda)
+    cid[-1] = 0
+    ch = torch.zeros(3, batch, device=cuda)
+    lpd = torch.zeros(big + 1, device=cuda)
+    out = ext.sparse_csr_forward(ch, off, cid, lpd)
+    gout = torch.ones_like(out)
+    gc, gl = ext.sparse_csr_backward(ch, out, gout, off, cid, lpd)
+    want = torch.tensor([1.0, float(big), 0.0], device=cuda)
+    assert torch.equal(gc, want[:, None].expand(3, batch)) and torch.equal(gl, torch.full_like(gl, float(batch)))
