@@ -56,6 +56,8 @@ SIGNATURES = {
     "fl_sparse_blocked_fwd": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _int, _vp]),
     "fl_sparse_blocked_bwd": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _int, _vp, _vp,
                                      _i64, _vp, _vp, _vp, _vp]),
+    "fl_sparse_blocked_grad": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _int, _int, _vp,
+                                      _vp, _i64, _vp, _vp, _vp, _vp]),
 }
 
 # the measurement library (include/fuselse_amd_diag.h)

@@ -579,8 +579,20 @@ __global__ __launch_bounds__(64) void blocked_bwd_params(float* __restrict__ par
 // default allocation took 197 + 48 AGPRs; 448 -> 443 us), 16 parents run
 // three waves per SIMD instead of two, and rows that are not 16-byte vectors
 // two instead of one.
-template <int ET, int NKP, bool VEC, bool LOGP, bool NTP>
+//
+// SET (element_flows is written, not added to): the flows of an edge that is
+// its element row's only one go straight to that row, not through the
+// workspace; where each of the chunk's rows goes is held in LDS.  At the bench
+// layer (8192 blocks of 32, 32 edges, 262144 element rows) 37% of the edges are
+// such; with the element rows and parameters written instead of cleared and
+// added to, and the forward's fill left out, the layer's forward and backward
+// went from 1045 to 730 us.  With adds the same shortcut needs atomics and took
+// longer than the workspace.  mode: 0 param_flows takes atomic adds, 1 plain adds (disjoint
+// parameters), 2 plain stores (disjoint parameters, SET).
+template <int ET, int NKP, bool VEC, bool LOGP, bool NTP, bool SET>
 __global__ __launch_bounds__(64, 2) void blocked_bwd_fused(float* __restrict__ edge_flows,
+                                                        float* __restrict__ element_flows,
+                                                        const int64_t* __restrict__ csc_offsets,
                                                         float* __restrict__ param_flows,
                                                         const float* __restrict__ gf, const float* __restrict__ om,
                                                         const float* __restrict__ xm, const float* __restrict__ params,
@@ -588,7 +600,7 @@ __global__ __launch_bounds__(64, 2) void blocked_bwd_fused(float* __restrict__ e
                                                         const int64_t* __restrict__ cids,
                                                         const int64_t* __restrict__ pids, int64_t ne, int64_t bs,
                                                         int64_t batch, int64_t chunks, int64_t items, int64_t id0,
-                                                        int disjoint) {
+                                                        int mode) {
     constexpr int MP = (NKP + 3) / 4;
     constexpr int LD = kTileLD;  // tile row; columns placed by tile_col
     constexpr int KC = NKP < 4 ? NKP : 4;
@@ -615,6 +627,22 @@ __global__ __launch_bounds__(64, 2) void blocked_bwd_fused(float* __restrict__ e
     // transposed reads (rows 16 pt + jc)
     const int colw = tile_col(4 * kq, 4 * jc);
     const int swt = tile_swz(jc);
+    // SET: the row each of the chunk's edges writes
+    __shared__ float* rows[SET ? 16 * ET : 1];
+    if constexpr (SET) {
+        if (l < 16 * ET && c0 + l < ne) {
+            const int64_t el = cids[ebase + c0 + l];
+            const bool sole = csc_offsets[el + 1] - csc_offsets[el] == 1;
+            rows[l] = sole ? element_flows + el * batch : edge_flows + (ebase + c0 + l) * batch;
+        }
+        __builtin_amdgcn_wave_barrier();  // one wave: its LDS operations complete in order
+    }
+    const auto flow_row = [&](int64_t e) {
+        if constexpr (SET)
+            return rows[e - c0];
+        else
+            return edge_flows + (ebase + e) * batch;
+    };
 
     // weights of the edge-flow product, A[p = 4*ks + kq][e = c0 + 16*et + jc], and
     // the row maxima (log) over the chunk's edges
@@ -766,7 +794,7 @@ __global__ __launch_bounds__(64, 2) void blocked_bwd_fused(float* __restrict__ e
                     res[u] = zz == 0.0f ? 0.0f : xe[u] * zz;
                 }
                 if (e >= ne) continue;
-                float* orow = edge_flows + (ebase + e) * batch;
+                float* orow = flow_row(e);
                 if constexpr (VEC) {
                     if (col < batch) store_stream(f32x4{res[0], res[1], res[2], res[3]}, orow + col);
                 } else {
@@ -864,7 +892,7 @@ __global__ __launch_bounds__(64, 2) void blocked_bwd_fused(float* __restrict__ e
                 for (int r = 0; r < 4; ++r) {
                     const int64_t e = c0 + 16 * et + 4 * kq + r;
                     if (e >= ne) continue;
-                    float* orow = edge_flows + (ebase + e) * batch;
+                    float* orow = flow_row(e);
 #pragma unroll
                     for (int u = 0; u < 4; ++u) {
                         const float t = xt[16 * et + 4 * kq + r][colw + u];
@@ -918,7 +946,16 @@ __global__ __launch_bounds__(64, 2) void blocked_bwd_fused(float* __restrict__ e
                 pfv[pt][r][et] = v;
             }
         }
-    if (disjoint) {
+    if (mode == 2) {
+#pragma unroll
+        for (int pt = 0; pt < MP; ++pt)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int et = 0; et < ET; ++et)
+                    if (16 * pt + 4 * kq + r < bs && c0 + 16 * et + jc < ne)
+                        param_flows[q[et] + 16 * pt + 4 * kq + r] = pfv[pt][r][et];
+    } else if (mode == 1) {
         // No parameter is shared by two (block, parent, edge) triples of the
         // layer, so this lane's cells are its own: a plain load, add and store,
         // every load issued before the first store.  The wave covers each block
@@ -957,18 +994,21 @@ __global__ __launch_bounds__(64, 2) void blocked_bwd_fused(float* __restrict__ e
 // per pass (two 16-byte vectors per lane, both issued before either is
 // used); the edge rows and the element row are read once, with the
 // nontemporal hint (221 -> 210 us at the bench layer), and the sums stored
-// with it.
-template <bool VEC>
+// with it.  SET: the rows are written, not added to: zeros where no edge
+// arrives, and rows whose only edge wrote them itself (sole_done) are done.
+// At the bench layer that leaves 0.68 GB of traffic of the 1.22, and spares the
+// caller's clearing of the rows (another 0.54).
+template <bool VEC, bool SET>
 __global__ __launch_bounds__(256) void blocked_bwd_elements(float* __restrict__ element_flows,
                                                             const float* __restrict__ edge_flows,
                                                             const int64_t* __restrict__ csc_offsets,
                                                             const int32_t* __restrict__ csc_edges, int64_t nel,
-                                                            int64_t batch, int64_t block0) {
+                                                            int64_t batch, int64_t block0, int sole_done) {
     const int64_t c = (block0 + (int64_t)blockIdx.x) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (c >= nel) return;
     const int64_t k0 = csc_offsets[c];
     const int64_t k1 = csc_offsets[c + 1];
-    if (k0 >= k1) return;
+    if (SET ? sole_done && k1 - k0 == 1 : k0 >= k1) return;
     const int l = lane_id();
     float* er = element_flows + c * batch;
     for (int64_t b0 = 0; b0 < batch; b0 += 512) {
@@ -986,12 +1026,14 @@ __global__ __launch_bounds__(256) void blocked_bwd_elements(float* __restrict__ 
                 for (int u = 0; u < 4; ++u) s[h][u] += v[h][u];
             }
         }
-        float cur[2][4];
+        float cur[2][4] = {};
+        if constexpr (!SET) {
 #pragma unroll
-        for (int h = 0; h < 2; ++h) ld4_raw_nt<VEC, true>(er, col[h], batch, cur[h]);
+            for (int h = 0; h < 2; ++h) ld4_raw_nt<VEC, true>(er, col[h], batch, cur[h]);
+        }
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            ld4_fill<VEC>(col[h], batch, 0.0f, cur[h]);
+            if constexpr (!SET) ld4_fill<VEC>(col[h], batch, 0.0f, cur[h]);
             if constexpr (VEC) {
                 if (col[h] < batch)
                     store_stream(f32x4{cur[h][0] + s[h][0], cur[h][1] + s[h][1], cur[h][2] + s[h][2],
@@ -1073,58 +1115,69 @@ void launch_et(float* edge_flows, float* param_flows, const float* gf, const flo
         launch_params<2, ET, VEC, LOGP>(param_flows, gf, om, xm, params, nids, cids, pids, nb, ne, bs, batch, st);
 }
 
+// Where the edges' flows go: the workspace rows; with `set` (SET) the element
+// rows too.
+struct EdgeOut {
+    float* edge_flows;
+    float* element_flows;
+    const int64_t* csc_offsets;
+    bool set;
+};
+
 template <int ET, int NKP, bool VEC, bool LOGP>
-void launch_fused(float* edge_flows, float* param_flows, const float* gf, const float* om, const float* xm,
+void launch_fused(const EdgeOut& eo, float* param_flows, const float* gf, const float* om, const float* xm,
                   const float* params, const int64_t* nids, const int64_t* cids, const int64_t* pids, int64_t nb,
-                  int64_t ne, int64_t bs, int64_t batch, int disjoint, hipStream_t st) {
+                  int64_t ne, int64_t bs, int64_t batch, int mode, hipStream_t st) {
     const int64_t chunks = (ne + CE - 1) / CE;
     const int64_t items = nb * chunks;
     for (int64_t id0 = 0; id0 < items; id0 += kMaxGroups) {
         const int64_t n = items - id0 < kMaxGroups ? items - id0 : kMaxGroups;
         const dim3 grid((unsigned)((n + 7) / 8 * 8));
+        const auto go = [&](auto kernel) {
+            kernel<<<grid, dim3(64), 0, st>>>(eo.edge_flows, eo.element_flows, eo.csc_offsets, param_flows, gf, om, xm,
+                                              params, nids, cids, pids, ne, bs, batch, chunks, items, id0, mode);
+        };
         if (chunks == 1)
-            blocked_bwd_fused<ET, NKP, VEC, LOGP, true><<<grid, dim3(64), 0, st>>>(
-                edge_flows, param_flows, gf, om, xm, params, nids, cids, pids, ne, bs, batch, chunks, items, id0,
-                disjoint);
+            eo.set ? go(blocked_bwd_fused<ET, NKP, VEC, LOGP, true, true>)
+                   : go(blocked_bwd_fused<ET, NKP, VEC, LOGP, true, false>);
         else
-            blocked_bwd_fused<ET, NKP, VEC, LOGP, false><<<grid, dim3(64), 0, st>>>(
-                edge_flows, param_flows, gf, om, xm, params, nids, cids, pids, ne, bs, batch, chunks, items, id0,
-                disjoint);
+            eo.set ? go(blocked_bwd_fused<ET, NKP, VEC, LOGP, false, true>)
+                   : go(blocked_bwd_fused<ET, NKP, VEC, LOGP, false, false>);
     }
 }
 
 template <int ET, bool VEC, bool LOGP>
-void launch_fused_et(float* edge_flows, float* param_flows, const float* gf, const float* om, const float* xm,
+void launch_fused_et(const EdgeOut& eo, float* param_flows, const float* gf, const float* om, const float* xm,
                      const float* params, const int64_t* nids, const int64_t* cids, const int64_t* pids, int64_t nb,
-                     int64_t ne, int64_t bs, int64_t batch, int disjoint, hipStream_t st) {
+                     int64_t ne, int64_t bs, int64_t batch, int mode, hipStream_t st) {
     if (bs <= 4)
-        launch_fused<ET, 1, VEC, LOGP>(edge_flows, param_flows, gf, om, xm, params, nids, cids, pids, nb, ne, bs, batch, disjoint, st);
+        launch_fused<ET, 1, VEC, LOGP>(eo, param_flows, gf, om, xm, params, nids, cids, pids, nb, ne, bs, batch, mode, st);
     else if (bs <= 8)
-        launch_fused<ET, 2, VEC, LOGP>(edge_flows, param_flows, gf, om, xm, params, nids, cids, pids, nb, ne, bs, batch,
-                                       disjoint, st);
+        launch_fused<ET, 2, VEC, LOGP>(eo, param_flows, gf, om, xm, params, nids, cids, pids, nb, ne, bs, batch,
+                                       mode, st);
     else if (bs <= 16)
-        launch_fused<ET, 4, VEC, LOGP>(edge_flows, param_flows, gf, om, xm, params, nids, cids, pids, nb, ne, bs, batch,
-                                       disjoint, st);
+        launch_fused<ET, 4, VEC, LOGP>(eo, param_flows, gf, om, xm, params, nids, cids, pids, nb, ne, bs, batch,
+                                       mode, st);
     else
-        launch_fused<ET, 8, VEC, LOGP>(edge_flows, param_flows, gf, om, xm, params, nids, cids, pids, nb, ne, bs, batch,
-                                       disjoint, st);
+        launch_fused<ET, 8, VEC, LOGP>(eo, param_flows, gf, om, xm, params, nids, cids, pids, nb, ne, bs, batch,
+                                       mode, st);
 }
 
 template <bool VEC, bool LOGP>
-void launch_all(float* edge_flows, float* param_flows, const float* gf, const float* om, const float* xm,
+void launch_all(const EdgeOut& eo, float* param_flows, const float* gf, const float* om, const float* xm,
                 const float* params, const int64_t* nids, const int64_t* cids, const int64_t* pids, int64_t nb,
-                int64_t ne, int64_t bs, int64_t batch, int disjoint, hipStream_t st) {
+                int64_t ne, int64_t bs, int64_t batch, int mode, hipStream_t st) {
     if (bs <= kFusedMaxBs) {
         if (ne <= 16)
-            launch_fused_et<1, VEC, LOGP>(edge_flows, param_flows, gf, om, xm, params, nids, cids, pids, nb, ne, bs,
-                                          batch, disjoint, st);
+            launch_fused_et<1, VEC, LOGP>(eo, param_flows, gf, om, xm, params, nids, cids, pids, nb, ne, bs,
+                                          batch, mode, st);
         else
-            launch_fused_et<2, VEC, LOGP>(edge_flows, param_flows, gf, om, xm, params, nids, cids, pids, nb, ne, bs,
-                                          batch, disjoint, st);
+            launch_fused_et<2, VEC, LOGP>(eo, param_flows, gf, om, xm, params, nids, cids, pids, nb, ne, bs,
+                                          batch, mode, st);
     } else if (ne <= 16) {
-        launch_et<1, VEC, LOGP>(edge_flows, param_flows, gf, om, xm, params, nids, cids, pids, nb, ne, bs, batch, st);
+        launch_et<1, VEC, LOGP>(eo.edge_flows, param_flows, gf, om, xm, params, nids, cids, pids, nb, ne, bs, batch, st);
     } else {
-        launch_et<2, VEC, LOGP>(edge_flows, param_flows, gf, om, xm, params, nids, cids, pids, nb, ne, bs, batch, st);
+        launch_et<2, VEC, LOGP>(eo.edge_flows, param_flows, gf, om, xm, params, nids, cids, pids, nb, ne, bs, batch, st);
     }
 }
 
@@ -1134,6 +1187,45 @@ void launch_all(float* edge_flows, float* param_flows, const float* gf, const fl
 }  // namespace fl
 
 using namespace fl;
+
+// mode: see blocked_bwd_fused.
+static int blocked_bwd_entry(const char* name, const float* node_flows, const float* node_mars,
+                             const float* element_mars, const float* params, const int64_t* nids, const int64_t* cids,
+                             const int64_t* pids, int64_t nb, int64_t ne, int64_t bs, int64_t batch,
+                             int params_are_log, int mode, const int64_t* csc_offsets, const int32_t* csc_edges,
+                             int64_t num_elements, float* edge_flows, float* element_flows, float* param_flows,
+                             bool set, hipStream_t st) {
+    FL_CHECK(node_flows && node_mars && element_mars && params && nids && cids && pids && csc_offsets && csc_edges &&
+                 edge_flows && element_flows && param_flows,
+             "%s: NULL pointer argument", name);
+    FL_CHECK(nb * ne < ((int64_t)1 << 31), "%s: block edges must be < 2^31", name);
+    const bool vec = (batch % 4 == 0) &&
+                     ((reinterpret_cast<uintptr_t>(node_flows) | reinterpret_cast<uintptr_t>(node_mars) |
+                       reinterpret_cast<uintptr_t>(element_mars) | reinterpret_cast<uintptr_t>(edge_flows) |
+                       reinterpret_cast<uintptr_t>(element_flows)) & 15) == 0;
+    const sparse::EdgeOut eo{edge_flows, element_flows, csc_offsets, set};
+    const auto products = [&](auto launch) {
+        launch(eo, param_flows, node_flows, node_mars, element_mars, params, nids, cids, pids, nb, ne, bs, batch, mode,
+               st);
+    };
+    if (vec)
+        params_are_log ? products(sparse::launch_all<true, true>) : products(sparse::launch_all<true, false>);
+    else
+        params_are_log ? products(sparse::launch_all<false, true>) : products(sparse::launch_all<false, false>);
+    // the single pass leaves rows with one edge done; the two kernels do not
+    const int sole_done = bs <= sparse::kFusedMaxBs;
+    for_grid_chunks((num_elements + 3) / 4, 256, [&](int64_t b0, int64_t n) {
+        const auto go = [&](auto kernel) {
+            kernel<<<dim3((unsigned)n), dim3(256), 0, st>>>(element_flows, edge_flows, csc_offsets, csc_edges,
+                                                            num_elements, batch, b0, sole_done);
+        };
+        if (vec)
+            set ? go(sparse::blocked_bwd_elements<true, true>) : go(sparse::blocked_bwd_elements<true, false>);
+        else
+            set ? go(sparse::blocked_bwd_elements<false, true>) : go(sparse::blocked_bwd_elements<false, false>);
+    });
+    return launch_status(name);
+}
 
 extern "C" int fl_sparse_blocked_bwd(const float* node_flows, const float* node_mars, const float* element_mars,
                                      const float* params, const int64_t* nids, const int64_t* cids,
@@ -1145,40 +1237,26 @@ extern "C" int fl_sparse_blocked_bwd(const float* node_flows, const float* node_
     FL_CHECK(num_nblocks >= 0 && num_edges >= 0 && block_size >= 0 && batch >= 0 && num_elements >= 0,
              "%s: negative size", name);
     if (num_nblocks == 0 || num_edges == 0 || block_size == 0 || batch == 0) return ok();
-    FL_CHECK(node_flows && node_mars && element_mars && params && nids && cids && pids && csc_offsets && csc_edges &&
-                 edge_flows && element_flows && param_flows,
-             "%s: NULL pointer argument", name);
-    FL_CHECK(num_nblocks * num_edges < ((int64_t)1 << 31), "%s: block edges must be < 2^31", name);
-    const bool vec = (batch % 4 == 0) &&
-                     ((reinterpret_cast<uintptr_t>(node_flows) | reinterpret_cast<uintptr_t>(node_mars) |
-                       reinterpret_cast<uintptr_t>(element_mars) | reinterpret_cast<uintptr_t>(edge_flows) |
-                       reinterpret_cast<uintptr_t>(element_flows)) & 15) == 0;
-    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    const int64_t nb = num_nblocks, ne = num_edges, bs = block_size;
-    if (vec) {
-        if (params_are_log)
-            sparse::launch_all<true, true>(edge_flows, param_flows, node_flows, node_mars, element_mars, params, nids,
-                                           cids, pids, nb, ne, bs, batch, params_disjoint ? 1 : 0, st);
-        else
-            sparse::launch_all<true, false>(edge_flows, param_flows, node_flows, node_mars, element_mars, params,
-                                            nids, cids, pids, nb, ne, bs, batch, params_disjoint ? 1 : 0, st);
-    } else {
-        if (params_are_log)
-            sparse::launch_all<false, true>(edge_flows, param_flows, node_flows, node_mars, element_mars, params,
-                                            nids, cids, pids, nb, ne, bs, batch, params_disjoint ? 1 : 0, st);
-        else
-            sparse::launch_all<false, false>(edge_flows, param_flows, node_flows, node_mars, element_mars, params,
-                                             nids, cids, pids, nb, ne, bs, batch, params_disjoint ? 1 : 0, st);
-    }
-    if (num_elements > 0) {
-        for_grid_chunks((num_elements + 3) / 4, 256, [&](int64_t b0, int64_t nb) {
-            if (vec)
-                sparse::blocked_bwd_elements<true><<<dim3((unsigned)nb), dim3(256), 0, st>>>(
-                    element_flows, edge_flows, csc_offsets, csc_edges, num_elements, batch, b0);
-            else
-                sparse::blocked_bwd_elements<false><<<dim3((unsigned)nb), dim3(256), 0, st>>>(
-                    element_flows, edge_flows, csc_offsets, csc_edges, num_elements, batch, b0);
-        });
-    }
-    return launch_status(name);
+    return blocked_bwd_entry(name, node_flows, node_mars, element_mars, params, nids, cids, pids, num_nblocks,
+                             num_edges, block_size, batch, params_are_log, params_disjoint ? 1 : 0, csc_offsets,
+                             csc_edges, num_elements, edge_flows, element_flows, param_flows, false,
+                             reinterpret_cast<hipStream_t>(stream));
+}
+
+extern "C" int fl_sparse_blocked_grad(const float* node_flows, const float* node_mars, const float* element_mars,
+                                      const float* params, const int64_t* nids, const int64_t* cids,
+                                      const int64_t* pids, int64_t num_nblocks, int64_t num_edges, int64_t block_size,
+                                      int64_t batch, int params_are_log, int params_disjoint, int write_params,
+                                      const int64_t* csc_offsets, const int32_t* csc_edges, int64_t num_elements,
+                                      float* edge_flows, float* element_flows, float* param_flows, void* stream) {
+    const char* name = "fl_sparse_blocked_grad";
+    FL_CHECK(num_nblocks > 0 && num_edges > 0 && block_size > 0 && batch > 0 && num_elements > 0,
+             "%s: an empty layer", name);
+    FL_CHECK(!write_params || (params_disjoint && block_size <= sparse::kFusedMaxBs),
+             "%s: parameters are written only where disjoint, in blocks of at most %d", name,
+             (int)sparse::kFusedMaxBs);
+    return blocked_bwd_entry(name, node_flows, node_mars, element_mars, params, nids, cids, pids, num_nblocks,
+                             num_edges, block_size, batch, params_are_log, write_params ? 2 : params_disjoint ? 1 : 0,
+                             csc_offsets, csc_edges, num_elements, edge_flows, element_flows, param_flows, true,
+                             reinterpret_cast<hipStream_t>(stream));
 }

@@ -496,6 +496,8 @@ class BlockedPlan(NamedTuple):
     # no two (block, parent, edge) triples share a parameter: the ranges
     # [pids[j, e], pids[j, e] + block_size) do not overlap
     params_disjoint: bool = False
+    # the blocks write the node rows [0, written_rows) in full (0: not known)
+    written_rows: int = 0
 
 
 def sparse_blocked_transpose(nids, cids, pids, block_size, num_elements):
@@ -539,7 +541,10 @@ def _blocked_plan(nids, cids, pids, block_size, num_elements):
     # writer and takes a plain add instead of an atomic one)
     starts = torch.sort(pids.reshape(-1)).values
     disjoint = bool(starts.numel() < 2 or int((starts[1:] - starts[:-1]).min()) >= bs)
-    return BlockedPlan(csc_off, order.to(torch.int32), nodes, qids, disjoint)
+    # blocks side by side from row 0 on, in any order
+    first_rows = torch.sort(nids).values
+    packed = nb > 0 and bool((first_rows == torch.arange(nb, device=dev, dtype=torch.int64) * bs).all())
+    return BlockedPlan(csc_off, order.to(torch.int32), nodes, qids, disjoint, nb * bs if packed else 0)
 
 
 def sparse_blocked_backward(node_flows, element_flows, node_mars, element_mars, params, param_flows, nids, cids, pids,
@@ -566,41 +571,17 @@ def sparse_blocked_backward(node_flows, element_flows, node_mars, element_mars, 
     _check(tuple(node_flows.shape) == tuple(node_mars.shape), "node_flows must have node_mars's shape")
     _check(tuple(element_flows.shape) == tuple(element_mars.shape), "element_flows must have element_mars's shape")
     _check(param_flows.numel() == params.numel(), "param_flows must have params's size")
-    # the forward's layout checks
-    _check(node_mars.is_cuda and element_mars.is_cuda and params.is_cuda, "node_mars, element_mars, params must be CUDA")
-    _check(node_mars.dtype == torch.float32 and element_mars.dtype == torch.float32 and params.dtype == torch.float32,
-           "node_mars, element_mars and params must be float32")
-    _check(node_mars.dim() == 2 and element_mars.dim() == 2 and node_mars.size(1) == element_mars.size(1),
-           "node_mars and element_mars must be 2-D [nodes, batch] with the same batch")
-    _check(node_mars.is_contiguous() and element_mars.is_contiguous() and params.is_contiguous(),
-           "node_mars, element_mars and params must be contiguous")
-    for name, t in (("nids", nids), ("cids", cids), ("pids", pids)):
-        _check(t.is_cuda and t.dtype == torch.int64 and t.is_contiguous(), f"{name} must be a contiguous CUDA int64 tensor")
-    _check(cids.dim() == 2 and pids.shape == cids.shape and nids.dim() == 1 and nids.size(0) == cids.size(0),
-           "nids [nblocks], cids and pids [nblocks, num_edges] shapes disagree")
-    _check_device(node_mars, "node_mars", node_flows=node_flows, element_flows=element_flows,
-                  element_mars=element_mars, params=params, param_flows=param_flows, nids=nids, cids=cids, pids=pids)
+    _check_blocked_layer(node_mars, element_mars, params, nids, cids, pids, node_flows=node_flows,
+                         element_flows=element_flows, param_flows=param_flows)
     nb, ne = cids.shape
     bs = int(block_size)
     num_el, batch = element_mars.shape
     if nb * ne * bs == 0 or batch == 0:
         return None
-    _check(nb * bs * ne < 2 ** 31 and num_el < 2 ** 31 and node_mars.size(0) < 2 ** 31,
-           "edges, element rows and node rows must each be < 2^31")
-    if plan is None:
-        plan = sparse_blocked_transpose(nids, cids, pids, bs, num_el)
-    csc_off, csc_edge, csc_node, q, disjoint = plan
-    _check_device(node_mars, "node_mars", csc_offsets=csc_off, csc_edges=csc_edge, csc_nodes=csc_node, param_ids=q)
-    _check(csc_off.dtype == torch.int64 and csc_off.numel() == num_el + 1 and csc_edge.dtype == torch.int32
-           and csc_edge.numel() == nb * ne and (bs != 1 or (csc_node is not None and q is not None
-                                                             and csc_node.numel() == nb * ne and q.numel() == nb * ne)),
-           "plan does not fit this layer")
+    csc_off, csc_edge, csc_node, q, disjoint = _fit_plan(plan, node_mars, element_mars, nids, cids, pids, bs)
     if bs == 1:
-        w = params.reshape(-1)[q]
-        logp = (w if params_are_log else torch.log(torch.clamp_min(w, 1e-45))).contiguous()
-        grad_el = torch.empty_like(element_mars)
-        grad_lp = torch.empty_like(logp)
-        _launch_csr_bwd(element_mars, node_mars, node_flows, logp, csc_off, csc_edge, csc_node, grad_el, grad_lp)
+        grad_el, grad_lp = _blocked_as_csr(node_flows, node_mars, element_mars, params, q, params_are_log, csc_off,
+                                           csc_edge, csc_node)
         element_flows.add_(grad_el)
         param_flows.view(-1).index_add_(0, q, grad_lp)
         return None
@@ -612,6 +593,83 @@ def sparse_blocked_backward(node_flows, element_flows, node_mars, element_mars, 
                   edge_flows.data_ptr(),
                   element_flows.data_ptr(), param_flows.data_ptr(), _stream(element_mars))
     return None
+
+
+def _check_blocked_layer(node_mars, element_mars, params, nids, cids, pids, **flows):
+    """The forward's layout checks, and that every operand is on node_mars's GPU."""
+    _check(node_mars.is_cuda and element_mars.is_cuda and params.is_cuda, "node_mars, element_mars, params must be CUDA")
+    _check(node_mars.dtype == torch.float32 and element_mars.dtype == torch.float32 and params.dtype == torch.float32,
+           "node_mars, element_mars and params must be float32")
+    _check(node_mars.dim() == 2 and element_mars.dim() == 2 and node_mars.size(1) == element_mars.size(1),
+           "node_mars and element_mars must be 2-D [nodes, batch] with the same batch")
+    _check(node_mars.is_contiguous() and element_mars.is_contiguous() and params.is_contiguous(),
+           "node_mars, element_mars and params must be contiguous")
+    for name, t in (("nids", nids), ("cids", cids), ("pids", pids)):
+        _check(t.is_cuda and t.dtype == torch.int64 and t.is_contiguous(), f"{name} must be a contiguous CUDA int64 tensor")
+    _check(cids.dim() == 2 and pids.shape == cids.shape and nids.dim() == 1 and nids.size(0) == cids.size(0),
+           "nids [nblocks], cids and pids [nblocks, num_edges] shapes disagree")
+    _check_device(node_mars, "node_mars", element_mars=element_mars, params=params, nids=nids, cids=cids, pids=pids,
+                  **flows)
+
+
+def _fit_plan(plan, node_mars, element_mars, nids, cids, pids, bs):
+    """The transposed structure of `plan` (built here when None), checked
+    against a non-empty layer."""
+    nb, ne = cids.shape
+    num_el = element_mars.size(0)
+    _check(nb * bs * ne < 2 ** 31 and num_el < 2 ** 31 and node_mars.size(0) < 2 ** 31,
+           "edges, element rows and node rows must each be < 2^31")
+    if plan is None:
+        plan = sparse_blocked_transpose(nids, cids, pids, bs, num_el)
+    csc_off, csc_edge, csc_node, q, disjoint = plan[:5]
+    _check_device(node_mars, "node_mars", csc_offsets=csc_off, csc_edges=csc_edge, csc_nodes=csc_node, param_ids=q)
+    _check(csc_off.dtype == torch.int64 and csc_off.numel() == num_el + 1 and csc_edge.dtype == torch.int32
+           and csc_edge.numel() == nb * ne and (bs != 1 or (csc_node is not None and q is not None
+                                                             and csc_node.numel() == nb * ne and q.numel() == nb * ne)),
+           "plan does not fit this layer")
+    return csc_off, csc_edge, csc_node, q, disjoint
+
+
+def _blocked_as_csr(node_flows, node_mars, element_mars, params, q, params_are_log, csc_off, csc_edge, csc_node):
+    """Block size 1: the CSR flows kernel's (element flows, log-weight flows)."""
+    w = params.reshape(-1)[q]
+    logp = (w if params_are_log else torch.log(torch.clamp_min(w, 1e-45))).contiguous()
+    grad_el = torch.empty_like(element_mars)
+    grad_lp = torch.empty_like(logp)
+    _launch_csr_bwd(element_mars, node_mars, node_flows, logp, csc_off, csc_edge, csc_node, grad_el, grad_lp)
+    return grad_el, grad_lp
+
+
+def _sparse_blocked_grads(grad_out, node_mars, element_mars, logparams, nids, cids, pids, block_size, plan):
+    """The gradients of pc.sparse_blocked_layer: (element_mars's, logparams's),
+    as sparse_blocked_backward adds them to zeros, without the zeros."""
+    _check(grad_out.is_cuda and grad_out.dtype == torch.float32 and grad_out.is_contiguous()
+           and tuple(grad_out.shape) == tuple(node_mars.shape),
+           "grad_out must be contiguous CUDA float32 of node_mars's shape")
+    _check_blocked_layer(node_mars, element_mars, logparams, nids, cids, pids, grad_out=grad_out)
+    nb, ne = cids.shape
+    bs = int(block_size)
+    num_el, batch = element_mars.shape
+    if nb * ne * bs == 0 or batch == 0:
+        return torch.zeros_like(element_mars), torch.zeros_like(logparams)
+    csc_off, csc_edge, csc_node, q, disjoint = _fit_plan(plan, node_mars, element_mars, nids, cids, pids, bs)
+    if bs == 1:
+        grad_el, grad_lp = _blocked_as_csr(grad_out, node_mars, element_mars, logparams, q, True, csc_off, csc_edge,
+                                           csc_node)
+        grad_params = torch.zeros_like(logparams)
+        grad_params.view(-1).index_add_(0, q, grad_lp)
+        return grad_el, grad_params
+    # disjoint ranges of as many parameters as there are: each is written once
+    write_params = bool(disjoint) and bs <= 32 and nb * ne * bs == logparams.numel()
+    grad_el = torch.empty_like(element_mars)
+    grad_params = torch.empty_like(logparams) if write_params else torch.zeros_like(logparams)
+    edge_flows = torch.empty(nb * ne, batch, dtype=torch.float32, device=element_mars.device)
+    with _on_device(element_mars):
+        _lib.call("fl_sparse_blocked_grad", grad_out.data_ptr(), node_mars.data_ptr(), element_mars.data_ptr(),
+                  logparams.data_ptr(), nids.data_ptr(), cids.data_ptr(), pids.data_ptr(), nb, ne, bs, batch, 1,
+                  int(disjoint), int(write_params), csc_off.data_ptr(), csc_edge.data_ptr(), num_el,
+                  edge_flows.data_ptr(), grad_el.data_ptr(), grad_params.data_ptr(), _stream(element_mars))
+    return grad_el, grad_params
 
 
 def sparse_csr_forward(child, offsets, child_ids, logparams, q16=False, out=None):

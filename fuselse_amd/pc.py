@@ -70,8 +70,10 @@ class _SparseBlockedLayer(torch.autograd.Function):
     def forward(ctx, element_mars, logparams, nids, cids, pids, block_size, num_nodes, plan):
         from . import ext
 
-        node_mars = torch.full((num_nodes, element_mars.size(1)), float("-inf"), dtype=torch.float32,
-                               device=element_mars.device)
+        node_mars = torch.empty((num_nodes, element_mars.size(1)), dtype=torch.float32, device=element_mars.device)
+        # rows that no block writes are -inf; a plan knows the leading rows
+        # that blocks write in full
+        node_mars[getattr(plan, "written_rows", 0):].fill_(float("-inf"))
         ext.sparse_forward_float(node_mars, element_mars, logparams, nids, cids, pids, block_size, params_are_log=True)
         ctx.save_for_backward(element_mars, logparams, nids, cids, pids, node_mars)
         ctx.block_size = block_size
@@ -85,10 +87,8 @@ class _SparseBlockedLayer(torch.autograd.Function):
         element_mars, logparams, nids, cids, pids, node_mars = ctx.saved_tensors
         if ctx.plan is None:
             ctx.plan = ext.sparse_blocked_transpose(nids, cids, pids, ctx.block_size, element_mars.size(0))
-        ge = torch.zeros_like(element_mars)
-        gl = torch.zeros_like(logparams)
-        ext.sparse_blocked_backward(grad_out.contiguous(), ge, node_mars, element_mars, logparams, gl, nids, cids, pids,
-                                    ctx.block_size, params_are_log=True, plan=ctx.plan)
+        ge, gl = ext._sparse_blocked_grads(grad_out.contiguous(), node_mars, element_mars, logparams, nids, cids, pids,
+                                           ctx.block_size, ctx.plan)
         return ge, gl, None, None, None, None, None, None
 
 
@@ -97,8 +97,10 @@ def sparse_blocked_layer(element_mars, logparams, nids, cids, pids, block_size, 
     out[nids[j] + p, b] = LSE over e of (logparams[pids[j, e] + p] + element_mars[cids[j, e], b])
     for every block j and position p < block_size; rows of out [num_nodes, batch]
     that no block writes are -inf.  Differentiable in element_mars and
-    logparams: the backward is ext.sparse_blocked_backward with the upstream
-    gradient as node flows (a term through a row of -inf contributes 0).
-    plan: a cached ext.sparse_blocked_transpose(nids, cids, pids, block_size,
-    element_mars.size(0)) for this layer."""
+    logparams: the backward gives the flows of ext.sparse_blocked_backward with
+    the upstream gradient as node flows (a term through a row of -inf
+    contributes 0).  plan: a cached ext.sparse_blocked_transpose(nids, cids,
+    pids, block_size, element_mars.size(0)) for this layer (these very nids,
+    cids and pids): the backward walks it, and the forward does not clear the
+    rows that it says blocks write."""
     return _SparseBlockedLayer.apply(element_mars, logparams, nids, cids, pids, int(block_size), int(num_nodes), plan)

@@ -284,6 +284,20 @@ int fl_sparse_blocked_bwd(const float* node_flows, const float* node_mars, const
                           int64_t num_elements, float* edge_flows, float* element_flows, float* param_flows,
                           void* stream);
 
+/* ---------------------------------------------------------------------------
+ * The same, as gradients of the layer: element_flows is written in full (0
+ * where no edge arrives), not added to, and needs no clearing.  param_flows is
+ * added to as above, or, with write_params (block_size <= 32 and
+ * params_disjoint), written: every parameter of the layer's ranges, no other.
+ * No size may be 0.
+ * ------------------------------------------------------------------------- */
+int fl_sparse_blocked_grad(const float* node_flows, const float* node_mars, const float* element_mars,
+                           const float* params, const int64_t* nids, const int64_t* cids, const int64_t* pids,
+                           int64_t num_nblocks, int64_t num_edges, int64_t block_size, int64_t batch,
+                           int params_are_log, int params_disjoint, int write_params, const int64_t* csc_offsets,
+                           const int32_t* csc_edges, int64_t num_elements, float* edge_flows, float* element_flows,
+                           float* param_flows, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -813,3 +813,48 @@ def test_csr_runs_past_the_streams_edges(cuda, batch):
     gc, gl = ext.sparse_csr_backward(ch, out, gout, off, cid, lpd)
     want = torch.tensor([1.0, float(big), 0.0], device=cuda)
     assert torch.equal(gc, want[:, None].expand(3, batch)) and torch.equal(gl, torch.full_like(gl, float(batch)))
+
+
+@pytest.mark.parametrize("bs,ne,batch", [(1, 5, 33), (2, 3, 64), (16, 16, 130), (24, 33, 66), (32, 32, 128), (32, 40, 5),
+                                         (48, 20, 68)])
+@pytest.mark.parametrize("shared,packed", [(False, True), (True, True), (False, False)])
+def test_blocked_layer_gradients_without_clearing(cuda, bs, ne, batch, shared, packed):
+    """The layer with a plan leaves out its fills: node rows the blocks write,
+    element rows (some with no edge, one or several), parameters of a layer
+    whose ranges cover them all.  Every result bit equals the in-place forward
+    over -inf rows and the backward over cleared flows; memory the allocator
+    hands out is filled with NaN first.  A plan of five fields (written_rows not
+    among them) does the same."""
+    print(f"case blocked grads bs={bs} ne={ne} batch={batch} shared={shared} packed={packed}", flush=True)
+    from fuselse_amd import pc
+
+    ext = _ext()
+    rng = np.random.default_rng(bs * ne + batch)
+    nb, nelem = 9, 200
+    first = rng.permutation(nb) * bs + (0 if packed else 2)
+    num_nodes = nb * bs + (5 if packed else 7)
+    pids = (rng.permutation(nb * ne) * bs).reshape(nb, ne)
+    if shared:
+        pids[1] = pids[0]
+    nids, cids, pids = _to(cuda, first.astype(np.int64), rng.integers(0, nelem, (nb, ne)).astype(np.int64),
+                           pids.astype(np.int64))
+    lw = torch.from_numpy(np.log(rng.random(nb * ne * bs) + 1e-3).astype(np.float32)).to(cuda)
+    em = torch.from_numpy(np.log(rng.random((nelem, batch)) + 1e-12).astype(np.float32)).to(cuda)
+    g = torch.from_numpy(rng.standard_normal((num_nodes, batch)).astype(np.float32)).to(cuda)
+    plan = ext.sparse_blocked_transpose(nids, cids, pids, bs, nelem)
+    assert plan.written_rows == (nb * bs if packed else 0)
+    want = torch.full((num_nodes, batch), float("-inf"), device=cuda)
+    ext.sparse_forward_float(want, em, lw, nids, cids, pids, bs, params_are_log=True)
+    ge, gp = torch.zeros_like(em), torch.zeros_like(lw)
+    ext.sparse_blocked_backward(g, ge, want, em, lw, gp, nids, cids, pids, bs, params_are_log=True, plan=plan)
+    for p in (plan, tuple(plan[:5])):
+        junk = [torch.full_like(t, float("nan")) for t in (want, em, lw, em) for _ in range(3)]
+        del junk  # the allocator's next blocks of these sizes hold NaN
+        e, w = em.clone().requires_grad_(True), lw.clone().requires_grad_(True)
+        y = pc.sparse_blocked_layer(e, w, nids, cids, pids, bs, num_nodes, plan=p)
+        de, dw = torch.autograd.grad(y, (e, w), g)
+        assert torch.equal(y, want) and torch.equal(de, ge)
+        if shared or bs > 32:  # parameter sums by atomics, in any order
+            torch.testing.assert_close(dw, gp, rtol=1e-5, atol=1e-5)
+        else:
+            assert torch.equal(dw, gp)
