@@ -40,6 +40,10 @@ SIGNATURES = {
     "fl_selective_logsoftmax_slices_bwd_f32": (_int, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp]),
     "fl_lse_bwd_f16": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _vp]),
     "fl_lse_bwd_bf16": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _vp]),
+    "fl_lse_fwd_f16_typed": (_int, [_vp, _vp, _vp, _i64, _i64, _int, _int, _vp, ctypes.c_size_t, _vp]),
+    "fl_lse_fwd_bf16_typed": (_int, [_vp, _vp, _vp, _i64, _i64, _int, _int, _vp, ctypes.c_size_t, _vp]),
+    "fl_lse_bwd_f16_typed": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _vp]),
+    "fl_lse_bwd_bf16_typed": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _vp]),
     "fl_lse_fwd_workspace_bytes": (ctypes.c_size_t, [_i64, _i64, _int]),
     "fl_lse_fwd_f32_ws": (_int, [_vp, _vp, _i64, _i64, _int, _vp, ctypes.c_size_t, _vp]),
     "fl_lse_fwd_f16_ws": (_int, [_vp, _vp, _i64, _i64, _int, _vp, ctypes.c_size_t, _vp]),

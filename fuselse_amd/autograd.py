@@ -57,6 +57,10 @@ def make_fuselse_logsumexp(ext, robust: bool = True, half_inputs: bool = False, 
             ext.batched_logsumexp_bf16
         half_fwd_grad = {torch.float16: lambda x: f16k(x, robust), torch.bfloat16: lambda x: bf16k(x, robust)}
         half_bwd = ext.onepass_lse_half_backward
+    # the same with results and gradients in the input's dtype, where the ext
+    # has them: no conversion kernels
+    typed = getattr(ext, "logsumexp_half_typed", None) if half_inputs else None
+    typed_bwd = getattr(ext, "logsumexp_half_typed_backward", None)
 
     class _RowLSE(torch.autograd.Function):
         @staticmethod
@@ -83,15 +87,22 @@ def make_fuselse_logsumexp(ext, robust: bool = True, half_inputs: bool = False, 
         def forward(ctx, inp):
             n = inp.shape[-1]
             rows = inp.reshape(-1, n).contiguous()
-            lse = half_fwd_grad[inp.dtype](rows)
+            if typed is not None:
+                y, lse = typed(rows, robust, keep, with_lse=True)
+            else:
+                lse = half_fwd_grad[inp.dtype](rows)
+                y = lse.to(inp.dtype)
             ctx.save_for_backward(rows, lse)
             ctx.in_shape = tuple(inp.shape)
-            return lse.to(inp.dtype).reshape(inp.shape[:-1])
+            return y.reshape(inp.shape[:-1])
 
         @staticmethod
         def backward(ctx, grad_out):
             rows, lse = ctx.saved_tensors
-            g = half_bwd(grad_out.reshape(-1).to(torch.float32).contiguous(), rows, lse)
+            if typed is not None and grad_out.dtype == rows.dtype:
+                g = typed_bwd(grad_out.reshape(-1).contiguous(), rows, lse)
+            else:
+                g = half_bwd(grad_out.reshape(-1).to(torch.float32).contiguous(), rows, lse)
             return g.reshape(ctx.in_shape)
 
     def logsumexp(input, dim=-1, keepdim=False):
@@ -105,7 +116,12 @@ def make_fuselse_logsumexp(ext, robust: bool = True, half_inputs: bool = False, 
         else:
             n = input.shape[-1]
             rows = input if (input.dim() == 2 and input.is_contiguous()) else input.reshape(-1, n).contiguous()
-            out = half_fwd[input.dtype](rows).to(input.dtype) if half else fwd(rows)
+            if not half:
+                out = fwd(rows)
+            elif typed is not None:
+                out = typed(rows, robust)
+            else:
+                out = half_fwd[input.dtype](rows).to(input.dtype)
             out = out.reshape(input.shape[:-1])
         return out.unsqueeze(-1) if keepdim else out
 

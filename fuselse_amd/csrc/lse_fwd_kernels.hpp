@@ -244,6 +244,25 @@ struct LseOut {
     __device__ __forceinline__ void end(int64_t row, Row, float lse) const { out[row] = lse; }
 };
 
+// Half-type rows: the LSE rounded to the input's type, and in fp32 when lse is
+// not NULL.
+template <typename T>
+struct TypedOut {
+    using Map = PackedRows;
+    static constexpr PackedRows map{};
+    T* __restrict__ y;
+    float* __restrict__ lse;
+    struct Row {};
+    __device__ __forceinline__ Row begin(int64_t) const { return {}; }
+    __device__ __forceinline__ void end(int64_t row, Row, float l) const {
+        // rounded from the fp32 value: without the barrier the compiler forms
+        // v_fma_mixlo_f16, which rounds the last sum once, to fp16
+        asm("" : "+v"(l));
+        Elem<T>::put(y + row, l);
+        if (lse) lse[row] = l;
+    }
+};
+
 // Selective log-softmax: logp[row] = x[row, index[row]] - lse[row], and lse[row]
 // when lse is not NULL.  An index outside [0, N) gives NaN (torch.gather would
 // raise); the special values follow from the robust LSE (a +inf target in a

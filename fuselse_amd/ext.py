@@ -340,6 +340,49 @@ def onepass_lse_half_backward(grad_output: torch.Tensor, x: torch.Tensor, lse_ou
     return grad_input
 
 
+_TYPED = {torch.float16: "f16", torch.bfloat16: "bf16"}
+
+
+def logsumexp_half_typed(x: torch.Tensor, robust: bool = True, keep: bool = False, with_lse: bool = False):
+    """Row LSE of a contiguous fp16 or bf16 (B, N) CUDA tensor with fp32
+    accumulation, rounded to x's dtype (what batched_logsumexp_fp16 / _bf16
+    return in fp32); with_lse: that and the fp32 values.  keep as for the
+    _keep functions."""
+    _check(x.dim() == 2, "Expected 2-D tensor (B, N)")
+    _check(x.is_cuda and x.dtype in _TYPED, "Input must be CUDA fp16 or bf16")
+    _check(x.is_contiguous(), "Input must be contiguous")
+    B, N = x.shape
+    y = torch.empty((B,), dtype=x.dtype, device=x.device)
+    lse = torch.empty((B,), dtype=torch.float32, device=x.device) if with_lse else None
+    if B:
+        with _on_device(x):
+            nbytes = _workspace_bytes(B, N, 2)
+            ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device) if nbytes else None
+            _lib.call(f"fl_lse_fwd_{_TYPED[x.dtype]}_typed", x.data_ptr(), y.data_ptr(),
+                      lse.data_ptr() if with_lse else None, B, N, int(robust), int(keep),
+                      ws.data_ptr() if ws is not None else None, nbytes, _stream(x))
+    return (y, lse) if with_lse else y
+
+
+def logsumexp_half_typed_backward(grad_output: torch.Tensor, x: torch.Tensor, lse: torch.Tensor) -> torch.Tensor:
+    """onepass_lse_half_backward with grad_output (B,) in x's dtype."""
+    _check(grad_output.is_cuda and x.is_cuda and lse.is_cuda, "grad_output, x and lse must be CUDA")
+    _check(x.dtype in _TYPED and grad_output.dtype == x.dtype, "x and grad_output must be float16 or bfloat16")
+    _check(lse.dtype == torch.float32, "lse must be float32")
+    _check(x.dim() == 2 and grad_output.dim() == 1 and lse.dim() == 1, "x must be 2D (B, N), grad_output and lse 1D (B)")
+    _check(x.is_contiguous() and grad_output.is_contiguous() and lse.is_contiguous(), "inputs must be contiguous")
+    _check(grad_output.size(0) == x.size(0) and lse.size(0) == x.size(0),
+           "grad_output and lse batch dimensions must match x")
+    _check_device(x, "x", grad_output=grad_output, lse=lse)
+    B, N = x.shape
+    grad_input = torch.empty_like(x)
+    if B * N:
+        with _on_device(x):
+            _lib.call(f"fl_lse_bwd_{_TYPED[x.dtype]}_typed", grad_output.data_ptr(), x.data_ptr(), lse.data_ptr(),
+                      grad_input.data_ptr(), B, N, _stream(x))
+    return grad_input
+
+
 def batched_logsumexp_fp16(x: torch.Tensor, robust: bool = False) -> torch.Tensor:
     """fp16 (B, N) -> fp32 (B,) LSE with fp32 accumulation
     (fused_fp16_kernel.cu:112-132)."""

@@ -127,6 +127,23 @@ int fl_lse_bwd_bf16(const float* grad, const void* x, const float* lse, void* gr
                     void* stream);
 
 /* ---------------------------------------------------------------------------
+ * The half entries with results and upstream gradients in x's own type, as
+ * torch.logsumexp's dtype contract has them:
+ * fl_lse_fwd_*_typed: y[r] = the fp32 LSE rounded to nearest even to x's type;
+ *   lse (may be NULL) receives it in fp32, for the backward.  keep as for the
+ *   _keep entries, workspace as for the _ws entries below.
+ * fl_lse_bwd_*_typed: fl_lse_bwd_* with grad [B] of x's type.
+ * ------------------------------------------------------------------------- */
+int fl_lse_fwd_f16_typed(const void* x, void* y, float* lse, int64_t B, int64_t N, int robust, int keep,
+                         void* workspace, size_t workspace_bytes, void* stream);
+int fl_lse_fwd_bf16_typed(const void* x, void* y, float* lse, int64_t B, int64_t N, int robust, int keep,
+                          void* workspace, size_t workspace_bytes, void* stream);
+int fl_lse_bwd_f16_typed(const void* grad, const void* x, const float* lse, void* grad_x, int64_t B, int64_t N,
+                         void* stream);
+int fl_lse_bwd_bf16_typed(const void* grad, const void* x, const float* lse, void* grad_x, int64_t B, int64_t N,
+                          void* stream);
+
+/* ---------------------------------------------------------------------------
  * Forward with a caller workspace, for few long rows.  The reference launches
  * one block per row (fused_fp32_kernel.cu:168-170, fused_fp16_kernel.cu:
  * 127-129), which leaves most of the GPU idle when B is small against the

@@ -720,3 +720,38 @@ def test_fwd_keep_bit_identical(cuda, dtype, B, N):
         f, fk = ((ext.batched_logsumexp_fp16, ext.batched_logsumexp_fp16_keep) if dtype == torch.float16
                  else (ext.batched_logsumexp_bf16, ext.batched_logsumexp_bf16_keep))
         assert torch.equal(fk(xd, robust=True), f(xd, robust=True))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,N", [(1, 2), (7, 3), (300, 63), (129, 257), (1030, 1000), (40, 9001), (1100, 9001), (3, 70001),
+                                 (250, 70001)])
+def test_half_typed_entries_are_the_fp32_ones_rounded(cuda, dtype, B, N):
+    """Results and gradients in the input's type: every bit is the fp32
+    entry's, converted by torch (row groups, blocks per row, split rows, the
+    keeping loads; rows off the 16-byte grid; special values)."""
+    import fuselse_amd
+
+    print(f"case half typed {dtype} B={B} N={N}", flush=True)
+    ext = fuselse_amd.ext
+    gen = torch.Generator(device=cuda)
+    gen.manual_seed(B + N)
+    x = (torch.randn(B, N, device=cuda, generator=gen) * 3).to(dtype)
+    if B > 6:
+        x[0] = float("-inf")
+        x[1, 1] = float("inf")
+        x[2, 0] = float("nan")
+    fp32 = ext.batched_logsumexp_fp16 if dtype == torch.float16 else ext.batched_logsumexp_bf16
+    for robust in (True, False):
+        want = fp32(x, robust)
+        for keep in (False, True):
+            y, lse = ext.logsumexp_half_typed(x, robust, keep, with_lse=True)
+            assert y.dtype == dtype and lse.dtype == torch.float32
+            assert torch.equal(lse.nan_to_num(9.0), want.nan_to_num(9.0)) and torch.equal(lse.isnan(), want.isnan())
+            assert torch.equal(y.nan_to_num(9.0), want.to(dtype).nan_to_num(9.0)) and torch.equal(y.isnan(), want.isnan())
+        y = ext.logsumexp_half_typed(x, robust)
+        assert torch.equal(y.nan_to_num(9.0), want.to(dtype).nan_to_num(9.0))
+    g = torch.randn(B, device=cuda, generator=gen).to(dtype)
+    lse = fp32(x, True)
+    got = ext.logsumexp_half_typed_backward(g, x, lse)
+    want = ext.onepass_lse_half_backward(g.float(), x, lse)
+    assert torch.equal(got.nan_to_num(9.0), want.nan_to_num(9.0)) and torch.equal(got.isnan(), want.isnan())
