@@ -106,23 +106,25 @@ def make_fuselse_logsumexp(ext, robust: bool = True, half_inputs: bool = False, 
             return g.reshape(ctx.in_shape)
 
     def logsumexp(input, dim=-1, keepdim=False):
-        last = input.dim() - 1
-        d = dim if dim >= 0 else input.dim() + dim
-        half = input.dtype in half_fwd
-        if not (input.is_cuda and (input.dtype == torch.float32 or half) and d == last and input.shape[-1] >= 2):
+        # the host side of this call is most of a small launch's time
+        nd = input.dim()
+        d = dim if dim >= 0 else nd + dim
+        dtype = input.dtype
+        half = dtype in half_fwd
+        if not (input.is_cuda and (dtype == torch.float32 or half) and d == nd - 1 and input.shape[-1] >= 2):
             return torch_logsumexp(input, dim=dim, keepdim=keepdim)
         if torch.is_grad_enabled() and input.requires_grad:
             out = (_HalfRowLSE if half else _RowLSE).apply(input)
         else:
-            n = input.shape[-1]
-            rows = input if (input.dim() == 2 and input.is_contiguous()) else input.reshape(-1, n).contiguous()
+            rows = input if (nd == 2 and input.is_contiguous()) else input.reshape(-1, input.shape[-1]).contiguous()
             if not half:
                 out = fwd(rows)
             elif typed is not None:
                 out = typed(rows, robust)
             else:
-                out = half_fwd[input.dtype](rows).to(input.dtype)
-            out = out.reshape(input.shape[:-1])
+                out = half_fwd[dtype](rows).to(dtype)
+            if nd != 2:
+                out = out.reshape(input.shape[:-1])
         return out.unsqueeze(-1) if keepdim else out
 
     logsumexp.fuselse_robust = robust

@@ -60,10 +60,15 @@ class _Same:
 _SAME = _Same()
 
 
+# torch.cuda.current_device() without its lazy initialisation, which a CUDA
+# tensor's existence implies.
+_current_device = getattr(torch._C, "_cuda_getDevice", None) or torch.cuda.current_device
+
+
 def _on_device(t: torch.Tensor):
     """A guard that makes t's device current for the enclosed launch."""
     idx = t.device.index
-    if idx is None or idx == torch.cuda.current_device():
+    if idx is None or idx == _current_device():
         return _SAME
     return torch.cuda.device(idx)
 
@@ -91,8 +96,14 @@ def _launch_fwd(entry: str, x: torch.Tensor, out: torch.Tensor, elem_bytes: int,
     Infinity Cache for the backward), or the split-row kernels (entry +
     "_ws") for few long rows, where the library asks for a workspace."""
     B, N = x.shape
+    nbytes = _workspace_bytes(B, N, elem_bytes)
+    idx = x.device.index
+    if not nbytes and _raw_stream is not None and idx == _current_device():
+        # one launch on the current device: no guard to enter
+        _lib.call(entry + "_keep" if keep else entry, x.data_ptr(), out.data_ptr(), B, N, 1 if robust else 0,
+                  _raw_stream(idx))
+        return
     with _on_device(x):
-        nbytes = _workspace_bytes(B, N, elem_bytes)
         if nbytes:
             # partials between the two split kernels; stream-ordered reuse by
             # torch's caching allocator keeps it valid until they have run
@@ -106,12 +117,13 @@ def _launch_fwd(entry: str, x: torch.Tensor, out: torch.Tensor, elem_bytes: int,
 
 def _fwd_f32(x: torch.Tensor, robust: bool, keep: bool = False) -> torch.Tensor:
     # fused_fp32_kernel.cu:155-158 / :176-179
-    _check(x.is_cuda, "x must be CUDA")
-    _check(x.dtype == torch.float32, "x must be float32")
-    _check(x.dim() == 2, "x must be 2D (B, N)")
-    _check(x.is_contiguous(), "x must be contiguous")
-    B, N = x.shape
-    out = torch.empty((B,), dtype=torch.float32, device=x.device)
+    if not (x.is_cuda and x.dtype == torch.float32 and x.dim() == 2 and x.is_contiguous()):
+        _check(x.is_cuda, "x must be CUDA")
+        _check(x.dtype == torch.float32, "x must be float32")
+        _check(x.dim() == 2, "x must be 2D (B, N)")
+        _check(x.is_contiguous(), "x must be contiguous")
+    B = x.shape[0]
+    out = torch.empty(B, dtype=torch.float32, device=x.device)
     if B == 0:
         return out
     _launch_fwd("fl_lse_fwd_f32", x, out, 4, robust, keep)
