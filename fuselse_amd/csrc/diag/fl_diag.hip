@@ -129,7 +129,7 @@ __global__ __launch_bounds__(1024) void chain_latency_kernel(int steps, uint64_t
             } else if constexpr (KIND == 2) {
                 a = q10_pair(a, (int)(((uint32_t)k * 2654435761u) >> 22) - 512, tab8);
             } else if constexpr (KIND == 3) {
-                a = q16_pair<true>(a, (int)((uint32_t)k * 2654435761u) >> 6, lut);
+                a = (int)q16_pair<true>((uint32_t)a, ((uint32_t)k * 2654435761u) >> 6, lut);
             } else {
                 u32x4* slot = reinterpret_cast<u32x4*>(&tabw[slot_word<KIND>(a)]);
                 // the lane's own slot only: every wave writes the same words,

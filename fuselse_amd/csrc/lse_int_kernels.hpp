@@ -80,12 +80,14 @@ __device__ __forceinline__ int q16_quant(float v) {
 }
 
 // Element sources for the trees: fp32 quantised in the kernel, int32, int16.
+// kBias is what the tree's values are biased by (q16_pair's operands).
 // bload() fetches one 4-element chunk by raw buffer load, unpack() turns it
 // into Q values, one() reads a single (prefix or suffix) element.
 struct SrcF32 {
     using T = float;
     using Raw = f32x4;
-    __device__ static __forceinline__ int cvt(float v) { return q16_quant(v); }
+    static constexpr int kBias = (int)kQBias;
+    __device__ static __forceinline__ int cvt(float v) { return q16_quant(v) ^ kBias; }
     __device__ static __forceinline__ float sload(__amdgpu_buffer_rsrc_t r, int voff) {
         return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, voff, 0, 0));
     }
@@ -93,13 +95,14 @@ struct SrcF32 {
         return __builtin_bit_cast(Raw, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, kBufNT));
     }
     __device__ static __forceinline__ void unpack(Raw v, int (&q)[4]) {
-        q[0] = q16_quant(v.x); q[1] = q16_quant(v.y); q[2] = q16_quant(v.z); q[3] = q16_quant(v.w);
+        q[0] = cvt(v.x); q[1] = cvt(v.y); q[2] = cvt(v.z); q[3] = cvt(v.w);
     }
 };
 struct SrcI32 {
     using T = int32_t;
     using Raw = u32x4;
-    __device__ static __forceinline__ int cvt(int32_t v) { return v; }
+    static constexpr int kBias = (int)kQBias;
+    __device__ static __forceinline__ int cvt(int32_t v) { return v ^ kBias; }
     __device__ static __forceinline__ int32_t sload(__amdgpu_buffer_rsrc_t r, int voff) {
         return (int32_t)__builtin_amdgcn_raw_buffer_load_b32(r, voff, 0, 0);
     }
@@ -107,13 +110,14 @@ struct SrcI32 {
         return __builtin_bit_cast(Raw, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, kBufNT));
     }
     __device__ static __forceinline__ void unpack(Raw v, int (&q)[4]) {
-        q[0] = (int)v.x; q[1] = (int)v.y; q[2] = (int)v.z; q[3] = (int)v.w;
+        q[0] = cvt((int)v.x); q[1] = cvt((int)v.y); q[2] = cvt((int)v.z); q[3] = cvt((int)v.w);
     }
 };
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 struct SrcI16 {
     using T = int16_t;
     using Raw = u32x2;
+    static constexpr int kBias = 0;
     __device__ static __forceinline__ int cvt(int16_t v) { return (int)v; }
     __device__ static __forceinline__ int16_t sload(__amdgpu_buffer_rsrc_t r, int voff) {
         return (int16_t)__builtin_amdgcn_raw_buffer_load_b16(r, voff, 0, 0);
@@ -192,7 +196,8 @@ __device__ __forceinline__ int tree_row(const typename SRC::T* row, int64_t n, c
     const bool has_suf = t < tail;
     const T suf = SRC::sload(rrow, (int)((has_suf ? prefix + 4 * n4 + t : n) * (int64_t)sizeof(T)));
 
-    int acc = kQNegInf;
+    constexpr int kEmpty = kQNegInf ^ SRC::kBias;
+    int acc = kEmpty;
     bool has = has_pre;
     auto fold_first = [&](const typename SRC::Raw& raw) {
         int qq[4];
@@ -260,9 +265,9 @@ __device__ __forceinline__ int tree_row(const typename SRC::T* row, int64_t n, c
     acc = pair(acc, exact_xor<1>(acc), tab);
     if ((t & 31) == 0) sh_warp[t >> 5] = acc;
     __syncthreads();
-    int v = kQNegInf;
+    int v = kEmpty;
     if (t < 64) {
-        v = (t & 31) < 8 ? sh_warp[t & 31] : kQNegInf;
+        v = (t & 31) < 8 ? sh_warp[t & 31] : kEmpty;
         v = pair(v, exact_xor<16>(v), tab);
         v = pair(v, exact_xor<8>(v), tab);
         v = pair(v, exact_xor<4>(v), tab);
@@ -271,7 +276,7 @@ __device__ __forceinline__ int tree_row(const typename SRC::T* row, int64_t n, c
     }
     clk.tree_end();
     __syncthreads();  // sh_warp is reused by the next row
-    return v;
+    return v ^ SRC::kBias;
 }
 
 // A 64-entry table held across a wave's lanes: lane i gets tab[i], written
@@ -310,7 +315,7 @@ __global__ __launch_bounds__(256) void intlse_q16_rows(const typename SRC::T* __
     __shared__ int lut[64];
     __shared__ int sh_warp[8];
     Q16Setup<USE_LUT> setup{lut, 0};
-    auto pair = [](int a, int b, const int* t) { return q16_pair<USE_LUT>(a, b, t); };
+    auto pair = [](int a, int b, const int* t) { return (int)q16_pair<USE_LUT>((uint32_t)a, (uint32_t)b, t); };
     const int64_t row = blockIdx.x;
     const int v = tree_row<SRC, 16, D>(x + row * N, N, lut, pair, sh_warp, setup, clk);
     if (threadIdx.x == 0) {

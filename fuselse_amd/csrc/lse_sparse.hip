@@ -35,6 +35,7 @@
 #include "fl_status.hpp"
 #include "lse_blocked.hpp"
 #include "lse_common.hpp"
+#include "lse_pair.hpp"
 
 namespace fl {
 namespace sparse {
@@ -55,41 +56,17 @@ __constant__ int kLut[64] = {
      312,  235,  168,  113,   69,   35,   13,    2,
 };
 
-// Fixed-point values inside the folds are biased by 2^31, as unsigned: the
-// order is the same, and |a - b| is one instruction on unsigned operands.
-constexpr uint32_t kBias = 0x80000000u;
-constexpr uint32_t kNegInfU = (uint32_t)kNegInfQ ^ kBias;
+constexpr uint32_t kNegInfU = (uint32_t)kNegInfQ ^ kQBias;
 
-// The reference's pair op, max + M + LUT[(M >> 10) & 63] with
-// M = (2^16 + ((lo - hi) & 0xFFFF)) >> ceil((hi - lo) / 2^16), the shift
-// clamped to 31.  With t = |a - b| + 0xFFFF mod 2^32 (v_sad_u32) the shift is
-// t >> 16, and 2^16 plus the low half of lo - hi is 2^16 plus the complement of
-// t's low half, one bit select.  (Differences within 2^16 of 2^32, which only
-// accumulators wrapped past the int32 limit reach, wrap t to a shift of 0, as
-// the signed 32-bit difference does.)  Seven vector instructions and the table
-// read; max, min, their difference, its halves and a two-instruction table
-// offset took ten: the block layer of 2048 x 32 nodes, 32 edges, batch 512,
-// whose time this is, went from 472 to 424 us.
 __device__ __forceinline__ uint32_t pair(uint32_t a, uint32_t b, const int* __restrict__ lut) {
-    const uint32_t hi = a > b ? a : b;
-    uint32_t t, fr, off;
-    asm("v_sad_u32 %0, %1, %2, %3" : "=v"(t) : "v"(a), "v"(b), "s"(0xFFFFu));
-    const uint32_t th = t >> 16;
-    const uint32_t sh = th < 31u ? th : 31u;
-    asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(fr) : "v"(t), "v"(0x10000u), "s"(0x1FFFFu));
-    const uint32_t m = fr >> sh;
-    // table offset (m >> 8) & 0xFC: byte 1 of m, masked
-    asm("v_and_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_1 src1_sel:DWORD"
-        : "=v"(off)
-        : "v"(m), "s"(0xFCu));
-    return hi + m + (uint32_t)*reinterpret_cast<const int*>(reinterpret_cast<const char*>(lut) + off);
+    return q16_pair<true>(a, b, lut);
 }
 
 __device__ __forceinline__ uint32_t quant(float logit) {
     const float r = __builtin_rintf(fmaxf(logit, -20000.0f) * kConv);
     int q;
     asm("v_cvt_i32_f32 %0, %1" : "=v"(q) : "v"(r));
-    return (uint32_t)q ^ kBias;
+    return (uint32_t)q ^ kQBias;
 }
 
 // Vectors of VW floats and their buffer loads.
@@ -366,7 +343,7 @@ __device__ __forceinline__ void reduce_q16_et(const LAYOUT& L, const DESC& d, co
             for (int c = 0; c < 2; ++c) acc[c][i] = pair(acc[c][i], acc[c + 2][i], lut);
         }
         if constexpr (ET >= 2) acc[0][i] = pair(acc[0][i], acc[1][i], lut);
-        const int q = (int)(acc[0][i] ^ kBias);
+        const int q = (int)(acc[0][i] ^ kQBias);
         res[i] = q > kNegInfQ ? (float)q * kOutScale : -kInf;
     }
     Cols<VW, P>::store(L.out_row(d), b0, l, batch, res);
@@ -624,7 +601,7 @@ struct FoldQ16 {
         }
 #pragma unroll
         for (int i = 0; i < P; ++i) {
-            const int q = (int)(acc[0][i] ^ kBias);
+            const int q = (int)(acc[0][i] ^ kQBias);
             res[i] = q > kNegInfQ ? (float)q * kOutScale : -kInf;
         }
     }
