@@ -12,8 +12,9 @@
 // Node values are [node][batch] rows, so each edge gathers one contiguous
 // child row.
 //
-// Mapping.  CSR layers: csr_fwd_kernel, a wave per run of nodes and tile of 64
-// or 128 columns, its edges one stream.  The block layout (and some Q16.16 CSR
+// Mapping.  CSR layers: csr_fwd_narrow, several nodes per wave, up to 32
+// columns; csr_fwd_kernel, a wave per run of nodes and tile of 64 or 128
+// columns, its edges one stream.  The block layout (and some Q16.16 CSR
 // layers): sparse_kernel, one wave per (node, tile of 64, 128 or 256 columns);
 // lane l owns 1, 2 or 4 columns (one vector when the batch is a multiple of it
 // and rows are aligned, else strided scalars), edge metadata is held one
@@ -657,7 +658,6 @@ __global__ __launch_bounds__(64) void csr_fwd_kernel(const float* __restrict__ c
         return;
     }
     const Run run{(int32_t)(at - e0)};
-    const int32_t edges = run.start(nn);
     const int64_t nnz = uniform64(off[nodes]);
     const u32x4v rc = words_rsrc(cids + e0, nnz - e0), rl = words_rsrc(logp + e0, nnz - e0);
     const float* child_b0 = child + b0;
@@ -708,6 +708,219 @@ __global__ __launch_bounds__(64) void csr_fwd_kernel(const float* __restrict__ c
     }
 }
 
+// ---------------------------------------------------------------------------
+// Batches of up to 32 columns: LG lanes (a power of two >= the batch) per node,
+// 64 / LG nodes per wave, so a narrow batch does not leave a wave's lanes idle.
+// A group folds the edges of its own node, four at a time, up to kOwnEdges of
+// them; the wave's groups then take each longer node together, an edge (Q16.16:
+// a chain of the node's eight) per group in turn, so that a large fan-in is not
+// one group's serial chain.  Loads are unconditional: ids and weights through
+// buffer ranges (an edge past the node's reads as id 0), a child row 0 there
+// and the last column in idle lanes, all masked after.  Against a wave per run
+// of nodes (csr_fwd_kernel with 1 column a lane; us, fp32 / Q16.16 / backward):
+// 300000 nodes, batch 4: 137 / 159 / 214 -> 33 / 50 / 142, batch 16 135 / 159 /
+// 215 -> 64 / 78 / 167, batch 32 133 / 157 / 214 -> 103 / 126 / 171; 2000 nodes,
+// batch 16, where the largest fan-in's chain is the time, 20.9 / 31.8 / 11.6 ->
+// 12.4 / 13.6 / 11.8.
+// ---------------------------------------------------------------------------
+constexpr int64_t kNarrowBatch = 32;
+constexpr int kOwnEdges = 32;  // fan-ins of one, two or four Q16.16 chains
+
+// A value of lane (lane ^ mask).
+__device__ __forceinline__ float shuffle_xor(float v, int mask) { return __shfl_xor(v, mask, 64); }
+__device__ __forceinline__ uint32_t shuffle_xor(uint32_t v, int mask) { return (uint32_t)__shfl_xor((int)v, mask, 64); }
+
+// Edges of the wave's nodes by their place in the run (the wave's node 0 starts
+// at 0): ids and weights with range checks.
+struct RunEdges {
+    __amdgpu_buffer_rsrc_t ids, lws;
+    const float* child;
+    int64_t batch;
+    int col;
+    // logits of edge i, -inf where !ok
+    __device__ __forceinline__ float logit(int32_t i, bool ok) const {
+        const int at = ok ? i * 4 : 0x7FFFFFFC;
+        const uint32_t id = __builtin_amdgcn_raw_buffer_load_b32(ids, at, 0, 0);
+        const float lw = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(lws, at, 0, 0));
+        const float t = lw + child[(int64_t)id * batch + col];
+        return ok ? t : -kInf;
+    }
+};
+
+template <bool Q16, int LG>
+__global__ __launch_bounds__(64) void csr_fwd_narrow(const float* __restrict__ child, const int64_t* __restrict__ off,
+                                                     const int32_t* __restrict__ cids, const float* __restrict__ logp,
+                                                     float* __restrict__ out, int64_t batch, int64_t nodes,
+                                                     int64_t block0) {
+    constexpr int NG = 64 / LG;
+    __shared__ int lut[64];
+    if constexpr (Q16) {
+        lut[threadIdx.x] = kLut[threadIdx.x];
+        __builtin_amdgcn_wave_barrier();
+    }
+    const int l = lane_id();
+    const int grp = l / LG, b = l % LG;
+    const int64_t n0 = (block0 + blockIdx.x) * NG;
+    const int64_t n = n0 + grp;
+    const int64_t nc = n < nodes ? n : nodes - 1;
+    const int64_t start = off[nc], e0 = uniform64(start);
+    const int64_t k64 = n < nodes ? off[nc + 1] - start : 0;
+    const int64_t total = uniform64(off[n0 + NG < nodes ? n0 + NG : nodes]) - e0;
+    float res = -kInf;
+    if (total > kRunEdges) {  // beyond 32-bit edge numbers: one edge at a time
+        const int64_t col = b < batch ? b : 0;
+        if constexpr (Q16) {
+            const int et = k64 <= 8 ? 1 : k64 <= 16 ? 2 : k64 <= 32 ? 4 : 8;
+            uint32_t acc[8];
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+                acc[c] = kNegInfU;
+                if (c < et)
+                    for (int64_t e = start + c; e < start + k64; e += et)
+                        acc[c] = pair(acc[c], quant(logp[e] + child[(int64_t)cids[e] * batch + col]), lut);
+            }
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                if (et > 4) acc[c] = pair(acc[c], acc[c + 4], lut);
+#pragma unroll
+            for (int c = 0; c < 2; ++c)
+                if (et > 2) acc[c] = pair(acc[c], acc[c + 2], lut);
+            if (et > 1) acc[0] = pair(acc[0], acc[1], lut);
+            const int q = (int)(acc[0] ^ kQBias);
+            res = q > kNegInfQ ? (float)q * kOutScale : -kInf;
+        } else {
+            float m = -kInf, s = 0.0f;
+            for (int64_t e = start; e < start + k64; e += 4) {  // groups of four, as the other kernels' sums
+                float t[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    t[u] = e + u < start + k64 ? logp[e + u] + child[(int64_t)cids[e + u] * batch + col] : -kInf;
+                lse_fold<true, 4>(m, s, t);
+            }
+            res = lse_finish<true>(m, s);
+        }
+    } else if (total > 0) {
+        const int64_t nnz = uniform64(off[nodes]);
+        const int left = (int)(nnz - e0 < kRunEdges * 2 ? nnz - e0 : kRunEdges * 2) * 4;
+        const RunEdges E{__builtin_amdgcn_make_buffer_rsrc(const_cast<int32_t*>(cids + e0), 0, left, 0x00020000),
+                         __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(logp + e0), 0, left, 0x00020000), child,
+                         batch, b < batch ? b : (int)batch - 1};
+        const int32_t s0 = (int32_t)(start - e0), k = (int32_t)k64;
+        const int32_t own = k <= kOwnEdges ? k : 0;
+        uint64_t longer = __ballot(k > kOwnEdges && b == 0);
+        if constexpr (Q16) {
+            uint32_t a0 = kNegInfU, a1 = kNegInfU, a2 = kNegInfU, a3 = kNegInfU;
+            const bool two = own > 8, four = own > 16;  // two or more chains, four
+            for (int32_t e = 0; __any(e < own); e += 4) {
+                float t[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) t[u] = E.logit(s0 + e + u, e + u < own);
+                // edge u belongs to chain u mod 1, 2 or 4; a masked one leaves its chain
+                const auto step = [&](uint32_t acc, int u) {
+                    const uint32_t r = pair(acc, quant(t[u]), lut);
+                    return e + u < own ? r : acc;
+                };
+                a0 = step(a0, 0);
+                const uint32_t r1 = step(two ? a1 : a0, 1);
+                a0 = two ? a0 : r1;
+                a1 = two ? r1 : a1;
+                const uint32_t r2 = step(four ? a2 : a0, 2);
+                a0 = four ? a0 : r2;
+                a2 = four ? r2 : a2;
+                const uint32_t r3 = step(four ? a3 : two ? a1 : a0, 3);
+                a0 = two ? a0 : r3;
+                a1 = two && !four ? r3 : a1;
+                a3 = four ? r3 : a3;
+            }
+            const uint32_t p0 = pair(a0, a2, lut), p1 = pair(a1, a3, lut);
+            a0 = four ? p0 : a0;
+            a1 = four ? p1 : a1;
+            const uint32_t p = pair(a0, a1, lut);
+            a0 = two ? p : a0;
+            // a longer node's chain grp + NC * i in acc[i]
+            constexpr int NC = NG < 8 ? NG : 8, CPG = 8 / NC;
+            while (longer) {
+                const int j = __builtin_ctzll(longer);
+                longer &= longer - 1;
+                const int32_t sj = __builtin_amdgcn_readlane(s0, j), kj = __builtin_amdgcn_readlane(k, j);
+                uint32_t acc[CPG];
+#pragma unroll
+                for (int i = 0; i < CPG; ++i) acc[i] = kNegInfU;
+                for (int32_t r = 0; r < kj; r += 16) {
+                    float t[2][CPG];
+#pragma unroll
+                    for (int v = 0; v < 2; ++v)
+#pragma unroll
+                        for (int i = 0; i < CPG; ++i) {
+                            const int32_t e = r + 8 * v + grp + NC * i;
+                            t[v][i] = E.logit(sj + e, grp < NC && e < kj);
+                        }
+#pragma unroll
+                    for (int v = 0; v < 2; ++v)
+#pragma unroll
+                        for (int i = 0; i < CPG; ++i) {
+                            const uint32_t p = pair(acc[i], quant(t[v][i]), lut);
+                            acc[i] = r + 8 * v + grp + NC * i < kj ? p : acc[i];
+                        }
+                }
+                // xor butterfly, distances 4, 2, 1: inside the lane while a
+                // chain's partner is there, then across the groups
+#pragma unroll
+                for (int d = 4; d >= 1; d >>= 1) {
+                    if (d >= NC) {
+#pragma unroll
+                        for (int i = 0; i < d / NC; ++i) acc[i] = pair(acc[i], acc[i + d / NC], lut);
+                    } else {
+                        acc[0] = pair(acc[0], shuffle_xor(acc[0], d * LG), lut);
+                    }
+                }
+                const uint32_t r = (uint32_t)__shfl((int)acc[0], b, 64);  // group 0's
+                a0 = grp == j / LG ? r : a0;
+            }
+            const int q = (int)(a0 ^ kQBias);
+            res = q > kNegInfQ ? (float)q * kOutScale : -kInf;
+        } else {
+            float m = -kInf, s = 0.0f;
+            for (int32_t e = 0; __any(e < own); e += 4) {
+                float t[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) t[u] = E.logit(s0 + e + u, e + u < own);
+                lse_fold<true, 4>(m, s, t);
+            }
+            while (longer) {
+                const int j = __builtin_ctzll(longer);
+                longer &= longer - 1;
+                const int32_t sj = __builtin_amdgcn_readlane(s0, j), kj = __builtin_amdgcn_readlane(k, j);
+                float mj = -kInf, sum = 0.0f;
+                for (int32_t r = 0; r < kj; r += 4 * NG) {
+                    float t[4];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) t[u] = E.logit(sj + r + u * NG + grp, r + u * NG + grp < kj);
+                    lse_fold<true, 4>(mj, sum, t);
+                }
+#pragma unroll
+                for (int d = LG; d < 64; d <<= 1) {
+                    const float m2 = shuffle_xor(mj, d), s2 = shuffle_xor(sum, d);
+                    lse_merge(mj, sum, m2, s2);
+                }
+                m = grp == j / LG ? mj : m;
+                s = grp == j / LG ? sum : s;
+            }
+            res = lse_finish<true>(m, s);
+        }
+    }
+    if (n < nodes && b < batch) out[n * batch + b] = res;
+}
+
+template <bool Q16, int LG>
+static void launch_csr_narrow(const CsrLayout& L, const float* child, int64_t nodes, hipStream_t st) {
+    constexpr int NG = 64 / LG;
+    for_grid_chunks((nodes + NG - 1) / NG, 64, [&](int64_t b0, int64_t nb) {
+        csr_fwd_narrow<Q16, LG><<<dim3((unsigned)nb), dim3(64), 0, st>>>(child, L.offsets, L.cids, L.logp, L.out,
+                                                                         L.batch, nodes, b0);
+    });
+}
+
 // Nodes per run, by the (node, column tile) pairs of the launch: longer runs
 // spare more of the wave starts, shorter ones keep a small layer's waves many
 // and its largest nodes apart (MI355X, fan-in k^-2 on [2, 256], us at 1 / 2 /
@@ -732,7 +945,8 @@ static void launch_csr_cols(const CsrLayout& L, const float* child, int64_t node
 // and at most a tenth of the last slice's lanes idle over all of them.
 static bool slices_fit(int64_t batch) { return batch % 32 == 0 && batch * 10 >= (batch + 127) / 128 * 128 * 9; }
 
-// Columns per lane: 1 up to a batch of 64, else 2 (200000 nodes, fp32, us, 1 / 2
+// Up to 32 columns: several nodes per wave (csr_fwd_narrow).  Columns per lane
+// above: 1 up to a batch of 64, else 2 (200000 nodes, fp32, us, 1 / 2
 // columns a lane: batch 64 99 / 105, 100 182 / 142, 512 515 / 497; 4 columns
 // 140, 152, 519).  Large layers whose rows do not cut into such slices take
 // tiles of 256 columns, in fp32 through the stream (us, 128 / 256 columns: 1M x
@@ -744,6 +958,17 @@ template <bool Q16>
 static void launch_csr(const CsrLayout& L, const float* child, int64_t nodes, hipStream_t st) {
     const uintptr_t at = reinterpret_cast<uintptr_t>(child) | reinterpret_cast<uintptr_t>(L.out);
     const int64_t batch = L.batch;
+    if (batch <= kNarrowBatch) {
+        if (batch <= 4)
+            launch_csr_narrow<Q16, 4>(L, child, nodes, st);
+        else if (batch <= 8)
+            launch_csr_narrow<Q16, 8>(L, child, nodes, st);
+        else if (batch <= 16)
+            launch_csr_narrow<Q16, 16>(L, child, nodes, st);
+        else
+            launch_csr_narrow<Q16, 32>(L, child, nodes, st);
+        return;
+    }
     if (batch <= 64) {
         launch_csr_cols<Q16, 1, 1>(L, child, nodes, run_nodes(nodes), st);
         return;
@@ -975,6 +1200,109 @@ __global__ __launch_bounds__(64) void csr_bwd_kernel(const float* __restrict__ c
     }
 }
 
+// The backward of a batch of up to 32 columns: csr_fwd_narrow's walk over the
+// children, LG lanes per child, both of an edge's parent rows per lane group.
+// An edge's sum is reduced over its group's lanes, four edges at a time.
+template <int LG>
+__global__ __launch_bounds__(64) void csr_bwd_narrow(const float* __restrict__ child, const float* __restrict__ out,
+                                                     const float* __restrict__ gout, const float* __restrict__ logp,
+                                                     const int64_t* __restrict__ csc_off,
+                                                     const int32_t* __restrict__ csc_edge,
+                                                     const int32_t* __restrict__ csc_node,
+                                                     float* __restrict__ gchild, float* __restrict__ glogp,
+                                                     int64_t children, int64_t batch, int64_t block0) {
+    constexpr int NG = 64 / LG;
+    const int l = lane_id();
+    const int grp = l / LG, b = l % LG;
+    const int64_t c0 = (block0 + blockIdx.x) * NG;
+    const int64_t c = c0 + grp;
+    const int64_t cc = c < children ? c : children - 1;
+    const int64_t start = csc_off[cc], e0 = uniform64(start);
+    const int64_t k64 = c < children ? csc_off[cc + 1] - start : 0;
+    const int64_t total = uniform64(csc_off[c0 + NG < children ? c0 + NG : children]) - e0;
+    const bool col_ok = b < batch;
+    const int64_t col = col_ok ? b : batch - 1;
+    const float x = child[cc * batch + col];
+    float acc = 0.0f;
+    if (total > kRunEdges) {  // beyond 32-bit edge numbers: one edge at a time
+        for (int64_t k = start; __any(k < start + k64); ++k) {
+            const bool ok = k < start + k64;
+            const int64_t kk = ok ? k : e0, row = (int64_t)csc_node[kk] * batch + col, e = csc_edge[kk];
+            float t = flow(gout[row], logp[e] + x, out[row], ok && col_ok);
+            acc += t;
+            for (int d = 1; d < LG; d <<= 1) t += shuffle_xor(t, d);
+            if (ok && b == 0) glogp[e] = t;
+        }
+    } else if (total > 0) {
+        const int64_t nnz = uniform64(csc_off[children]);
+        const int left = (int)(nnz - e0 < kRunEdges * 2 ? nnz - e0 : kRunEdges * 2) * 4;
+        const __amdgpu_buffer_rsrc_t re =
+            __builtin_amdgcn_make_buffer_rsrc(const_cast<int32_t*>(csc_edge + e0), 0, left, 0x00020000);
+        const __amdgpu_buffer_rsrc_t rn =
+            __builtin_amdgcn_make_buffer_rsrc(const_cast<int32_t*>(csc_node + e0), 0, left, 0x00020000);
+        // four edges i[u] of a child with value xv: their terms into sum,
+        // their sums over the batch into glogp
+        const auto four = [&](const int32_t (&i)[4], const bool (&ok)[4], float xv, float& sum) {
+            uint32_t ed[4];
+            float t[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int at = ok[u] ? i[u] * 4 : 0x7FFFFFFC;
+                ed[u] = __builtin_amdgcn_raw_buffer_load_b32(re, at, 0, 0);
+                const int64_t row = (int64_t)(uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rn, at, 0, 0) * batch + col;
+                t[u] = flow(gout[row], logp[ed[u]] + xv, out[row], ok[u] && col_ok);
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) sum += t[u];
+            const bool odd = b & 1, hi = b & 2;
+            const float p = (odd ? t[1] : t[0]) + reduce_partner<1>(odd ? t[0] : t[1]);
+            const float q = (odd ? t[3] : t[2]) + reduce_partner<1>(odd ? t[2] : t[3]);
+            float s = (hi ? q : p) + reduce_partner<2>(hi ? p : q);  // lane b: edge b % 4 over its quad
+            if constexpr (LG >= 8) s += exact_xor<4>(s);
+            if constexpr (LG >= 16) s += exact_xor<8>(s);
+            if constexpr (LG >= 32) s += exact_xor<16>(s);
+            const uint32_t lo = odd ? ed[1] : ed[0], up = odd ? ed[3] : ed[2];
+            const bool mine = hi ? (odd ? ok[3] : ok[2]) : (odd ? ok[1] : ok[0]);
+            if (b < 4 && mine) glogp[hi ? up : lo] = s;
+        };
+        const int32_t s0 = (int32_t)(start - e0), k = (int32_t)k64;
+        const int32_t own = k <= kOwnEdges ? k : 0;
+        uint64_t longer = __ballot(k > kOwnEdges && b == 0);
+        for (int32_t e = 0; __any(e < own); e += 4) {
+            const int32_t i[4] = {s0 + e, s0 + e + 1, s0 + e + 2, s0 + e + 3};
+            const bool ok[4] = {e < own, e + 1 < own, e + 2 < own, e + 3 < own};
+            four(i, ok, x, acc);
+        }
+        while (longer) {
+            const int j = __builtin_ctzll(longer);
+            longer &= longer - 1;
+            const int32_t sj = __builtin_amdgcn_readlane(s0, j), kj = __builtin_amdgcn_readlane(k, j);
+            const float xj = child[(c0 + j / LG) * batch + col];
+            float sum = 0.0f;
+            for (int32_t r = grp; __any(r < kj); r += 4 * NG) {
+                const int32_t i[4] = {sj + r, sj + r + NG, sj + r + 2 * NG, sj + r + 3 * NG};
+                const bool ok[4] = {r < kj, r + NG < kj, r + 2 * NG < kj, r + 3 * NG < kj};
+                four(i, ok, xj, sum);
+            }
+#pragma unroll
+            for (int d = LG; d < 64; d <<= 1) sum += shuffle_xor(sum, d);
+            acc = grp == j / LG ? sum : acc;
+        }
+    }
+    if (c < children && col_ok) gchild[c * batch + b] = acc;
+}
+
+template <int LG>
+static void launch_csr_bwd_narrow(const float* child, const float* out, const float* gout, const float* logp,
+                                  const int64_t* off, const int32_t* edge, const int32_t* node, float* gchild,
+                                  float* glogp, int64_t children, int64_t batch, hipStream_t st) {
+    constexpr int NG = 64 / LG;
+    for_grid_chunks((children + NG - 1) / NG, 64, [&](int64_t b0, int64_t nb) {
+        csr_bwd_narrow<LG><<<dim3((unsigned)nb), dim3(64), 0, st>>>(child, out, gout, logp, off, edge, node, gchild,
+                                                                    glogp, children, batch, b0);
+    });
+}
+
 template <bool DIRECT, int VW, int P>
 static void launch_csr_bwd_cols(const float* child, const float* out, const float* gout, const float* logp,
                                 const int64_t* off, const int32_t* edge, const int32_t* node, float* gchild,
@@ -1131,6 +1459,20 @@ static void launch_csr_bwd_rows(const float* child, const float* out, const floa
 static void launch_csr_bwd_plain(const float* child, const float* out, const float* gout, const float* logp,
                                  const int64_t* off, const int32_t* edge, const int32_t* node, float* gchild,
                                  float* glogp, int64_t children, int64_t batch, hipStream_t st) {
+    if (batch <= kNarrowBatch) {
+        const auto go = [&](auto launch) {
+            launch(child, out, gout, logp, off, edge, node, gchild, glogp, children, batch, st);
+        };
+        if (batch <= 4)
+            go(launch_csr_bwd_narrow<4>);
+        else if (batch <= 8)
+            go(launch_csr_bwd_narrow<8>);
+        else if (batch <= 16)
+            go(launch_csr_bwd_narrow<16>);
+        else
+            go(launch_csr_bwd_narrow<32>);
+        return;
+    }
     if (batch <= bwd_tile_cols(batch))
         launch_csr_bwd<true>(child, out, gout, logp, off, edge, node, gchild, glogp, children, batch, st);
     else

@@ -696,7 +696,8 @@ def _csr_fp64_torch(child, off, cids, lp):
     return top + torch.log(total), parent, t
 
 
-@pytest.mark.parametrize("nodes,batch", [(61, 1), (61, 63), (61, 64), (61, 65), (61, 127), (61, 128), (61, 129),
+@pytest.mark.parametrize("nodes,batch", [(61, 1), (61, 4), (61, 5), (61, 8), (61, 9), (61, 16), (61, 17), (61, 32),
+                                         (61, 33), (32, 3), (33, 16), (61, 63), (61, 64), (61, 65), (61, 127), (61, 128), (61, 129),
                                          (61, 256), (61, 510), (40001, 3), (20001, 130), (160003, 1), (40001, 200),
                                          (40001, 132)])
 def test_csr_forward_runs(cuda, nodes, batch):
@@ -719,7 +720,7 @@ def test_csr_forward_runs(cuda, nodes, batch):
     np.testing.assert_array_equal(gq.view(np.int32), O.sparse_q16_csr(child, off, cids, lp).view(np.int32))
 
 
-@pytest.mark.parametrize("batch", [5, 130])
+@pytest.mark.parametrize("batch", [3, 5, 12, 31, 40, 130])
 def test_csr_forward_special_values(cuda, batch):
     """-inf, +inf, NaN and magnitudes past the fused exponent's range, in a
     node's first group and in later ones."""
@@ -739,12 +740,13 @@ def test_csr_forward_special_values(cuda, batch):
     np.testing.assert_allclose(got, O.sparse_csr_fp64(child, off, cids, lp), rtol=1e-5, atol=1e-6)
 
 
-def test_csr_q16_saturated_pairs(cuda):
+@pytest.mark.parametrize("batch", [3, 7, 13, 29, 70])
+def test_csr_q16_saturated_pairs(cuda, batch):
     """Logits around the int32 limit (22713.2 saturates) and around the clamp
     at -20000, so that differences reach 2^32 and a maximum plus its correction
     passes 2^31: every bit as in the reference's 32-bit arithmetic."""
     rng = np.random.default_rng(9)
-    nodes, nch, batch = 300, 64, 70
+    nodes, nch = 300, 64
     off, cids, _ = _csr(rng, nodes, nch, fanin=rng.integers(1, 40, nodes))
     lp = np.zeros(off[-1], np.float32)
     child = rng.choice(np.float32([22713.3, 22713.2, 22713.1, 22713, 22702, 22701.5, 22690, 0, -20000, -3e4, -np.inf,
@@ -754,7 +756,8 @@ def test_csr_q16_saturated_pairs(cuda):
     np.testing.assert_array_equal(gq.view(np.int32), O.sparse_q16_csr(child, off, cids, lp).view(np.int32))
 
 
-@pytest.mark.parametrize("nodes,children,batch", [(300, 61, 1), (300, 61, 64), (300, 61, 65), (300, 61, 128),
+@pytest.mark.parametrize("nodes,children,batch", [(300, 61, 1), (300, 61, 4), (300, 61, 7), (300, 61, 16), (300, 61, 30),
+                                                  (300, 61, 33), (3000, 16, 2), (300, 61, 64), (300, 61, 65), (300, 61, 128),
                                                   (30000, 40001, 3), (20000, 16100, 512), (20000, 22000, 384)])
 def test_csr_backward_runs(cuda, nodes, children, batch):
     """The streamed backward: one tile (weights and sums by edge id) and, from
@@ -784,7 +787,7 @@ def test_csr_backward_runs(cuda, nodes, children, batch):
     assert ((gc.double() - want).abs() <= 1e-5 * size + 1e-30).all()
 
 
-@pytest.mark.parametrize("batch", [3, 130])
+@pytest.mark.parametrize("batch", [3, 40, 130])
 def test_csr_runs_past_the_streams_edges(cuda, batch):
     """A node, and a child, of more edges than the stream's 32-bit edge numbers
     are for (2^20 a run), between ordinary ones."""
