@@ -32,6 +32,8 @@
 #include <math.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "../../include/fuselse_amd.h"
 #include "fl_status.hpp"
 #include "lse_blocked.hpp"
@@ -730,22 +732,156 @@ constexpr int kOwnEdges = 32;  // fan-ins of one, two or four Q16.16 chains
 __device__ __forceinline__ float shuffle_xor(float v, int mask) { return __shfl_xor(v, mask, 64); }
 __device__ __forceinline__ uint32_t shuffle_xor(uint32_t v, int mask) { return (uint32_t)__shfl_xor((int)v, mask, 64); }
 
-// Edges of the wave's nodes by their place in the run (the wave's node 0 starts
-// at 0): ids and weights with range checks.
-struct RunEdges {
+// The edges of the nodes a wave's lane groups hold.  Node: what says where a
+// node's edges are; logit(node, i, ok): the lane's column of its edge i, -inf
+// where !ok; of_lane(node, j): lane j's, wave-uniform.
+// CSR: Node is the node's first edge's place in the wave's run of edges, and ids
+// and weights have range checks.
+struct CsrNarrow {
+    typedef int32_t Node;
     __amdgpu_buffer_rsrc_t ids, lws;
     const float* child;
     int64_t batch;
     int col;
-    // logits of edge i, -inf where !ok
-    __device__ __forceinline__ float logit(int32_t i, bool ok) const {
-        const int at = ok ? i * 4 : 0x7FFFFFFC;
+    __device__ __forceinline__ float logit(Node first, int32_t i, bool ok) const {
+        const int at = ok ? (first + i) * 4 : 0x7FFFFFFC;
         const uint32_t id = __builtin_amdgcn_raw_buffer_load_b32(ids, at, 0, 0);
         const float lw = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(lws, at, 0, 0));
         const float t = lw + child[(int64_t)id * batch + col];
         return ok ? t : -kInf;
     }
+    __device__ __forceinline__ Node of_lane(Node n, int j) const { return __builtin_amdgcn_readlane(n, j); }
 };
+// Block layout: Node is the parent's number (block * block_size + position); an
+// edge past the node's reads the block's first.
+template <bool LOGP>
+struct BlockNarrow {
+    typedef int64_t Node;
+    BlockLayout<LOGP> L;
+    const float* child;
+    int col;
+    __device__ __forceinline__ float logit(Node item, int32_t i, bool ok) const {
+        const int64_t j = div_small(item, L.block_size);
+        const EdgeMeta m = L.meta({j * L.num_edges, L.num_edges, item - j * L.block_size, 0}, ok ? i : 0);
+        const float t = m.logw + child[m.cid * L.batch + col];
+        return ok ? t : -kInf;
+    }
+    __device__ __forceinline__ Node of_lane(Node n, int j) const { return bcast64(n, j); }
+    __device__ static __forceinline__ int64_t div_small(int64_t a, int64_t b) {
+        return ((uint64_t)a | (uint64_t)b) >> 32 ? a / b : (int64_t)((uint32_t)a / (uint32_t)b);
+    }
+};
+
+// The result of each group's node (k edges, 0 for none) in the group's lanes.
+template <bool Q16, int LG, typename EDGES>
+__device__ __forceinline__ float reduce_narrow(const EDGES& E, const typename EDGES::Node node, int32_t k,
+                                               const int* __restrict__ lut) {
+    constexpr int NG = 64 / LG;
+    const int l = lane_id();
+    const int grp = l / LG, b = l % LG;
+    const int32_t own = k <= kOwnEdges ? k : 0;
+    uint64_t longer = __ballot(k > kOwnEdges && b == 0);
+    if constexpr (Q16) {
+        uint32_t a0 = kNegInfU, a1 = kNegInfU, a2 = kNegInfU, a3 = kNegInfU;
+        const bool two = own > 8, four = own > 16;  // two or more chains, four
+        for (int32_t e = 0; __any(e < own); e += 4) {
+            float t[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) t[u] = E.logit(node, e + u, e + u < own);
+            // edge u belongs to chain u mod 1, 2 or 4; a masked one leaves its chain
+            const auto step = [&](uint32_t acc, int u) {
+                const uint32_t r = pair(acc, quant(t[u]), lut);
+                return e + u < own ? r : acc;
+            };
+            a0 = step(a0, 0);
+            const uint32_t r1 = step(two ? a1 : a0, 1);
+            a0 = two ? a0 : r1;
+            a1 = two ? r1 : a1;
+            const uint32_t r2 = step(four ? a2 : a0, 2);
+            a0 = four ? a0 : r2;
+            a2 = four ? r2 : a2;
+            const uint32_t r3 = step(four ? a3 : two ? a1 : a0, 3);
+            a0 = two ? a0 : r3;
+            a1 = two && !four ? r3 : a1;
+            a3 = four ? r3 : a3;
+        }
+        const uint32_t p0 = pair(a0, a2, lut), p1 = pair(a1, a3, lut);
+        a0 = four ? p0 : a0;
+        a1 = four ? p1 : a1;
+        const uint32_t p = pair(a0, a1, lut);
+        a0 = two ? p : a0;
+        // a longer node's chain grp + NC * i in acc[i]
+        constexpr int NC = NG < 8 ? NG : 8, CPG = 8 / NC;
+        while (longer) {
+            const int j = __builtin_ctzll(longer);
+            longer &= longer - 1;
+            const typename EDGES::Node nj = E.of_lane(node, j);
+            const int32_t kj = __builtin_amdgcn_readlane(k, j);
+            uint32_t acc[CPG];
+#pragma unroll
+            for (int i = 0; i < CPG; ++i) acc[i] = kNegInfU;
+            for (int32_t r = 0; r < kj; r += 16) {
+                float t[2][CPG];
+#pragma unroll
+                for (int v = 0; v < 2; ++v)
+#pragma unroll
+                    for (int i = 0; i < CPG; ++i) {
+                        const int32_t e = r + 8 * v + grp + NC * i;
+                        t[v][i] = E.logit(nj, e, grp < NC && e < kj);
+                    }
+#pragma unroll
+                for (int v = 0; v < 2; ++v)
+#pragma unroll
+                    for (int i = 0; i < CPG; ++i) {
+                        const uint32_t p = pair(acc[i], quant(t[v][i]), lut);
+                        acc[i] = r + 8 * v + grp + NC * i < kj ? p : acc[i];
+                    }
+            }
+            // xor butterfly, distances 4, 2, 1: inside the lane while a
+            // chain's partner is there, then across the groups
+            if constexpr (CPG == 4) {
+                acc[0] = pair(acc[0], acc[2], lut);
+                acc[1] = pair(acc[1], acc[3], lut);
+            }
+            if constexpr (CPG >= 2) acc[0] = pair(acc[0], acc[1], lut);
+            if constexpr (CPG == 1) acc[0] = pair(acc[0], shuffle_xor(acc[0], 4 * LG), lut);
+            if constexpr (CPG <= 2) acc[0] = pair(acc[0], shuffle_xor(acc[0], 2 * LG), lut);
+            acc[0] = pair(acc[0], shuffle_xor(acc[0], LG), lut);
+            const uint32_t r = (uint32_t)__shfl((int)acc[0], b, 64);  // group 0's
+            a0 = grp == j / LG ? r : a0;
+        }
+        const int q = (int)(a0 ^ kQBias);
+        return q > kNegInfQ ? (float)q * kOutScale : -kInf;
+    } else {
+        float m = -kInf, s = 0.0f;
+        for (int32_t e = 0; __any(e < own); e += 4) {
+            float t[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) t[u] = E.logit(node, e + u, e + u < own);
+            lse_fold<true, 4>(m, s, t);
+        }
+        while (longer) {
+            const int j = __builtin_ctzll(longer);
+            longer &= longer - 1;
+            const typename EDGES::Node nj = E.of_lane(node, j);
+            const int32_t kj = __builtin_amdgcn_readlane(k, j);
+            float mj = -kInf, sum = 0.0f;
+            for (int32_t r = 0; r < kj; r += 4 * NG) {
+                float t[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) t[u] = E.logit(nj, r + u * NG + grp, r + u * NG + grp < kj);
+                lse_fold<true, 4>(mj, sum, t);
+            }
+            for (int d = LG; d < 64; d <<= 1) {
+                const float m2 = shuffle_xor(mj, d), s2 = shuffle_xor(sum, d);
+                lse_merge(mj, sum, m2, s2);
+            }
+            m = grp == j / LG ? mj : m;
+            s = grp == j / LG ? sum : s;
+        }
+        return lse_finish<true>(m, s);
+    }
+}
 
 template <bool Q16, int LG>
 __global__ __launch_bounds__(64) void csr_fwd_narrow(const float* __restrict__ child, const int64_t* __restrict__ off,
@@ -802,114 +938,61 @@ __global__ __launch_bounds__(64) void csr_fwd_narrow(const float* __restrict__ c
     } else if (total > 0) {
         const int64_t nnz = uniform64(off[nodes]);
         const int left = (int)(nnz - e0 < kRunEdges * 2 ? nnz - e0 : kRunEdges * 2) * 4;
-        const RunEdges E{__builtin_amdgcn_make_buffer_rsrc(const_cast<int32_t*>(cids + e0), 0, left, 0x00020000),
-                         __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(logp + e0), 0, left, 0x00020000), child,
-                         batch, b < batch ? b : (int)batch - 1};
-        const int32_t s0 = (int32_t)(start - e0), k = (int32_t)k64;
-        const int32_t own = k <= kOwnEdges ? k : 0;
-        uint64_t longer = __ballot(k > kOwnEdges && b == 0);
-        if constexpr (Q16) {
-            uint32_t a0 = kNegInfU, a1 = kNegInfU, a2 = kNegInfU, a3 = kNegInfU;
-            const bool two = own > 8, four = own > 16;  // two or more chains, four
-            for (int32_t e = 0; __any(e < own); e += 4) {
-                float t[4];
-#pragma unroll
-                for (int u = 0; u < 4; ++u) t[u] = E.logit(s0 + e + u, e + u < own);
-                // edge u belongs to chain u mod 1, 2 or 4; a masked one leaves its chain
-                const auto step = [&](uint32_t acc, int u) {
-                    const uint32_t r = pair(acc, quant(t[u]), lut);
-                    return e + u < own ? r : acc;
-                };
-                a0 = step(a0, 0);
-                const uint32_t r1 = step(two ? a1 : a0, 1);
-                a0 = two ? a0 : r1;
-                a1 = two ? r1 : a1;
-                const uint32_t r2 = step(four ? a2 : a0, 2);
-                a0 = four ? a0 : r2;
-                a2 = four ? r2 : a2;
-                const uint32_t r3 = step(four ? a3 : two ? a1 : a0, 3);
-                a0 = two ? a0 : r3;
-                a1 = two && !four ? r3 : a1;
-                a3 = four ? r3 : a3;
-            }
-            const uint32_t p0 = pair(a0, a2, lut), p1 = pair(a1, a3, lut);
-            a0 = four ? p0 : a0;
-            a1 = four ? p1 : a1;
-            const uint32_t p = pair(a0, a1, lut);
-            a0 = two ? p : a0;
-            // a longer node's chain grp + NC * i in acc[i]
-            constexpr int NC = NG < 8 ? NG : 8, CPG = 8 / NC;
-            while (longer) {
-                const int j = __builtin_ctzll(longer);
-                longer &= longer - 1;
-                const int32_t sj = __builtin_amdgcn_readlane(s0, j), kj = __builtin_amdgcn_readlane(k, j);
-                uint32_t acc[CPG];
-#pragma unroll
-                for (int i = 0; i < CPG; ++i) acc[i] = kNegInfU;
-                for (int32_t r = 0; r < kj; r += 16) {
-                    float t[2][CPG];
-#pragma unroll
-                    for (int v = 0; v < 2; ++v)
-#pragma unroll
-                        for (int i = 0; i < CPG; ++i) {
-                            const int32_t e = r + 8 * v + grp + NC * i;
-                            t[v][i] = E.logit(sj + e, grp < NC && e < kj);
-                        }
-#pragma unroll
-                    for (int v = 0; v < 2; ++v)
-#pragma unroll
-                        for (int i = 0; i < CPG; ++i) {
-                            const uint32_t p = pair(acc[i], quant(t[v][i]), lut);
-                            acc[i] = r + 8 * v + grp + NC * i < kj ? p : acc[i];
-                        }
-                }
-                // xor butterfly, distances 4, 2, 1: inside the lane while a
-                // chain's partner is there, then across the groups
-#pragma unroll
-                for (int d = 4; d >= 1; d >>= 1) {
-                    if (d >= NC) {
-#pragma unroll
-                        for (int i = 0; i < d / NC; ++i) acc[i] = pair(acc[i], acc[i + d / NC], lut);
-                    } else {
-                        acc[0] = pair(acc[0], shuffle_xor(acc[0], d * LG), lut);
-                    }
-                }
-                const uint32_t r = (uint32_t)__shfl((int)acc[0], b, 64);  // group 0's
-                a0 = grp == j / LG ? r : a0;
-            }
-            const int q = (int)(a0 ^ kQBias);
-            res = q > kNegInfQ ? (float)q * kOutScale : -kInf;
-        } else {
-            float m = -kInf, s = 0.0f;
-            for (int32_t e = 0; __any(e < own); e += 4) {
-                float t[4];
-#pragma unroll
-                for (int u = 0; u < 4; ++u) t[u] = E.logit(s0 + e + u, e + u < own);
-                lse_fold<true, 4>(m, s, t);
-            }
-            while (longer) {
-                const int j = __builtin_ctzll(longer);
-                longer &= longer - 1;
-                const int32_t sj = __builtin_amdgcn_readlane(s0, j), kj = __builtin_amdgcn_readlane(k, j);
-                float mj = -kInf, sum = 0.0f;
-                for (int32_t r = 0; r < kj; r += 4 * NG) {
-                    float t[4];
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) t[u] = E.logit(sj + r + u * NG + grp, r + u * NG + grp < kj);
-                    lse_fold<true, 4>(mj, sum, t);
-                }
-#pragma unroll
-                for (int d = LG; d < 64; d <<= 1) {
-                    const float m2 = shuffle_xor(mj, d), s2 = shuffle_xor(sum, d);
-                    lse_merge(mj, sum, m2, s2);
-                }
-                m = grp == j / LG ? mj : m;
-                s = grp == j / LG ? sum : s;
-            }
-            res = lse_finish<true>(m, s);
-        }
+        const CsrNarrow E{__builtin_amdgcn_make_buffer_rsrc(const_cast<int32_t*>(cids + e0), 0, left, 0x00020000),
+                          __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(logp + e0), 0, left, 0x00020000), child,
+                          batch, b < batch ? b : (int)batch - 1};
+        res = reduce_narrow<Q16, LG>(E, (int32_t)(start - e0), (int32_t)k64, lut);
     }
     if (n < nodes && b < batch) out[n * batch + b] = res;
+}
+
+template <bool Q16, int LG, bool LOGP>
+__global__ __launch_bounds__(64) void block_fwd_narrow(BlockLayout<LOGP> L, const float* __restrict__ child,
+                                                       int64_t items, int per_wave, int64_t block0) {
+    // per_wave: parents a wave holds, 64 / LG or, the other groups only
+    // helping, 1
+    __shared__ int lut[64];
+    if constexpr (Q16) {
+        lut[threadIdx.x] = kLut[threadIdx.x];
+        __builtin_amdgcn_wave_barrier();
+    }
+    const int l = lane_id();
+    const int b = l % LG;
+    const int64_t item = (block0 + blockIdx.x) * per_wave + l / LG;
+    const bool ok = l / LG < per_wave && item < items;
+    const int64_t it = ok ? item : items - 1;
+    const BlockNarrow<LOGP> E{L, child, b < L.batch ? b : (int)L.batch - 1};
+    const float res = reduce_narrow<Q16, LG>(E, it, ok ? (int32_t)L.num_edges : 0, lut);
+    const int64_t j = BlockNarrow<LOGP>::div_small(it, L.block_size);
+    if (ok && b < L.batch) L.node_mars[(L.nids[j] + it - j * L.block_size) * L.batch + b] = res;
+}
+
+// Q16.16, us, a wave per (parent, 64 columns) -> this: 2048 x 32 parents, 32
+// edges, batch 4 237 -> 20, batch 32 238 -> 109; 1651 x 24 parents, 72 edges,
+// batch 3 345 -> 75; 200 x 16 parents, 100 edges, batch 4 55 -> 9.
+template <bool Q16, bool LOGP>
+static void launch_block(const BlockLayout<LOGP>& L, const float* child, int64_t items, hipStream_t st) {
+    if (L.batch > kNarrowBatch || L.num_edges == 0 || L.num_edges > kRunEdges) {
+        launch<Q16>(L, child, L.node_mars, items, L.batch, st);
+        return;
+    }
+    const auto go = [&](auto lg) {
+        constexpr int LG = decltype(lg)::value;
+        const int per = L.num_edges > kOwnEdges && items < 8192 ? 1 : 64 / LG;
+        for_grid_chunks((items + per - 1) / per, 64, [&](int64_t b0, int64_t nb) {
+            block_fwd_narrow<Q16, LG, LOGP><<<dim3((unsigned)nb), dim3(64), 0, st>>>(L, child, items, per, b0);
+        });
+    };
+    // parents of more than kOwnEdges edges are taken one after the other by all
+    // groups, of which Q16.16 uses eight; few enough of them take a wave each
+    if (L.batch <= 4 && L.num_edges <= kOwnEdges)
+        go(std::integral_constant<int, 4>{});
+    else if (L.batch <= 8)
+        go(std::integral_constant<int, 8>{});
+    else if (L.batch <= 16)
+        go(std::integral_constant<int, 16>{});
+    else
+        go(std::integral_constant<int, 32>{});
 }
 
 template <bool Q16, int LG>
@@ -1284,7 +1367,6 @@ __global__ __launch_bounds__(64) void csr_bwd_narrow(const float* __restrict__ c
                 const bool ok[4] = {r < kj, r + NG < kj, r + 2 * NG < kj, r + 3 * NG < kj};
                 four(i, ok, xj, sum);
             }
-#pragma unroll
             for (int d = LG; d < 64; d <<= 1) sum += shuffle_xor(sum, d);
             acc = grp == j / LG ? sum : acc;
         }
@@ -1581,12 +1663,12 @@ extern "C" int fl_sparse_blocked_fwd(float* node_mars, const float* element_mars
     const int64_t items = num_nblocks * block_size;
     if (params_are_log) {
         const sparse::BlockLayout<true> L{node_mars, params, nids, cids, pids, num_edges, block_size, batch};
-        if (q16) sparse::launch<true>(L, element_mars, node_mars, items, batch, st);
-        else sparse::launch<false>(L, element_mars, node_mars, items, batch, st);
+        if (q16) sparse::launch_block<true>(L, element_mars, items, st);
+        else sparse::launch_block<false>(L, element_mars, items, st);
     } else {
         const sparse::BlockLayout<false> L{node_mars, params, nids, cids, pids, num_edges, block_size, batch};
-        if (q16) sparse::launch<true>(L, element_mars, node_mars, items, batch, st);
-        else sparse::launch<false>(L, element_mars, node_mars, items, batch, st);
+        if (q16) sparse::launch_block<true>(L, element_mars, items, st);
+        else sparse::launch_block<false>(L, element_mars, items, st);
     }
     return launch_status(name);
 }

@@ -593,12 +593,14 @@ def _blocked_plan(nids, cids, pids, block_size, num_elements):
         qids = pids.reshape(-1)
     # parameter ranges of the block edges, sorted: disjoint when consecutive
     # starts are at least block_size apart (then each parameter flow has one
-    # writer and takes a plain add instead of an atomic one)
+    # writer and takes a plain add instead of an atomic one); blocks side by
+    # side in order from row 0 on write these rows in full
     starts = torch.sort(pids.reshape(-1)).values
-    disjoint = bool(starts.numel() < 2 or int((starts[1:] - starts[:-1]).min()) >= bs)
-    # blocks side by side from row 0 on, in any order
-    first_rows = torch.sort(nids).values
-    packed = nb > 0 and bool((first_rows == torch.arange(nb, device=dev, dtype=torch.int64) * bs).all())
+    disjoint = torch.ones((), dtype=torch.bool, device=dev)
+    if starts.numel() > 1:
+        disjoint = (starts[1:] - starts[:-1]).min() >= bs
+    packed = (nids == torch.arange(0, nb * bs, bs, dtype=torch.int64, device=dev)).all() if bs > 0 else ~disjoint
+    disjoint, packed = torch.stack((disjoint, packed)).tolist()
     return BlockedPlan(csc_off, order.to(torch.int32), nodes, qids, disjoint, nb * bs if packed else 0)
 
 

@@ -81,7 +81,8 @@ def _blocked(rng, nb, ne, bs, batch, nelem, nparams):
     return nids, cids, pids, params, em
 
 
-@pytest.mark.parametrize("ne,bs,batch", [(5, 4, 32), (12, 2, 130), (30, 3, 512), (70, 1, 64), (300, 2, 16)])
+@pytest.mark.parametrize("ne,bs,batch", [(5, 4, 32), (12, 2, 130), (30, 3, 512), (70, 1, 64), (300, 2, 16), (8, 1, 1),
+                                         (9, 7, 4), (17, 1, 5), (33, 5, 8), (32, 3, 17), (40, 1, 31), (1, 9, 3)])
 def test_blocked_float_and_q16(cuda, ne, bs, batch):
     print(f"case blocked ne={ne} bs={bs} batch={batch}", flush=True)
     rng = np.random.default_rng(ne * bs + batch)
@@ -834,7 +835,7 @@ def test_blocked_layer_gradients_without_clearing(cuda, bs, ne, batch, shared, p
     ext = _ext()
     rng = np.random.default_rng(bs * ne + batch)
     nb, nelem = 9, 200
-    first = rng.permutation(nb) * bs + (0 if packed else 2)
+    first = np.arange(nb) * bs if packed else rng.permutation(nb) * bs + 2
     num_nodes = nb * bs + (5 if packed else 7)
     pids = (rng.permutation(nb * ne) * bs).reshape(nb, ne)
     if shared:
