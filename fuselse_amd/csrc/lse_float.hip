@@ -556,7 +556,7 @@ __global__ __launch_bounds__(64) void lse_bwd_flat(const GT* __restrict__ g, con
 // waves share a cache line at each end, and nt loads took 1% more).  A vector
 // that spans two rows, or the matrix's end, goes element by element.  Bound by
 // memory: the gradient of fp32 (8 x 1023, 50257) cut from 8 x 1024 rows moves
-// 3.29 GB in about 525 us; a launch per slice took 6 x 146 + 2 x 65 us, six of
+// 3.29 GB in about 515 us; a launch per slice took 6 x 146 + 2 x 65 us, six of
 // them in the scalar kernel below, whose slice and gradient differ in phase.
 template <typename T, typename GT, typename GR>
 __global__ __launch_bounds__(64) void lse_bwd_flat_shifted(const GT* __restrict__ g, const T* __restrict__ x,
@@ -597,7 +597,11 @@ __global__ __launch_bounds__(64) void lse_bwd_flat_shifted(const GT* __restrict_
             Elem<T>::cvt(*reinterpret_cast<const u32x4_a4*>(xe), v);
         else
             Elem<T>::cvt(*reinterpret_cast<const u32x4_a2*>(xe), v);
-        bwd_vals<VE>(gr_t.coef(row, g0), lv, __builtin_fabsf(lv) < 64.0f, v);
+        // the exact difference, as the scalar kernel below: the one-FMA form cost up
+        // to 10% more error and saved nothing beside the memory
+        const float gv = gr_t.coef(row, g0);
+#pragma unroll
+        for (int k = 0; k < VE; ++k) v[k] = bwd_elem(gv, lv, v[k]);
         add_at<GR::kSel, VE>(v, col, gr_t.target(row), g0);
         Elem<T>::put_vec_buf(ry, (int)threadIdx.x * 16, v);
         return;
