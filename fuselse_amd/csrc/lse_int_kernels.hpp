@@ -504,6 +504,187 @@ __global__ __launch_bounds__(128) void intlse_q10_6_rows_paired(const int16_t* _
     }
 }
 
+// ---------------------------------------------------------------------------
+// Short rows: at most 256 chunks, so a virtual thread has at most one.  A wave
+// takes 8 / VT rows, lane l holding the virtual threads l + 64 * j (j < VT) of
+// each: eight chains a lane, folded side by side.  The eight warp butterflies
+// run as one: at distances 16, 8 and 4 the two halves of the exchange take
+// different chains, so each step halves the chains a lane holds instead of
+// computing every pair on both sides (pair is symmetric, so both sides hold the
+// same value), and a lane ends with the warp result of chain (l >> 2) & 7 of its
+// 32-lane half.  14 pair steps serve 8 / VT rows where each row took 10 in each
+// of four waves, three quarters of them, at 256 columns, of empty virtual
+// threads.  Those and the identity lanes of the last butterfly are constants
+// here (ShortConsts).  Every pair is one of the reference tree's, so the bits
+// are the same.  Bound by memory at 65536 x 256 (67 MB in 10.2 us; 62.5 with a
+// block per row), by the VALU below that.
+// ---------------------------------------------------------------------------
+// The pair ops on unbiased values at compile time.
+constexpr int const_pair(int a, int b, int bits, const int (&tab)[64], bool lut) {
+    const int one = 1 << bits;
+    const int hi = a > b ? a : b, d = a > b ? a - b : b - a;
+    const int sh = (d + one - 1) >> bits;
+    const int m = sh > 30 ? 0 : (one + ((-d) & (one - 1))) >> sh;
+    return hi + m + (lut ? tab[(m >> (bits - 6)) & 63] : 0);
+}
+// id2: a pair of identities, as lanes 8-15 of the last butterfly hold after its
+// first distance; empty: an empty warp's lane after the first two; empty2: a
+// pair of those.
+struct ShortConsts {
+    int id2, empty, empty2;
+};
+constexpr ShortConsts short_consts(int bits, const int (&tab)[64], bool lut) {
+    int k = kQNegInf;
+    for (int i = 0; i < 5; ++i) k = const_pair(k, k, bits, tab, lut);
+    const int id2 = const_pair(kQNegInf, kQNegInf, bits, tab, lut);
+    const int e = const_pair(const_pair(k, kQNegInf, bits, tab, lut), id2, bits, tab, lut);
+    return {id2, e, const_pair(e, e, bits, tab, lut)};
+}
+
+// One distance of the joint butterfly: chains a and b become one value, chain
+// a's pair in the lanes whose bit K is clear, chain b's in the others.
+template <int K, typename TAB, typename PAIR>
+__device__ __forceinline__ int pair_split(int a, int b, const TAB* __restrict__ tab, PAIR pair) {
+    static_assert(K == 16 || K == 8 || K == 4, "row exchanges");
+    if constexpr (K == 16) {
+        const auto s = __builtin_amdgcn_permlane16_swap((uint32_t)a, (uint32_t)b, false, false);
+        return pair((int)s[0], (int)s[1], tab);
+    } else if constexpr (K == 8) {  // row_ror:8 into the upper, the lower eight lanes of each row
+        const int lo = __builtin_amdgcn_update_dpp(a, b, 0x128, 0xF, 0xC, false);
+        const int hi = __builtin_amdgcn_update_dpp(b, a, 0x128, 0xF, 0x3, false);
+        return pair(lo, hi, tab);
+    } else {  // row_shr:4 into the odd, row_shl:4 into the even quads
+        const int lo = __builtin_amdgcn_update_dpp(a, b, 0x114, 0xF, 0xA, false);
+        const int hi = __builtin_amdgcn_update_dpp(b, a, 0x104, 0xF, 0x5, false);
+        return pair(lo, hi, tab);
+    }
+}
+
+__device__ __forceinline__ int hold(int v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
+// EDGE: rows with prefix or suffix elements (N not a multiple of 4 or x off the
+// chunks' alignment).
+template <typename SRC, int ALIGN, int VT, bool EDGE, typename TAB, typename PAIR, typename SETUP>
+__device__ __forceinline__ void tree_short_rows(const typename SRC::T* __restrict__ x, float* __restrict__ out,
+                                                int32_t* __restrict__ acc_out, int64_t B, int64_t N, int64_t block,
+                                                const TAB* __restrict__ tab, PAIR pair, SETUP& setup,
+                                                const ShortConsts kc, float scale) {
+    using T = typename SRC::T;
+    constexpr int R = 8 / VT;
+    constexpr int CB = 4 * (int)sizeof(T);
+    constexpr int kEmpty = kQNegInf ^ SRC::kBias;
+    const int l = threadIdx.x & 63;
+    const int64_t row0 = (block * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * R;
+    const int rows = row0 >= B ? 0 : B - row0 < R ? (int)(B - row0) : R;
+    const T* base = x + (rows ? row0 * N : 0);
+    const int n = (int)N;
+    // the wave's rows as one buffer from the chunk boundary at or before them (no
+    // offset is below base's): a lane past a row's chunks reads the next row or,
+    // past the last, zeros, and drops them
+    const int at0 = EDGE ? (int)(reinterpret_cast<uintptr_t>(base) & (ALIGN - 1)) : 0;
+    const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<char*>(reinterpret_cast<const char*>(base)) - at0, 0,
+        rows ? at0 + rows * n * (int)sizeof(T) : 0, 0x00020000);
+    int pre_n[R], n4[R];
+    T pre[R], suf[R];
+    typename SRC::Raw raw[8];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        pre_n[r] = 0;
+        n4[r] = n / 4;
+        if constexpr (EDGE) {
+            const int mis = (int)(reinterpret_cast<uintptr_t>(base + (int64_t)r * N) & (ALIGN - 1));
+            pre_n[r] = mis ? (ALIGN - mis) / (int)sizeof(T) : 0;
+            if (pre_n[r] > n) pre_n[r] = n;
+            n4[r] = (n - pre_n[r]) / 4;
+            pre[r] = SRC::sload(rb, at0 + (r * n + l) * (int)sizeof(T));
+            suf[r] = SRC::sload(rb, at0 + (r * n + pre_n[r] + 4 * n4[r] + l) * (int)sizeof(T));
+        }
+#pragma unroll
+        for (int j = 0; j < VT; ++j)
+            raw[j * R + r] = SRC::bload(rb, l * CB, at0 + (r * n + pre_n[r]) * (int)sizeof(T) + j * 64 * CB);
+    }
+    setup.finish();
+    int acc[8], q[8][4];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+        SRC::unpack(raw[c], q[c]);
+        acc[c] = q[c][0];
+    }
+    // pairs of the elements past the chunks are computed in every lane and
+    // selected after (held: the compiler would branch around each row's)
+    int edge[R];
+    if constexpr (EDGE) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) edge[r] = hold(pair(SRC::cvt(pre[r]), acc[r], tab));
+#pragma unroll
+        for (int r = 0; r < R; ++r) acc[r] = l < pre_n[r] ? edge[r] : acc[r];
+    }
+#pragma unroll
+    for (int i = 1; i < 4; ++i)
+#pragma unroll
+        for (int c = 0; c < 8; ++c) acc[c] = pair(acc[c], q[c][i], tab);
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+        const int r = c % R;
+        const bool has = l + 64 * (c / R) < n4[r];
+        acc[c] = has ? acc[c] : EDGE && c < R && l < pre_n[r] ? SRC::cvt(pre[r]) : kEmpty;
+    }
+    if constexpr (EDGE) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) edge[r] = hold(pair(acc[r], SRC::cvt(suf[r]), tab));
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int with = l < n4[r] || l < pre_n[r] ? edge[r] : SRC::cvt(suf[r]);
+            acc[r] = l < n - pre_n[r] - 4 * n4[r] ? with : acc[r];
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) acc[c] = pair_split<16>(acc[c], acc[c + 4], tab, pair);
+#pragma unroll
+    for (int c = 0; c < 2; ++c) acc[c] = pair_split<8>(acc[c], acc[c + 2], tab, pair);
+    int v = pair_split<4>(acc[0], acc[1], tab, pair);
+    v = pair(v, __builtin_amdgcn_update_dpp(v, v, 0x4E, 0xF, 0xF, false), tab);  // quad_perm: lane ^ 2
+    v = pair(v, __builtin_amdgcn_update_dpp(v, v, 0xB1, 0xF, 0xF, false), tab);  // lane ^ 1
+    // the last butterfly's lane 2 * j + (l >> 5) of row r, chain (l >> 2) & 7 = j * R + r
+    v = pair(v, kEmpty, tab);
+    v = pair(v, kc.id2 ^ SRC::kBias, tab);
+    v = pair(v, VT == 4 ? exact_xor<16>(v) : kc.empty ^ SRC::kBias, tab);
+    v = pair(v, VT == 4 ? exact_xor<8>(v) : VT == 2 ? exact_xor<16>(v) : kc.empty2 ^ SRC::kBias, tab);
+    const auto h = __builtin_amdgcn_permlane32_swap((uint32_t)v, (uint32_t)v, false, false);
+    v = pair((int)h[0], (int)h[1], tab) ^ SRC::kBias;
+    if (l < 4 * rows && (l & 3) == 0) {
+        const int64_t row = row0 + (l >> 2);
+        out[row] = (float)v * scale;
+        if (acc_out) acc_out[row] = v;
+    }
+}
+
+template <typename SRC, bool USE_LUT, int VT, bool EDGE>
+__global__ __launch_bounds__(256) void intlse_q16_short_rows(const typename SRC::T* __restrict__ x,
+                                                             float* __restrict__ out, int32_t* __restrict__ acc_out,
+                                                             int64_t B, int64_t N, int64_t block0) {
+    __shared__ int lut[64];
+    Q16Setup<USE_LUT> setup{lut, 0};
+    constexpr ShortConsts kc = short_consts(16, kLutQ16, USE_LUT);
+    auto pair = [](int a, int b, const int* t) { return (int)q16_pair<USE_LUT>((uint32_t)a, (uint32_t)b, t); };
+    tree_short_rows<SRC, 16, VT, EDGE>(x, out, acc_out, B, N, block0 + blockIdx.x, lut, pair, setup, kc, kQ16Out);
+}
+
+template <int VT, bool EDGE>
+__global__ __launch_bounds__(256) void intlse_q10_6_short_rows(const int16_t* __restrict__ x, float* __restrict__ out,
+                                                               int32_t* __restrict__ acc_out, int64_t B, int64_t N,
+                                                               int64_t block0) {
+    __shared__ __align__(16) uint8_t gap[388];
+    Q10Setup setup{gap, 0, 0};
+    constexpr ShortConsts kc = short_consts(6, kLutQ10, true);
+    tree_short_rows<SrcI16, 8, VT, EDGE>(x, out, acc_out, B, N, block0 + blockIdx.x, gap, q10_pair, setup, kc,
+                                         kQ10Out);
+}
+
 // Chunks per lane kept in flight ahead of the pair chain.  Every block starts
 // its row at once and issues its first chunks together; a wave whose loads
 // cannot issue yet (its CU's queue is full) also cannot start its chain, so

@@ -240,3 +240,42 @@ def test_rows_of_zero_and_one_elements(cuda, N):
     out, acc = _run(ext.batched_logsumexp_q10_6, qd)
     want, want_acc = O.q10_6_rows(q, base_mod=qd.data_ptr() & 15, raw=True)
     _assert_bits(out, acc, want, want_acc)
+
+
+@pytest.mark.parametrize("N,elem_offset", [(1, 0), (2, 1), (3, 3), (5, 2), (8, 0), (64, 0), (127, 1), (256, 0), (256, 1),
+                                           (259, 0), (260, 0), (260, 2), (512, 0), (515, 3), (516, 0), (1000, 0),
+                                           (1024, 0), (1024, 1), (1027, 0), (1028, 0)])
+@pytest.mark.parametrize("fmt", ["f32", "f32 no lut", "i32", "q10_6"])
+def test_many_short_rows(cuda, N, elem_offset, fmt):
+    """Many rows of at most 256 chunks (several rows per wave) and the first
+    length past them: 1, 2 or 4 virtual threads a lane, whole rows and rows with
+    prefix and suffix elements, rows left over in the last wave, entries at the
+    type's limits and around the identity; the oracle's tree bit for bit."""
+    B = 1027 if N % 4 == 0 and elem_offset == 0 else 4099
+    print(f"case short rows {fmt} N={N} off={elem_offset}", flush=True)
+    rng = np.random.default_rng(N * 5 + elem_offset)
+    x = rng.standard_normal((B, N), dtype=np.float32) * np.float32(2.0)
+    if fmt == "q10_6":
+        a = O.to_q10_6(x)
+        a[0, ::5], a[1, :], a[2, 1::3] = 32767, -32768, -32768
+    elif fmt == "i32":
+        a = np.round(x * np.float32(94548.0)).astype(np.int32)
+        a[0, :], a[1, :], a[2, ::3] = -0x3fffffff, -2**31, -2**31
+        a[3, :] = -0x3fffffff + rng.integers(-2**20, 2**20, N)
+        a[4, :], a[5, ::2] = -0x3fffffff - 1, 2**29
+    else:
+        a = x
+        a[0, :], a[1, :], a[2, ::3] = -1e9, -11356.5, np.inf
+        a[3, :], a[4, 0] = -np.inf, np.nan
+    ext = _ext()
+    fn = {"f32": ext.batched_logsumexp, "f32 no lut": ext.batched_logsumexp_nolut,
+          "i32": ext.batched_logsumexp_q16_i32, "q10_6": ext.batched_logsumexp_q10_6}[fmt]
+    ad = _offset_view(a, cuda, elem_offset) if elem_offset else torch.from_numpy(a).to(cuda)
+    out, acc = _run(fn, ad)
+    if fmt == "q10_6":
+        want, want_acc = O.q10_6_rows(a, base_mod=ad.data_ptr() & 7, raw=True)
+    elif fmt == "i32":
+        want, want_acc = O.q16_gpu_rows(a, base_mod=ad.data_ptr() & 15, raw=True)
+    else:
+        want, want_acc = O.q16_gpu_rows(a, base_mod=ad.data_ptr() & 15, use_lut=fmt == "f32", raw=True)
+    _assert_bits(out, acc, want, want_acc)
