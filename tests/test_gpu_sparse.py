@@ -698,7 +698,7 @@ def _csr_fp64_torch(child, off, cids, lp):
 
 
 @pytest.mark.parametrize("nodes,batch", [(61, 1), (61, 4), (61, 5), (61, 8), (61, 9), (61, 16), (61, 17), (61, 32),
-                                         (61, 33), (32, 3), (33, 16), (61, 63), (61, 64), (61, 65), (61, 127), (61, 128), (61, 129),
+                                         (61, 33), (32, 3), (33, 16), (127, 40), (128, 40), (129, 40), (300, 200), (61, 63), (61, 64), (61, 65), (61, 127), (61, 128), (61, 129),
                                          (61, 256), (61, 510), (40001, 3), (20001, 130), (160003, 1), (40001, 200),
                                          (40001, 132)])
 def test_csr_forward_runs(cuda, nodes, batch):
