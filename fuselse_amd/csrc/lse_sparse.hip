@@ -982,6 +982,25 @@ __global__ __launch_bounds__(64) void block_fwd_narrow(BlockLayout<LOGP> L, cons
     if (ok && b < L.batch) L.node_mars[(L.nids[j] + it - j * L.block_size) * L.batch + b] = res;
 }
 
+// -inf into the rows [j * block_size, (j + 1) * block_size) of each block j that
+// does not write them itself (nids[j] elsewhere): with nids in order from 0 on, no
+// rows at all.  `per` blocks to a wave, at most one a lane.  262144 rows of 512
+// columns, us: in order 1.9, all elsewhere 99; a fill of all rows takes 78.
+__global__ __launch_bounds__(256) void block_clear_rows(float* __restrict__ node_mars, const int64_t* __restrict__ nids,
+                                                        int64_t nblocks, int64_t block_size, int64_t batch, int per,
+                                                        int64_t block0) {
+    const int l = lane_id();
+    const int64_t j0 = ((block0 + blockIdx.x) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * per;
+    const int64_t j = j0 + l;
+    uint64_t elsewhere = __ballot(l < per && j < nblocks && nids[j < nblocks ? j : 0] != j * block_size);
+    const int64_t span = block_size * batch;
+    while (elsewhere) {
+        float* rows = node_mars + (j0 + __builtin_ctzll(elsewhere)) * span;
+        elsewhere &= elsewhere - 1;
+        for (int64_t i = l; i < span; i += 64) rows[i] = -kInf;
+    }
+}
+
 // Q16.16, us, a wave per (parent, 64 columns) -> this: 2048 x 32 parents, 32
 // edges, batch 4 237 -> 20, batch 32 238 -> 109; 1651 x 24 parents, 72 edges,
 // batch 3 345 -> 75; 200 x 16 parents, 100 edges, batch 4 55 -> 9.
@@ -1657,6 +1676,22 @@ extern "C" int fl_sparse_csr_fwd(const float* child, const int64_t* offsets, con
         sparse::launch_csr<true>(L, child, num_nodes, st);
     else
         sparse::launch_csr<false>(L, child, num_nodes, st);
+    return launch_status(name);
+}
+
+extern "C" int fl_sparse_blocked_clear(float* node_mars, const int64_t* nids, int64_t num_nblocks, int64_t block_size,
+                                       int64_t batch, void* stream) {
+    const char* name = "fl_sparse_blocked_clear";
+    FL_CHECK(num_nblocks >= 0 && block_size >= 0 && batch >= 0, "%s: negative size", name);
+    if (num_nblocks == 0 || block_size == 0 || batch == 0) return ok();
+    FL_CHECK(node_mars && nids, "%s: NULL pointer argument", name);
+    // a wave per block up to 16384 waves, then a few blocks each
+    const int64_t share = (num_nblocks + 16383) / 16384;
+    const int per = (int)(share < 64 ? share : 64);
+    for_grid_chunks((num_nblocks + 4 * per - 1) / (4 * per), 256, [&](int64_t b0, int64_t n) {
+        sparse::block_clear_rows<<<dim3((unsigned)n), dim3(256), 0, reinterpret_cast<hipStream_t>(stream)>>>(
+            node_mars, nids, num_nblocks, block_size, batch, per, b0);
+    });
     return launch_status(name);
 }
 

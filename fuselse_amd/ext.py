@@ -497,7 +497,10 @@ def batched_logsumexp_q10_6(input: torch.Tensor, acc_out=None) -> torch.Tensor:
 # ---------------------------------------------------------------------------
 # Sparse probabilistic-circuit sum layers
 # ---------------------------------------------------------------------------
-def _sparse_blocked(node_mars, element_mars, params, nids, cids, pids, block_size, q16, params_are_log):
+def _sparse_blocked(node_mars, element_mars, params, nids, cids, pids, block_size, q16, params_are_log,
+                    written_rows=None):
+    """written_rows: node_mars comes uninitialised, and rows that no block
+    writes are to be -inf (_clear_unwritten); None: they are left alone."""
     # sparse_float_kernel.cu:119-121 / sparse_q16_kernel.cu:320-322
     _check(node_mars.is_cuda, "node_mars must be CUDA")
     _check(element_mars.is_cuda, "element_mars must be CUDA")
@@ -518,6 +521,8 @@ def _sparse_blocked(node_mars, element_mars, params, nids, cids, pids, block_siz
     batch = node_mars.size(1)
     num_nblocks = nids.size(0)
     num_edges = cids.size(1)
+    if written_rows is not None:
+        _clear_unwritten(node_mars, nids, int(block_size), written_rows)
     if batch == 0 or num_nblocks == 0 or block_size == 0:
         return None
     with _on_device(node_mars):
@@ -525,6 +530,22 @@ def _sparse_blocked(node_mars, element_mars, params, nids, cids, pids, block_siz
                   nids.data_ptr(), cids.data_ptr(), pids.data_ptr(), num_nblocks, num_edges, int(block_size), batch,
                   int(q16), int(params_are_log), _stream(node_mars))
     return None
+
+
+def _clear_unwritten(node_mars, nids, block_size, written_rows):
+    """-inf into the rows that this layer's blocks will not write.
+    written_rows: a plan's word that they write the rows [0, written_rows) in
+    order (0: not known).  The plan may be another layer's, or older than a
+    change of nids, so these rows are left out only where this call's own sizes
+    and, on the device, its nids say the same."""
+    if not (written_rows == nids.size(0) * block_size <= node_mars.size(0)):
+        written_rows = 0
+    if written_rows < node_mars.size(0):
+        node_mars[written_rows:].fill_(float("-inf"))
+    if written_rows and node_mars.size(1):
+        with _on_device(node_mars):
+            _lib.call("fl_sparse_blocked_clear", node_mars.data_ptr(), nids.data_ptr(), nids.size(0), block_size,
+                      node_mars.size(1), _stream(node_mars))
 
 
 def sparse_forward_float(node_mars, element_mars, params, nids, cids, pids, block_size, params_are_log=False):
@@ -551,7 +572,8 @@ class BlockedPlan(NamedTuple):
     # no two (block, parent, edge) triples share a parameter: the ranges
     # [pids[j, e], pids[j, e] + block_size) do not overlap
     params_disjoint: bool = False
-    # the blocks write the node rows [0, written_rows) in full (0: not known)
+    # the blocks write the node rows [0, written_rows) in order and in full (0:
+    # not known); a hint that the layer's forward confirms on its own nids
     written_rows: int = 0
 
 

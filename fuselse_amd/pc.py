@@ -71,10 +71,8 @@ class _SparseBlockedLayer(torch.autograd.Function):
         from . import ext
 
         node_mars = torch.empty((num_nodes, element_mars.size(1)), dtype=torch.float32, device=element_mars.device)
-        # rows that no block writes are -inf; a plan knows the leading rows
-        # that blocks write in full
-        node_mars[getattr(plan, "written_rows", 0):].fill_(float("-inf"))
-        ext.sparse_forward_float(node_mars, element_mars, logparams, nids, cids, pids, block_size, params_are_log=True)
+        ext._sparse_blocked(node_mars, element_mars, logparams, nids, cids, pids, block_size, False, True,
+                            written_rows=getattr(plan, "written_rows", 0))
         ctx.save_for_backward(element_mars, logparams, nids, cids, pids, node_mars)
         ctx.block_size = block_size
         ctx.plan = plan
@@ -100,7 +98,7 @@ def sparse_blocked_layer(element_mars, logparams, nids, cids, pids, block_size, 
     logparams: the backward gives the flows of ext.sparse_blocked_backward with
     the upstream gradient as node flows (a term through a row of -inf
     contributes 0).  plan: a cached ext.sparse_blocked_transpose(nids, cids,
-    pids, block_size, element_mars.size(0)) for this layer (these very nids,
-    cids and pids): the backward walks it, and the forward does not clear the
-    rows that it says blocks write."""
+    pids, block_size, element_mars.size(0)) for this layer, which the backward
+    walks.  The forward leaves the rows uncleared that the plan says blocks
+    write, where the nids of this call say so too."""
     return _SparseBlockedLayer.apply(element_mars, logparams, nids, cids, pids, int(block_size), int(num_nodes), plan)

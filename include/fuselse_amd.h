@@ -235,6 +235,16 @@ int fl_sparse_blocked_fwd(float* node_mars, const float* element_mars, const flo
                           int64_t block_size, int64_t batch, int q16, int params_are_log, void* stream);
 
 /* ---------------------------------------------------------------------------
+ * For a caller that hands fl_sparse_blocked_fwd rows it has not initialised:
+ * -inf into the rows [j * block_size, (j + 1) * block_size) of every block j
+ * with nids[j] != j * block_size.  Blocks that lie in order from row 0 on write
+ * these rows in full; then nothing is written here.  node_mars holds at least
+ * num_nblocks * block_size rows.
+ * ------------------------------------------------------------------------- */
+int fl_sparse_blocked_clear(float* node_mars, const int64_t* nids, int64_t num_nblocks, int64_t block_size,
+                            int64_t batch, void* stream);
+
+/* ---------------------------------------------------------------------------
  * Sparse CSR backward ("flows"; the reference has no backward for its sparse
  * kernels).  For out = fl_sparse_csr_fwd(child, offsets, child_ids,
  * logparams) in fp32 and an upstream gradient grad_out [num_nodes, batch]:

@@ -862,3 +862,43 @@ def test_blocked_layer_gradients_without_clearing(cuda, bs, ne, batch, shared, p
             torch.testing.assert_close(dw, gp, rtol=1e-5, atol=1e-5)
         else:
             assert torch.equal(dw, gp)
+
+
+@pytest.mark.parametrize("nb,bs,batch", [(9, 4, 40), (7, 32, 130), (40000, 1, 3), (70001, 2, 1)])
+@pytest.mark.parametrize("other", ["elsewhere", "one block", "in place", "subset", "smaller blocks"])
+def test_blocked_layer_rows_with_another_layers_plan(cuda, nb, bs, batch, other):
+    """A plan says that its blocks write the leading rows, and the layer it is
+    passed with has other nids (all of them, one, or the plan's own tensor changed
+    in place), fewer blocks, or smaller blocks: rows that no block writes are -inf
+    and the others the in-place forward's, in memory that held NaN."""
+    print(f"case blocked rows of another plan nb={nb} bs={bs} batch={batch} {other}", flush=True)
+    from fuselse_amd import pc
+
+    ext = _ext()
+    rng = np.random.default_rng(nb + bs)
+    ne, nelem, num_nodes = 3, 50, 2 * nb * bs + 5
+    nids, cids, pids = _to(cuda, (np.arange(nb) * bs).astype(np.int64), rng.integers(0, nelem, (nb, ne)).astype(np.int64),
+                           (np.arange(nb * ne) * bs).astype(np.int64).reshape(nb, ne))
+    lw = torch.from_numpy(np.log(rng.random(nb * ne * bs) + 1e-3).astype(np.float32)).to(cuda)
+    em = torch.from_numpy(np.log(rng.random((nelem, batch)) + 1e-12).astype(np.float32)).to(cuda)
+    plan = ext.sparse_blocked_transpose(nids, cids, pids, bs, nelem)
+    assert plan.written_rows == nb * bs
+    if other == "elsewhere":
+        nids = nids + nb * bs + 1
+    elif other == "one block":
+        nids = nids.clone()
+        nids[nb // 2] = nb * bs + 3
+    elif other == "in place":
+        nids += 2
+    elif other == "subset":
+        nids, cids, pids = nids[1::2].contiguous(), cids[1::2].contiguous(), pids[1::2].contiguous()
+    else:
+        bs = max(bs // 2, 1)
+        nids = nids + bs
+    want = torch.full((num_nodes, batch), float("-inf"), device=cuda)
+    ext.sparse_forward_float(want, em, lw, nids, cids, pids, bs, params_are_log=True)
+    junk = [torch.full_like(want, float("nan")) for _ in range(3)]
+    del junk
+    with torch.no_grad():
+        got = pc.sparse_blocked_layer(em, lw, nids, cids, pids, bs, num_nodes, plan=plan)
+    assert torch.equal(got, want)
