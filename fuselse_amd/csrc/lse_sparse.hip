@@ -678,7 +678,7 @@ __global__ __launch_bounds__(64) void csr_fwd_kernel(const float* __restrict__ c
     const int64_t nnz = uniform64(off[nodes]);
     const u32x4v rc = words_rsrc(cids + e0, nnz - e0), rl = words_rsrc(logp + e0, nnz - e0);
     const float* child_b0 = child + b0;
-    const uint32_t row_bytes = (uint32_t)batch * 4u;
+    const uint32_t row_bytes = (uint32_t)batch * 4u;  // launch_csr sends larger rows elsewhere
     const int rec = cols_bytes(batch, b0);
     const auto load_meta = [&](const Group& g) {
         return GroupMeta{s_buffer_load4(rc, g.e * 4, 0), s_buffer_load4(rl, g.e * 4, 0)};
@@ -1088,6 +1088,12 @@ static void launch_csr(const CsrLayout& L, const float* child, int64_t nodes, hi
     }
     if (batch <= 64) {
         launch_csr_cols<Q16, 1, 1>(L, child, nodes, run_nodes(nodes), st);
+        return;
+    }
+    // rows of 4 GiB: the stream holds a row's bytes in 32 bits (in 64 the extra
+    // scalar arithmetic per edge took 200000 x 100 Q16.16 from 176.9 to 178.4 us)
+    if (batch >= (int64_t)1 << 30) {
+        launch<Q16>(L, child, L.out, nodes, batch, st);
         return;
     }
     if (batch > 128 && batch % 4 == 0 && (at & 15) == 0 && nodes >= 40000 && !slices_fit(batch)) {

@@ -303,3 +303,24 @@ def test_sparse_blocked_elements_past_4g_bytes(big):
                            params_are_log=True)
     want = O.sparse_q16_blocked(nm0, em_small, logw, nids, cids_small, bs)
     np.testing.assert_array_equal(nmq.cpu().numpy().view(np.int32), want.view(np.int32))
+
+
+@pytest.mark.parametrize("q16", [False, True])
+def test_sparse_csr_rows_of_4_gib(big, q16):
+    """CSR forward with rows of 2^32 bytes (a batch of 2^30), whose size in bytes
+    does not fit 32 bits: one node, its edge to the second of two child rows."""
+    batch = 1 << 30
+    print(f"case large csr batch={batch} q16={q16}", flush=True)
+    child = torch.empty((2, batch), dtype=torch.float32, device=big)
+    child[0] = -3.0
+    child[1] = -1.0
+    off = torch.tensor([0, 1], device=big)
+    cid = torch.ones(1, dtype=torch.int32, device=big)
+    lp = torch.full((1,), -0.5, device=big)
+    out = _ext().sparse_csr_forward(child, off, cid, lp, q16=q16)
+    # one edge: the logit itself, in Q16.16 rounded to 2^-16 in base 2; in fp32
+    # the exponent 1.5 * log2(e) = 2.16 is rounded (half an ulp: 2^-23), and so are
+    # the logarithm of the sum next to 1 and the result (2^-24 each): 2^-22 in all
+    tol = 2.0 ** -16 if q16 else 2.0 ** -22
+    assert out.shape == (1, batch)
+    assert float(out.min()) >= -1.5 - tol and float(out.max()) <= -1.5 + tol
