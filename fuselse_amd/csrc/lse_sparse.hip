@@ -1202,7 +1202,9 @@ __global__ __launch_bounds__(64) void csr_bwd_kernel(const float* __restrict__ c
     const int64_t at = csc_off[n0 + (l < nn ? l : nn)];
     const int64_t nnz = uniform64(csc_off[children]);
     const int64_t e0 = uniform64(at);
-    const bool streamed = bcast64(at, nn) - e0 <= kRunEdges;
+    // a layer without any edge goes the other way too: the stream reads the weight
+    // of edge 0 for a masked one
+    const bool streamed = nnz > 0 && bcast64(at, nn) - e0 <= kRunEdges;
     const int64_t b0 = tile * 64 * P;
     const int rec = cols_bytes(batch, b0);
     const float* child_b0 = child + b0;

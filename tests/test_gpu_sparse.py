@@ -902,3 +902,26 @@ def test_blocked_layer_rows_with_another_layers_plan(cuda, nb, bs, batch, other)
     with torch.no_grad():
         got = pc.sparse_blocked_layer(em, lw, nids, cids, pids, bs, num_nodes, plan=plan)
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("batch", [3, 40, 100, 128, 200])
+@pytest.mark.parametrize("entry", ["fl_sparse_csr_bwd", "fl_sparse_csr_bwd_ws"])
+def test_csr_backward_of_a_layer_without_edges(cuda, batch, entry):
+    """The C entries on a layer whose children have no edge: every gradient of a
+    child is 0, and no edge's gradient is written."""
+    print(f"case csr bwd without edges batch={batch} {entry}", flush=True)
+    from fuselse_amd import _lib
+
+    children, nodes = 70, 5
+    child = torch.zeros(children, batch, device=cuda)
+    out = torch.full((nodes, batch), float("-inf"), device=cuda)
+    gout = torch.ones(nodes, batch, device=cuda)
+    off = torch.zeros(children + 1, dtype=torch.int64, device=cuda)
+    # the entries refuse NULL, so the edge arrays have one element that is no edge
+    ids = torch.full((1,), 1 << 30, dtype=torch.int32, device=cuda)
+    lp = torch.full((1,), float("nan"), device=cuda)
+    gc, gl = torch.full_like(child, float("nan")), torch.full_like(lp, 7.0)
+    args = [t.data_ptr() for t in (child, out, gout, lp, off, ids, ids, gc, gl)]
+    tail = [children, batch] if entry == "fl_sparse_csr_bwd" else [children, 0, batch, None, 0]
+    _lib.call(entry, *args, *tail, torch.cuda.current_stream().cuda_stream)
+    assert (gc == 0).all() and float(gl) == 7.0
