@@ -1627,12 +1627,20 @@ extern "C" int fl_sparse_csr_bwd(const float* child, const float* out, const flo
 // us in them against 2099 in whole rows) of layers of at least 64000 (child,
 // column tile) pairs: it pays two more launches (us, workspace / none: 2000 x
 // 512 20 / 13, 12000 x 512 58 / 53, 20000 x 512 89 / 97, 50000 x 512 227 / 265).
+// It grows with the edges, so above 256 MB it is taken only up to the size of
+// the gradient of the children that it serves (about 100 edges a child); past
+// that, whole rows (20000 children of 200 edges, batch 512, 80 MB: 1887 us
+// against 2200; 16000 of 1000, 320 MB: 9156 against 9204).
+constexpr size_t kBwdWorkspaceSmall = (size_t)256 << 20;
+
 extern "C" size_t fl_sparse_csr_bwd_workspace_bytes(int64_t num_children, int64_t nnz, int64_t batch) {
     if (nnz <= 0 || batch <= 0) return 0;
     const int64_t cols = sparse::bwd_tile_cols(batch);
     const int64_t tiles = (batch + cols - 1) / cols;
     if (tiles < 2 || num_children * tiles < 64000 || !sparse::slices_fit(batch)) return 0;
-    return (size_t)nnz * (size_t)(tiles + 1) * sizeof(float);
+    const size_t need = (size_t)nnz * (size_t)(tiles + 1) * sizeof(float);
+    const size_t rows = (size_t)num_children * (size_t)batch * sizeof(float);
+    return need <= kBwdWorkspaceSmall || need <= rows ? need : 0;
 }
 
 extern "C" int fl_sparse_csr_bwd_ws(const float* child, const float* out, const float* grad_out,

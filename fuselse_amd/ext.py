@@ -842,10 +842,17 @@ def _launch_csr_bwd(child, out, grad_out, logparams, csc_off, csc_edge, csc_node
     nnz = csc_edge.numel()
     with _on_device(child):
         nbytes = _lib.load().fl_sparse_csr_bwd_workspace_bytes(num_children, nnz, batch)
-        # the weights and sums in the walk's order; stream-ordered reuse by
-        # torch's caching allocator keeps it valid until the kernels have run
-        ws = torch.empty(nbytes, dtype=torch.uint8, device=child.device) if nbytes else None
-        _lib.call("fl_sparse_csr_bwd_ws", child.data_ptr(), out.data_ptr(), grad_out.data_ptr(), logparams.data_ptr(),
-                  csc_off.data_ptr(), csc_edge.data_ptr(), csc_node.data_ptr(), grad_child.data_ptr(),
-                  grad_logp.data_ptr(), num_children, nnz, batch, ws.data_ptr() if ws is not None else None, nbytes,
-                  _stream(child))
+        ws = None
+        if nbytes:
+            # the weights and sums in the walk's order; stream-ordered reuse by
+            # torch's caching allocator keeps it valid until the kernels have run
+            try:
+                ws = torch.empty(nbytes, dtype=torch.uint8, device=child.device)
+            except torch.cuda.OutOfMemoryError:
+                pass  # the entry without a workspace needs no memory of its own
+        args = (child.data_ptr(), out.data_ptr(), grad_out.data_ptr(), logparams.data_ptr(), csc_off.data_ptr(),
+                csc_edge.data_ptr(), csc_node.data_ptr(), grad_child.data_ptr(), grad_logp.data_ptr(), num_children)
+        if ws is None:
+            _lib.call("fl_sparse_csr_bwd", *args, batch, _stream(child))
+        else:
+            _lib.call("fl_sparse_csr_bwd_ws", *args, nnz, batch, ws.data_ptr(), nbytes, _stream(child))

@@ -269,7 +269,8 @@ int fl_sparse_csr_bwd(const float* child, const float* out, const float* grad_ou
 /* ---------------------------------------------------------------------------
  * The same with a caller workspace of
  * fl_sparse_csr_bwd_workspace_bytes(num_children, nnz, batch) bytes (0: none needed, NULL
- * will do), 4-byte aligned, any contents: the edges' weights and batch sums
+ * will do; at most 256 MB or the size of grad_child, whichever is larger; a caller
+ * that cannot spare it calls fl_sparse_csr_bwd), 4-byte aligned, any contents: the edges' weights and batch sums
  * then pass through it in the walk's order instead of being gathered and
  * scattered once per column tile, and the tiles go one after the other over
  * all children.  nnz is csc_offsets[num_children].  Deterministic; the sum of

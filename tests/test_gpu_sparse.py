@@ -925,3 +925,34 @@ def test_csr_backward_of_a_layer_without_edges(cuda, batch, entry):
     tail = [children, batch] if entry == "fl_sparse_csr_bwd" else [children, 0, batch, None, 0]
     _lib.call(entry, *args, *tail, torch.cuda.current_stream().cuda_stream)
     assert (gc == 0).all() and float(gl) == 7.0
+
+
+def test_csr_backward_without_memory_for_the_workspace(cuda, monkeypatch):
+    """Where the workspace cannot be allocated the backward takes the entry that
+    needs none, and its bits."""
+    print("case csr bwd no workspace memory", flush=True)
+    from fuselse_amd import _lib
+
+    rng = np.random.default_rng(4)
+    nodes, children, batch = 3000, 33000, 256
+    off, cids, lp = _csr(rng, nodes, children, fanin=np.full(nodes, 50))
+    ch, offd, cid, lpd = _to(cuda, np.log(rng.random((children, batch)) + 1e-12).astype(np.float32), off, cids, lp)
+    ext = _ext()
+    assert _lib.load().fl_sparse_csr_bwd_workspace_bytes(children, cid.numel(), batch) > 0
+    out = ext.sparse_csr_forward(ch, offd, cid, lpd)
+    gout = torch.from_numpy(rng.standard_normal((nodes, batch)).astype(np.float32)).to(cuda)
+    csc = ext.sparse_csr_transpose(offd, cid, children)
+    want_c, want_l = torch.empty_like(ch), torch.empty_like(lpd)
+    _lib.call("fl_sparse_csr_bwd", *(t.data_ptr() for t in (ch, out, gout, lpd, *csc, want_c, want_l)), children, batch,
+              torch.cuda.current_stream().cuda_stream)
+    empty = torch.empty
+
+    def no_bytes(*args, **kwargs):
+        if kwargs.get("dtype") == torch.uint8:
+            raise torch.cuda.OutOfMemoryError("no memory for a workspace")
+        return empty(*args, **kwargs)
+
+    with monkeypatch.context() as m:
+        m.setattr(torch, "empty", no_bytes)
+        gc, gl = ext.sparse_csr_backward(ch, out, gout, offd, cid, lpd, csc)
+    assert torch.equal(gc, want_c) and torch.equal(gl, want_l)
