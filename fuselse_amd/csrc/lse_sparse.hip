@@ -640,7 +640,7 @@ __device__ __forceinline__ int64_t xcd_unit(int64_t u, int64_t total) {
     return g + 8 * kXcdRuns > total ? u : g + (i & 7) * kXcdRuns + (i >> 3);
 }
 
-template <bool Q16, int VW, int P>
+template <bool Q16, int VW, int P, bool SHORT>
 __global__ __launch_bounds__(64) void csr_fwd_kernel(const float* __restrict__ child, const int64_t* __restrict__ off,
                                                      const int32_t* __restrict__ cids, const float* __restrict__ logp,
                                                      float* __restrict__ out, int64_t batch, int64_t nodes,
@@ -701,13 +701,27 @@ __global__ __launch_bounds__(64) void csr_fwd_kernel(const float* __restrict__ c
     // ga, gb: the groups whose rows are in va, vb; the second one's ids (mb)
     // are loaded while the first one's rows are awaited.  Groups past the run
     // load nothing and store nothing: with an exit after the first fold the
-    // compiler sinks the ids' loads below it, next to their use.
+    // compiler sinks the ids' loads below it, next to their use.  Runs of one or
+    // two groups leave before the loop instead, without its waits for the ids of
+    // groups past them (8000 nodes, batch 128, 2 edges 7.9 -> 6.1 us, 5 edges 7.8 ->
+    // 7.1); kernels for longer runs (SHORT false) do without the test, which took
+    // 20000 nodes, batch 256, 5 edges, two nodes a run from 20.6 to 21.2.
     float va[G][P], vb[G][P];
     Group ga = {0, 0, run.start(1), 1, run.start(1)};
     GroupMeta ma = load_meta(ga);
     load_rows(va, ma, ga);
     Group gb = run.next(ga);
+    if (SHORT && gb.node >= nn) {
+        fold(va, ma, ga);
+        return;
+    }
     GroupMeta mb = load_meta(gb);
+    if (SHORT && run.next(gb).node >= nn) {
+        load_rows(vb, mb, gb);
+        fold(va, ma, ga);
+        fold(vb, mb, gb);
+        return;
+    }
     while (true) {
         load_rows(vb, mb, gb);
         const Group gc = run.next(gb);
@@ -1048,12 +1062,20 @@ static int run_nodes(int64_t pairs) {
     return pairs < 40000 ? 1 : pairs < 160000 ? 2 : pairs < 1000000 ? 4 : 8;
 }
 
+// brief: most runs have one or two groups.
 template <bool Q16, int VW, int P>
-static void launch_csr_cols(const CsrLayout& L, const float* child, int64_t nodes, int npw, hipStream_t st) {
+static void launch_csr_cols(const CsrLayout& L, const float* child, int64_t nodes, int npw, bool brief,
+                            hipStream_t st) {
     const int64_t tiles = (L.batch + 64 * P - 1) / (64 * P);
     for_grid_chunks((nodes + npw - 1) / npw * tiles, 64, [&](int64_t u0, int64_t n) {
-        csr_fwd_kernel<Q16, VW, P><<<dim3((unsigned)n), dim3(64), 0, st>>>(child, L.offsets, L.cids, L.logp, L.out,
-                                                                          L.batch, nodes, npw, u0);
+        const auto go = [&](auto kernel) {
+            kernel<<<dim3((unsigned)n), dim3(64), 0, st>>>(child, L.offsets, L.cids, L.logp, L.out, L.batch, nodes, npw,
+                                                           u0);
+        };
+        if (brief)
+            go(csr_fwd_kernel<Q16, VW, P, true>);
+        else
+            go(csr_fwd_kernel<Q16, VW, P, false>);
     });
 }
 
@@ -1062,15 +1084,29 @@ static void launch_csr_cols(const CsrLayout& L, const float* child, int64_t node
 // and at most a tenth of the last slice's lanes idle over all of them.
 static bool slices_fit(int64_t batch) { return batch % 32 == 0 && batch * 10 >= (batch + 127) / 128 * 128 * 9; }
 
+// Whether 256-column tiles leave no more lanes idle than 128-column ones.
+static bool wide_tiles_fit(int64_t batch) { return (batch + 127) / 128 == 2 * ((batch + 255) / 256); }
+
 // Up to 32 columns: several nodes per wave (csr_fwd_narrow).  Columns per lane
 // above: 1 up to a batch of 64, else 2 (200000 nodes, fp32, us, 1 / 2
 // columns a lane: batch 64 99 / 105, 100 182 / 142, 512 515 / 497; 4 columns
-// 140, 152, 519).  Large layers whose rows do not cut into such slices take
-// tiles of 256 columns, in fp32 through the stream (us, 128 / 256 columns: 1M x
-// 200 1304 / 1143, 500000 x 500 1482 / 1349, 50000 x 130 76 / 66, but 20000 x
-// 300 58 / 66), in Q16.16 with a wave per node and tile (200000 x 500: 618 in
-// slices, 595 through the stream, whose 8 chains of 4 columns leave it four
-// waves per SIMD).
+// 140, 152, 519).  Large layers whose rows do not cut into such slices but fit
+// tiles of 256 columns take these, in fp32 through the stream (us, 128 / 256
+// columns: 1M x 200 1304 / 1143, 500000 x 500 1482 / 1349, 200000 x 130, 16 edges
+// a node, 401 / 297; 100000 x 300, which does not fit, 212 / 231), in Q16.16 with
+// a wave per node and tile (200000 x 500: 618 in slices, 595 through the stream,
+// whose 8 chains of 4 columns leave it four waves per SIMD).
+//
+// From some thousand (node, 128-column tile) pairs on, the waves are more than
+// the GPU holds at once, and a short node is a wave's fixed cost; up to 40000,
+// where longer runs begin, half as many waves of 256 columns, or where these do
+// not fit and in Q16.16 of two nodes, take less.  Below, the longest node's chain
+// is the time, and a wave for it alone is fastest.  us at 2 / 5 / 16 / power-law
+// edges a node, one node and 128 columns a wave -> this: 8000 nodes, batch 512,
+// fp32 15.0 / 18.8 / 31.0 / 40.3 -> 10.0 / 15.9 / 27.6 / 43.4, Q16.16 15.9 / 20.2 /
+// 36.8 / 60.7 -> 12.7 / 19.2 / 34.5 / 61.3; 8000 x 300, fp32 12.5 / 15.5 / 24.3 /
+// 35.6 -> 9.9 / 14.9 / 23.5 / 37.2; 2000 x 256 4.7 / 5.3 / 7.3 / 22.4 against 4.0 /
+// 4.6 / 6.1 / 26.4 with 256 columns.
 template <bool Q16>
 static void launch_csr(const CsrLayout& L, const float* child, int64_t nodes, hipStream_t st) {
     const uintptr_t at = reinterpret_cast<uintptr_t>(child) | reinterpret_cast<uintptr_t>(L.out);
@@ -1087,7 +1123,7 @@ static void launch_csr(const CsrLayout& L, const float* child, int64_t nodes, hi
         return;
     }
     if (batch <= 64) {
-        launch_csr_cols<Q16, 1, 1>(L, child, nodes, run_nodes(nodes), st);
+        launch_csr_cols<Q16, 1, 1>(L, child, nodes, run_nodes(nodes), nodes < 40000, st);
         return;
     }
     // rows of 4 GiB: the stream holds a row's bytes in 32 bits (in 64 the extra
@@ -1096,18 +1132,28 @@ static void launch_csr(const CsrLayout& L, const float* child, int64_t nodes, hi
         launch<Q16>(L, child, L.out, nodes, batch, st);
         return;
     }
-    if (batch > 128 && batch % 4 == 0 && (at & 15) == 0 && nodes >= 40000 && !slices_fit(batch)) {
-        if constexpr (Q16)
-            launch_cols<true, 4, 4>(L, child, nodes, batch, st);
+    const int64_t pairs = nodes * ((batch + 127) / 128);
+    const bool brief = pairs < 40000;
+    const bool wide = batch > 128 && wide_tiles_fit(batch), slices = slices_fit(batch);
+    const bool large = wide && !slices && nodes >= 40000;
+    if constexpr (Q16) {
+        if (large) {
+            launch<true>(L, child, L.out, nodes, batch, st);
+            return;
+        }
+    } else if (large || (wide && pairs >= 12000 && (brief || (!slices && batch <= 256)))) {
+        const int npw = large ? 2 : 1;
+        if (batch % 4 == 0 && (at & 15) == 0)
+            launch_csr_cols<false, 4, 4>(L, child, nodes, npw, !large, st);
         else
-            launch_csr_cols<false, 4, 4>(L, child, nodes, batch <= 256 ? 2 : 1, st);
+            launch_csr_cols<false, 1, 4>(L, child, nodes, npw, !large, st);
         return;
     }
-    const int npw = run_nodes(nodes * ((batch + 127) / 128));
+    const int npw = batch > 128 && brief && pairs >= (Q16 ? 12000 : 6000) ? 2 : run_nodes(pairs);
     if (batch % 2 == 0 && (at & 7) == 0)
-        launch_csr_cols<Q16, 2, 2>(L, child, nodes, npw, st);
+        launch_csr_cols<Q16, 2, 2>(L, child, nodes, npw, brief, st);
     else
-        launch_csr_cols<Q16, 1, 2>(L, child, nodes, npw, st);
+        launch_csr_cols<Q16, 1, 2>(L, child, nodes, npw, brief, st);
 }
 
 // ---------------------------------------------------------------------------

@@ -956,3 +956,42 @@ def test_csr_backward_without_memory_for_the_workspace(cuda, monkeypatch):
         m.setattr(torch, "empty", no_bytes)
         gc, gl = ext.sparse_csr_backward(ch, out, gout, offd, cid, lpd, csc)
     assert torch.equal(gc, want_c) and torch.equal(gl, want_l)
+
+
+# (nodes, batch) -> columns of a tile, nodes of a run in fp32 / in Q16.16
+RUN_CASES = [
+    (500, 33), (500, 130),               # 64, 128: one / one
+    (2003, 385), (4001, 260),            # 128, odd and even rows: two / one, two / two
+    (6001, 132), (6001, 130),            # 256 in fp32, aligned and odd rows: one / two
+    (3001, 512), (20001, 190),           # 256 in fp32: one / two
+    (40001, 33), (40001, 96),            # 64, 128: two / two
+    (40001, 140), (40001, 131),          # 256: two / a wave per node and tile
+    (160003, 33), (40001, 512),          # 64, 128: four / four
+    (1000003, 40),                       # 64: eight / eight
+]
+
+
+@pytest.mark.parametrize("nodes,batch", RUN_CASES)
+def test_csr_forward_run_lengths(cuda, nodes, batch):
+    """The streamed forward at every tile width and run length: runs that are one
+    or two groups of edges, runs of more, the last run cut short, and empty nodes
+    at a run's start, middle and end (every place modulo 8 holds some)."""
+    print(f"case csr run lengths {nodes}x{batch}", flush=True)
+    rng = np.random.default_rng(nodes + batch)
+    fan = rng.choice([0, 0, 1, 2, 3, 4, 5, 8, 9, 13], nodes)
+    fan[:4], fan[-3:] = [0, 256, 0, 40], [0, 5, 0]
+    fan[nodes // 2:nodes // 2 + 16] = 0
+    off, cids, lp = _csr(rng, nodes, 300, fanin=fan)
+    child = np.log(rng.random((300, batch)) + 1e-12).astype(np.float32)
+    ch, offd, cid, lpd = _to(cuda, child, off, cids, lp)
+    ext = _ext()
+    got = ext.sparse_csr_forward(ch, offd, cid, lpd)
+    want = _csr_fp64_torch(ch, offd, cid, lpd)[0]
+    assert torch.equal(torch.isneginf(got), (offd.diff() == 0)[:, None].expand_as(got))
+    torch.testing.assert_close(got.double(), want, rtol=1e-5, atol=1e-6)
+    gq = ext.sparse_csr_forward(ch, offd, cid, lpd, q16=True)
+    part = min(nodes, 20000)  # the first and the last nodes, bit for bit
+    for a, b in ((0, part), (nodes - part, nodes)):
+        e = slice(off[a], off[b])
+        wq = O.sparse_q16_csr(child, off[a:b + 1] - off[a], cids[e], lp[e])
+        np.testing.assert_array_equal(gq[a:b].cpu().numpy().view(np.int32), wq.view(np.int32))
