@@ -1107,12 +1107,18 @@ static bool wide_tiles_fit(int64_t batch) { return (batch + 127) / 128 == 2 * ((
 // 36.8 / 60.7 -> 12.7 / 19.2 / 34.5 / 61.3; 8000 x 300, fp32 12.5 / 15.5 / 24.3 /
 // 35.6 -> 9.9 / 14.9 / 23.5 / 37.2; 2000 x 256 4.7 / 5.3 / 7.3 / 22.4 against 4.0 /
 // 4.6 / 6.1 / 26.4 with 256 columns.
+//
+// Up to 4 columns, 4 lanes a node; of fewer than 4000 nodes 8, as fan-ins past
+// kOwnEdges are then the time, and 16 nodes' worth of them queue in one wave (us,
+// 4 / 8 lanes, batch 4: 1000 nodes of 40 edges, fp32 14.3 / 10.7, Q16.16 21.1 /
+// 12.2; 4000 nodes of 16 edges 4.3 / 4.4, 4.8 / 5.0; power law, 1000 nodes 8.8 /
+// 9.3, 13.0 / 12.1).
 template <bool Q16>
 static void launch_csr(const CsrLayout& L, const float* child, int64_t nodes, hipStream_t st) {
     const uintptr_t at = reinterpret_cast<uintptr_t>(child) | reinterpret_cast<uintptr_t>(L.out);
     const int64_t batch = L.batch;
     if (batch <= kNarrowBatch) {
-        if (batch <= 4)
+        if (batch <= 4 && nodes >= 4000)
             launch_csr_narrow<Q16, 4>(L, child, nodes, st);
         else if (batch <= 8)
             launch_csr_narrow<Q16, 8>(L, child, nodes, st);

@@ -995,3 +995,20 @@ def test_csr_forward_run_lengths(cuda, nodes, batch):
         e = slice(off[a], off[b])
         wq = O.sparse_q16_csr(child, off[a:b + 1] - off[a], cids[e], lp[e])
         np.testing.assert_array_equal(gq[a:b].cpu().numpy().view(np.int32), wq.view(np.int32))
+
+
+@pytest.mark.parametrize("nodes", [1, 9, 300, 3999, 4000, 4003])
+@pytest.mark.parametrize("batch", [1, 3, 4])
+def test_csr_forward_few_columns(cuda, nodes, batch):
+    """Up to 4 columns on either side of the layer size that takes 8 lanes a node:
+    fan-ins a lane group folds by itself and ones that a wave shares."""
+    print(f"case csr few columns {nodes}x{batch}", flush=True)
+    rng = np.random.default_rng(nodes + batch)
+    off, cids, lp = _csr(rng, nodes, 300, fanin=rng.choice([0, 1, 3, 4, 8, 17, 32, 33, 40, 65, 200], nodes))
+    child = np.log(rng.random((300, batch)) + 1e-12).astype(np.float32)
+    ch, offd, cid, lpd = _to(cuda, child, off, cids, lp)
+    ext = _ext()
+    got = ext.sparse_csr_forward(ch, offd, cid, lpd).cpu().numpy()
+    np.testing.assert_allclose(got, O.sparse_csr_fp64(child, off, cids, lp), rtol=1e-5, atol=1e-6)
+    gq = ext.sparse_csr_forward(ch, offd, cid, lpd, q16=True).cpu().numpy()
+    np.testing.assert_array_equal(gq.view(np.int32), O.sparse_q16_csr(child, off, cids, lp).view(np.int32))
