@@ -1234,7 +1234,10 @@ __global__ __launch_bounds__(256) void csr_bwd_sums(const float* __restrict__ pa
     glogp[edges[k]] = s;
 }
 
-template <bool DIRECT, int VW, int P>
+// SHORT: most runs have one or two groups, which leave before the loop, as in
+// csr_fwd_kernel (20000 children, batch 64, us at 2 / 5 / 16 edges a child 20.4 /
+// 22.7 / 38.5 -> 16.3 / 19.7 / 39.6).
+template <bool DIRECT, int VW, int P, bool SHORT>
 __global__ __launch_bounds__(64) void csr_bwd_kernel(const float* __restrict__ child, const float* __restrict__ out,
                                                      const float* __restrict__ gout, const float* __restrict__ logp,
                                                      const int64_t* __restrict__ csc_off,
@@ -1337,6 +1340,12 @@ __global__ __launch_bounds__(64) void csr_bwd_kernel(const float* __restrict__ c
         load_rows(va, ma, ga);
         Group gb = run.next(ga);
         Meta mb = load_meta(gb);
+        if (SHORT && run.next(gb).node >= nn) {
+            load_rows(vb, mb, gb);
+            fold(va, ma, ga);
+            fold(vb, mb, gb);
+            return;
+        }
         while (true) {
             load_rows(vb, mb, gb);
             const Group gc = run.next(gb);
@@ -1487,8 +1496,14 @@ static void launch_csr_bwd_cols(const float* child, const float* out, const floa
     const int npw = run_nodes(DIRECT ? children : children * tiles);
     const int64_t runs = (children + npw - 1) / npw;
     for_grid_chunks(DIRECT ? runs : runs * tiles, 64, [&](int64_t u0, int64_t n) {
-        csr_bwd_kernel<DIRECT, VW, P><<<dim3((unsigned)n), dim3(64), 0, st>>>(
-            child, out, gout, logp, off, edge, node, gchild, glogp, children, batch, npw, tiles, u0);
+        const auto go = [&](auto kernel) {
+            kernel<<<dim3((unsigned)n), dim3(64), 0, st>>>(child, out, gout, logp, off, edge, node, gchild, glogp,
+                                                           children, batch, npw, tiles, u0);
+        };
+        if (DIRECT && npw == 1)
+            go(csr_bwd_kernel<DIRECT, VW, P, DIRECT>);
+        else
+            go(csr_bwd_kernel<DIRECT, VW, P, false>);
     });
 }
 
@@ -1679,6 +1694,9 @@ extern "C" int fl_sparse_csr_bwd(const float* child, const float* out, const flo
 // us in them against 2099 in whole rows) of layers of at least 64000 (child,
 // column tile) pairs: it pays two more launches (us, workspace / none: 2000 x
 // 512 20 / 13, 12000 x 512 58 / 53, 20000 x 512 89 / 97, 50000 x 512 227 / 265).
+// And of at least 5 edges a child, as each tile of a child is a walk of its own
+// (100000 x 384 at 2 / 4 / 5 / 8 edges a child 192 / 241 / 273 / 391, none 132 / 229 /
+// 278 / 412).
 // It grows with the edges, so above 256 MB it is taken only up to the size of
 // the gradient of the children that it serves (about 100 edges a child); past
 // that, whole rows (20000 children of 200 edges, batch 512, 80 MB: 1887 us
@@ -1689,7 +1707,7 @@ extern "C" size_t fl_sparse_csr_bwd_workspace_bytes(int64_t num_children, int64_
     if (nnz <= 0 || batch <= 0) return 0;
     const int64_t cols = sparse::bwd_tile_cols(batch);
     const int64_t tiles = (batch + cols - 1) / cols;
-    if (tiles < 2 || num_children * tiles < 64000 || !sparse::slices_fit(batch)) return 0;
+    if (tiles < 2 || num_children * tiles < 64000 || nnz / 5 < num_children || !sparse::slices_fit(batch)) return 0;
     const size_t need = (size_t)nnz * (size_t)(tiles + 1) * sizeof(float);
     const size_t rows = (size_t)num_children * (size_t)batch * sizeof(float);
     return need <= kBwdWorkspaceSmall || need <= rows ? need : 0;

@@ -216,8 +216,8 @@ def test_shim_rejects_operands_on_another_gpu(fn, make, msg):
 def test_csr_backward_workspace_is_bounded():
     """fl_sparse_csr_bwd_workspace_bytes: a float per edge and column tile and one
     more per edge, up to 256 MB or the size of the children's gradient; 0 (whole
-    rows, no workspace) above, for few children and for rows that do not cut into
-    128-column slices."""
+    rows, no workspace) above, for few children, for fewer than 5 edges a child and
+    for rows that do not cut into 128-column slices."""
     ws = _lib.load().fl_sparse_csr_bwd_workspace_bytes
     assert ws(1_000_000, 8_000_000, 512) == 8_000_000 * 5 * 4
     assert ws(20_000, 4_000_000, 512) == 4_000_000 * 5 * 4       # 200 edges a child, 80 MB
@@ -227,3 +227,4 @@ def test_csr_backward_workspace_is_bounded():
     assert ws(1_000_000, 102_400_001, 512) == 0
     assert ws(1_000, 2 ** 31 - 1, 2 ** 16) == 0
     assert ws(10_000, 80_000, 512) == 0 and ws(1_000_000, 8_000_000, 400) == 0 and ws(1_000_000, 8_000_000, 128) == 0
+    assert ws(100_000, 500_000, 512) == 500_000 * 5 * 4 and ws(100_000, 499_999, 512) == 0

@@ -935,7 +935,7 @@ def test_csr_backward_without_memory_for_the_workspace(cuda, monkeypatch):
 
     rng = np.random.default_rng(4)
     nodes, children, batch = 3000, 33000, 256
-    off, cids, lp = _csr(rng, nodes, children, fanin=np.full(nodes, 50))
+    off, cids, lp = _csr(rng, nodes, children, fanin=np.full(nodes, 60))
     ch, offd, cid, lpd = _to(cuda, np.log(rng.random((children, batch)) + 1e-12).astype(np.float32), off, cids, lp)
     ext = _ext()
     assert _lib.load().fl_sparse_csr_bwd_workspace_bytes(children, cid.numel(), batch) > 0
@@ -1012,3 +1012,37 @@ def test_csr_forward_few_columns(cuda, nodes, batch):
     np.testing.assert_allclose(got, O.sparse_csr_fp64(child, off, cids, lp), rtol=1e-5, atol=1e-6)
     gq = ext.sparse_csr_forward(ch, offd, cid, lpd, q16=True).cpu().numpy()
     np.testing.assert_array_equal(gq.view(np.int32), O.sparse_q16_csr(child, off, cids, lp).view(np.int32))
+
+
+@pytest.mark.parametrize("children,batch", [(61, 33), (39999, 40), (40003, 64), (39999, 65), (40003, 128), (160003, 33),
+                                            (22001, 512), (60000, 256), (41000, 512)])
+@pytest.mark.parametrize("edges", [2, 5])
+def test_csr_backward_run_lengths(cuda, children, batch, edges):
+    """The streamed backward at every run length: one, two and four children with
+    weights and sums by edge id, two and four through the workspace (from 5 edges a
+    child), runs of one or two groups and longer ones, children without edges at a
+    run's start, middle and end, and parents of probability 0 (-inf), through which
+    nothing flows.  A sum's error is bounded by 1e-5 of its terms' magnitudes."""
+    print(f"case csr bwd run lengths {children}x{batch} edges={edges}", flush=True)
+    rng = np.random.default_rng(children + batch)
+    nodes = 1000
+    fan = np.full(nodes, children * edges // nodes + 1)
+    off, cids, lp = _csr(rng, nodes, children, fanin=fan)
+    cids[cids % 11 == 3] = children // 2            # some children without edges, one with many
+    cids[:8] = [0, 1, 1, children - 2, children - 2, children - 2, children // 3, children // 3]
+    cids[cids == children - 1] = 5
+    lp[off[7]:off[8]] = -np.inf                      # a parent of probability 0
+    ch, offd, cid, lpd = _to(cuda, np.log(rng.random((children, batch)) + 1e-12).astype(np.float32), off, cids, lp)
+    ext = _ext()
+    out = ext.sparse_csr_forward(ch, offd, cid, lpd)
+    gout = torch.from_numpy(rng.standard_normal((nodes, batch)).astype(np.float32)).to(cuda)
+    gc, gl = ext.sparse_csr_backward(ch, out, gout, offd, cid, lpd)
+    out64, parent, t = _csr_fp64_torch(ch, offd, cid, lpd)  # NaN for the parent of probability 0
+    dead = torch.isneginf(out)
+    assert dead[7].all() and not dead[8:].any()
+    term = torch.where(dead[parent], 0.0, torch.exp(t - out64[parent]) * gout.double()[parent])
+    assert ((gl.double() - term.sum(1)).abs() <= 1e-5 * term.abs().sum(1) + 1e-30).all()
+    want = torch.zeros(children, batch, dtype=torch.float64, device=cuda)
+    size = want.clone().index_add_(0, cid.long(), term.abs())
+    want.index_add_(0, cid.long(), term)
+    assert ((gc.double() - want).abs() <= 1e-5 * size + 1e-30).all()
