@@ -261,3 +261,31 @@ def test_backward_of_rows_off_the_gradients_grid(cuda, dtype, B, N):
     want = g.double()[:, None] * torch.exp(xs.double() - lse[:, None])
     rel = {"f32": 1e-5, "f16": 2.0 ** -11 + 1e-5, "bf16": 2.0 ** -8 + 1e-5}[dtype]
     assert ((got - want).abs() <= rel * want.abs() + (2.0 ** -25 if dtype == "f16" else 1e-30)).all()
+
+
+@pytest.mark.parametrize("V", [3, 61, 257, 4099])
+@pytest.mark.parametrize("cut", ["step", "overlap", "inner", "one row"])
+def test_selective_slices_of_other_strides(cuda, V, cut):
+    """Slices with more than a row between them (a step over the batch, rows cut at
+    both ends), none (one slice expanded over the batch) and slices of one row:
+    values and gradients through the drop-in against fp64."""
+    import fuselse_amd
+
+    print(f"case sls strides {cut} V={V}", flush=True)
+    rng = np.random.default_rng(V)
+    full = torch.from_numpy((rng.standard_normal((6, 5, V)) * 3).astype(np.float32))
+    take = {"step": lambda t: t[::2], "overlap": lambda t: t[2:3].expand(4, 5, V), "inner": lambda t: t[1:, 1:-1],
+            "one row": lambda t: t[:, :1]}[cut]
+    leaf = full.to(cuda).requires_grad_(True)
+    view = take(leaf)
+    assert not view.is_contiguous()
+    idx = rng.integers(0, V, tuple(view.shape[:-1]))
+    w = rng.standard_normal(idx.shape).astype(np.float32)
+    y = fuselse_amd.selective_log_softmax(view, torch.from_numpy(idx).to(cuda))
+    (grad,) = torch.autograd.grad(y, view, torch.from_numpy(w).to(cuda))
+    rows = np.ascontiguousarray(take(full).numpy()).reshape(-1, V)
+    lse = O.lse_fp64(rows)
+    _check_fwd(y.detach().cpu().numpy().reshape(-1), lse.astype(np.float32), rows, idx.reshape(-1))
+    want = O.selective_logsoftmax_bwd_fp64(w.reshape(-1), rows, idx.reshape(-1), lse)
+    err = np.abs(grad.cpu().numpy().reshape(-1, V) - want)
+    assert (err <= 1e-5 * np.abs(want) + 1e-6 * np.abs(w).reshape(-1, 1)).all(), err.max()

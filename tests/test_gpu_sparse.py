@@ -702,10 +702,10 @@ def _csr_fp64_torch(child, off, cids, lp):
                                          (61, 256), (61, 510), (40001, 3), (20001, 130), (160003, 1), (40001, 200),
                                          (40001, 132)])
 def test_csr_forward_runs(cuda, nodes, batch):
-    """The streamed forward around its column tiles (64, 128, 256 columns, odd
-    batches), run lengths of 1, 2 and 4 nodes and a run cut short, with empty
-    nodes at the run's start, middle and end, groups of every remainder and
-    every chain count of the Q16.16 tree."""
+    """The forward around its column tiles (lane groups of 4 to 32 columns, streams
+    of 64, 128 and 256, odd batches), with empty nodes first, last and between,
+    groups of every remainder and every chain count of the Q16.16 tree; run
+    lengths above 2 are test_csr_forward_run_lengths's."""
     print(f"case csr runs {nodes}x{batch}", flush=True)
     rng = np.random.default_rng(nodes + batch)
     fan = O.powerlaw_fanin(nodes, seed=batch)
@@ -761,10 +761,10 @@ def test_csr_q16_saturated_pairs(cuda, batch):
                                                   (300, 61, 33), (3000, 16, 2), (300, 61, 64), (300, 61, 65), (300, 61, 128),
                                                   (30000, 40001, 3), (20000, 16100, 512), (20000, 22000, 384)])
 def test_csr_backward_runs(cuda, nodes, children, batch):
-    """The streamed backward: one tile (weights and sums by edge id) and, from
-    64000 (child, tile) pairs, several tiles through the workspace; children
-    without edges; twice the same bits.  A sum's error is bounded by 1e-5 of
-    its terms' magnitudes."""
+    """The backward of lane groups (up to 32 columns), of one streamed tile
+    (weights and sums by edge id) and, from 64000 (child, tile) pairs, of several
+    through the workspace; children without edges; twice the same bits.  A sum's
+    error is bounded by 1e-5 of its terms' magnitudes."""
     print(f"case csr bwd runs {nodes} {children} {batch}", flush=True)
     rng = np.random.default_rng(children + batch)
     off, cids, lp = _csr(rng, nodes, children, fanin=np.maximum(O.powerlaw_fanin(nodes, seed=batch), 1))
@@ -1046,3 +1046,73 @@ def test_csr_backward_run_lengths(cuda, children, batch, edges):
     size = want.clone().index_add_(0, cid.long(), term.abs())
     want.index_add_(0, cid.long(), term)
     assert ((gc.double() - want).abs() <= 1e-5 * size + 1e-30).all()
+
+
+@pytest.mark.parametrize("bs,ne,batch", [(4, 40, 68), (16, 40, 68), (32, 40, 68), (32, 32, 64), (16, 16, 128)])
+def test_blocked_layer_gradients_of_pairs_left_out(cuda, bs, ne, batch):
+    """The single pass's one-by-one terms (test_blocked_backward_product_form_pairs_left_out)
+    through the layer's own gradients, with an element row of one edge, which takes
+    them directly, among the children they belong to: the bits of the adding entry
+    over cleared flows."""
+    print(f"case blocked grads left-out pairs bs={bs} ne={ne} batch={batch}", flush=True)
+    from fuselse_amd import pc
+
+    ext = _ext()
+    rng = np.random.default_rng(23)
+    nb, nelem = 3, 2 * ne + 10
+    nids = (np.arange(nb) * bs).astype(np.int64)
+    cids = np.stack([rng.permutation(nelem - 10)[:ne] for _ in range(nb)]).astype(np.int64)
+    cids[2, 0], cids[2, 2] = nelem - 1, nelem - 2  # rows of one edge
+    pids = (np.arange(nb * ne, dtype=np.int64) * bs).reshape(nb, ne)
+    params = (rng.random(nb * ne * bs) + 1e-3).astype(np.float32)
+    em = np.log(rng.random((nelem, batch)) + 1e-9).astype(np.float32)
+    params[pids[2, :] + bs - 2] = 1e-36
+    params[pids[2, 0] + bs - 2] = 1.0
+    params[pids[2, 1] + bs - 2] = 0.0
+    em[:, 20:30] = -60.0
+    em[cids[2, 0], 20:30] = -200.0
+    em[cids[2, 1], 20:30] = 0.0
+    em[cids[2, 2], 20:30] = -1.0
+    em[:, 40] = -np.inf
+    with np.errstate(divide="ignore"):
+        lw = np.log(params)
+    num_nodes = nb * bs + 2
+    d_em, d_lw, d_n, d_c, d_p = _to(cuda, em, lw, nids, cids, pids)
+    g = torch.from_numpy(rng.standard_normal((num_nodes, batch)).astype(np.float32)).to(cuda)
+    plan = ext.sparse_blocked_transpose(d_n, d_c, d_p, bs, nelem)
+    counts = plan.csc_offsets.diff()
+    assert int(counts[nelem - 1]) == 1 and int(counts[nelem - 2]) == 1 and int(counts.max()) > 1
+    e, w = d_em.clone().requires_grad_(True), d_lw.clone().requires_grad_(True)
+    y = pc.sparse_blocked_layer(e, w, d_n, d_c, d_p, bs, num_nodes, plan=plan)
+    de, dw = torch.autograd.grad(y, (e, w), g)
+    ge, gp = torch.zeros_like(d_em), torch.zeros_like(d_lw)
+    ext.sparse_blocked_backward(g, ge, y.detach(), d_em, d_lw, gp, d_n, d_c, d_p, bs, params_are_log=True, plan=plan)
+    assert torch.equal(de, ge) and torch.equal(dw, gp)
+    # in these columns the left-out parent's whole flow goes to a row of one edge
+    rows = slice(2 * bs, 3 * bs)
+    t = np.exp(lw[pids[2, 2]:pids[2, 2] + bs, None].astype(np.float64) + em[cids[2, 2]] - y.detach().cpu().numpy()[rows])
+    terms = (t * g.cpu().numpy()[rows])[:, 20:30]
+    np.testing.assert_allclose(t[bs - 2, 20:30], 1.0, rtol=1e-4)
+    err = np.abs(de[nelem - 2, 20:30].cpu().numpy() - terms.sum(0))
+    assert (err <= 1e-5 * np.abs(terms).sum(0)).all(), err.max()
+
+
+def test_csr_backward_workspace_past_the_streams_edges(cuda):
+    """The workspace form with a child of more edges than a run's 32-bit edge
+    numbers are for (2^20), among children of a few and of none: sums of ones, exact
+    in fp32."""
+    big, children, batch = (1 << 20) + 7, 40000, 256
+    print(f"case csr bwd workspace long run {big}", flush=True)
+    from fuselse_amd import _lib
+
+    cid = torch.ones(big + 3, dtype=torch.int32, device=cuda)
+    cid[-3:] = torch.tensor([0, 4, 4])
+    off = torch.arange(big + 4, device=cuda)
+    assert _lib.load().fl_sparse_csr_bwd_workspace_bytes(children, big + 3, batch) > 0
+    ch = torch.zeros(children, batch, device=cuda)
+    lp = torch.zeros(big + 3, device=cuda)
+    out = torch.zeros(big + 3, batch, device=cuda)
+    gc, gl = _ext().sparse_csr_backward(ch, out, torch.ones_like(out), off, cid, lp)
+    want = torch.zeros(children, device=cuda)
+    want[0], want[1], want[4] = 1.0, float(big), 2.0
+    assert torch.equal(gc, want[:, None].expand(children, batch)) and torch.equal(gl, torch.full_like(gl, float(batch)))
