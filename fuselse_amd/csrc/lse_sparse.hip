@@ -13,7 +13,7 @@
 // child row.
 //
 // Mapping.  CSR layers: csr_fwd_narrow, several nodes per wave, up to 32
-// columns; csr_fwd_kernel, a wave per run of nodes and tile of 64 or 128
+// columns; csr_fwd_kernel, a wave per run of nodes and tile of 64, 128 or 256
 // columns, its edges one stream.  The block layout (and some Q16.16 CSR
 // layers): sparse_kernel, one wave per (node, tile of 64, 128 or 256 columns);
 // lane l owns 1, 2 or 4 columns (one vector when the batch is a multiple of it
@@ -192,7 +192,7 @@ struct BlockLayout {
 };
 
 // ---------------------------------------------------------------------------
-// Per-node reductions over one 256-column tile.
+// Per-node reductions over one tile of 64 * PP columns.
 // ---------------------------------------------------------------------------
 // The columns of lane l (as Cols<VW, PP>) from the row segment starting at b0
 // (`row` points at it), through a buffer resource of `rec` bytes: columns past
@@ -366,7 +366,7 @@ __device__ __forceinline__ void reduce_q16(const LAYOUT& L, const DESC& d, const
         reduce_q16_et<8, VW, P>(L, d, first, child, batch, b0, l, lut);
 }
 
-// One single-wave block per (node, 256-column tile) pair, pairs numbered
+// One single-wave block per (node, tile of 64 * P columns) pair, pairs numbered
 // tile-fastest from pair0.  A block lives exactly as long as its own node's
 // edge loop: with four nodes per block, a block held its slot until the
 // largest of four power-law fan-ins was done, and the Q16 table needed a block
@@ -1099,14 +1099,15 @@ static bool wide_tiles_fit(int64_t batch) { return (batch + 127) / 128 == 2 * ((
 //
 // From some thousand (node, 128-column tile) pairs on, the waves are more than
 // the GPU holds at once, and a short node is a wave's fixed cost; up to 40000,
-// where longer runs begin, half as many waves of 256 columns, or where these do
-// not fit and in Q16.16 of two nodes, take less.  Below, the longest node's chain
-// is the time, and a wave for it alone is fastest.  us at 2 / 5 / 16 / power-law
-// edges a node, one node and 128 columns a wave -> this: 8000 nodes, batch 512,
-// fp32 15.0 / 18.8 / 31.0 / 40.3 -> 10.0 / 15.9 / 27.6 / 43.4, Q16.16 15.9 / 20.2 /
-// 36.8 / 60.7 -> 12.7 / 19.2 / 34.5 / 61.3; 8000 x 300, fp32 12.5 / 15.5 / 24.3 /
-// 35.6 -> 9.9 / 14.9 / 23.5 / 37.2; 2000 x 256 4.7 / 5.3 / 7.3 / 22.4 against 4.0 /
-// 4.6 / 6.1 / 26.4 with 256 columns.
+// where longer runs begin, half as many waves in fp32, of 256 columns or where
+// these do not fit of two nodes, take less.  Below, the longest node's chain is the
+// time, and a wave for it alone is fastest, as in Q16.16, whose chains are longer.
+// us at 2 / 5 / 16 / power-law edges a node, one node and 128 columns a wave ->
+// this: 8000 nodes, batch 512, 15.0 / 18.8 / 31.0 / 40.3 -> 10.0 / 15.9 / 27.6 / 43.4;
+// 8000 x 300 12.5 / 15.5 / 24.3 / 35.6 -> 9.9 / 14.9 / 23.5 / 37.2; not 2000 x 256,
+// 4.7 / 5.3 / 7.3 / 22.4 against 4.0 / 4.6 / 6.1 / 26.4 with 256 columns, nor Q16.16,
+// 14000 x 256, 14.0 / 18.0 / 32.8 / 56.1 against 11.2 / 17.3 / 31.1 / 66.9 with two
+// nodes.
 //
 // Up to 4 columns, 4 lanes a node; of fewer than 4000 nodes 8, as fan-ins past
 // kOwnEdges are then the time, and 16 nodes' worth of them queue in one wave (us,
@@ -1155,7 +1156,7 @@ static void launch_csr(const CsrLayout& L, const float* child, int64_t nodes, hi
             launch_csr_cols<false, 1, 4>(L, child, nodes, npw, !large, st);
         return;
     }
-    const int npw = batch > 128 && brief && pairs >= (Q16 ? 12000 : 6000) ? 2 : run_nodes(pairs);
+    const int npw = !Q16 && batch > 128 && brief && pairs >= 8000 ? 2 : run_nodes(pairs);
     if (batch % 2 == 0 && (at & 7) == 0)
         launch_csr_cols<Q16, 2, 2>(L, child, nodes, npw, brief, st);
     else
