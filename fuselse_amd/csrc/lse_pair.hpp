@@ -25,8 +25,9 @@ constexpr uint32_t kQBias = 0x80000000u;
 // read, six of them in the chain with it; max, min, their difference, its
 // halves and a two-instruction table offset took ten, eight in the chain.  The
 // block-layout layer of 2048 x 32 nodes, 32 edges, batch 512, whose time this
-// is, went from 472 to 421 us; rows of (512, 128256) fp32 went from 40.3 to 39.9,
-// of (16384, 1000) from 20.1 to 18.9, of (65536, 256) from 62.9 to 59.9.
+// is, went from 472 to 421 us; rows of (16384, 1000) fp32 went from 20.1 to 18.9,
+// of (65536, 256) from 62.9 to 59.9 (a block per row); (512, 128256), at its memory
+// bound, did not change.
 template <bool USE_LUT>
 __device__ __forceinline__ uint32_t q16_pair(uint32_t a, uint32_t b, const int* __restrict__ lut) {
     const uint32_t hi = a > b ? a : b;

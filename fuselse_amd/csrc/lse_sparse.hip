@@ -423,8 +423,8 @@ static void launch(const LAYOUT& L, const float* child, const float* out_any, in
 }
 
 // ---------------------------------------------------------------------------
-// CSR forward: one wave per run of `npw` consecutive nodes and tile of 64 or
-// 128 columns, walking the run's edges as one stream of groups of up to G edges
+// CSR forward: one wave per run of `npw` consecutive nodes and tile of 64 * P
+// columns, walking the run's edges as one stream of groups of up to G edges
 // (a group never spans two nodes).  The next group's rows are in flight while
 // a group folds, across node boundaries too, and the group after that has its
 // edge ids and weights on the way through scalar loads, so a node costs no
@@ -432,10 +432,9 @@ static void launch(const LAYOUT& L, const float* child, const float* out_any, in
 // (offsets, ids, rows).  The tiles go one after the other over all runs, so
 // that at any time the gathers stay within one column slice of the children,
 // of which the 256 MB Infinity Cache holds a part: a 1M-row, 512-column layer
-// gathers 7.3 TB/s from random rows in slices where it took 5.9 in whole rows.
-// The layer (8.0M edges, fan-in k^-2 on [2, 256]) went from 3140 to 2554 us in
-// fp32 and to 2595 in Q16.16 (wave per node and 256-column tile, tile-fastest
-// -> this); the gathers alone, with the same stores, take 2354.
+// (8.0M edges to random rows, fan-in k^-2 on [2, 256], 18.5 GB) went from 3140 us,
+// 5.9 TB/s, to 2548 in fp32 and 2599 in Q16.16, 7.3 and 7.1 TB/s (wave per node and
+// 256-column tile, tile-fastest -> this).
 // ---------------------------------------------------------------------------
 // Scalar loads of 4 consecutive words through a buffer resource: words past
 // its range read as 0.
@@ -1183,7 +1182,7 @@ static void launch_csr(const CsrLayout& L, const float* child, int64_t nodes, hi
 // in a workspace, and csr_bwd_sums adds the tiles' sums in tile order and
 // scatters them.  DIRECT, a single tile, takes them where they are and spares
 // two launches.  The summation order is fixed either way.  The 1M-child,
-// 8.0M-edge layer at batch 512 went from 6160 to 5316 us (two gathered rows an
+// 8.0M-edge layer at batch 512 went from 6160 to 5270 us (two gathered rows an
 // edge, 33 GB; a wave per child over whole rows -> this); 200000 x 64 columns,
 // DIRECT, from 265 to 169.
 // ---------------------------------------------------------------------------
@@ -1540,9 +1539,8 @@ struct ParentMeta {
 
 constexpr int PB = 8;  // columns per lane
 // Parent edges per load group (two rows each), and columns per lane: 8 columns
-// and single-edge groups measured 7.2 ms on the 1M-node C5 layer, against
-// 7.8 ms for 4 columns and two-edge groups; the forward keeps 4 columns (8
-// measured 3.8 ms against 3.45 ms).
+// and single-edge groups measured 7.2 ms on the 1M-node layer of 8.0M edges,
+// batch 512, against 7.8 ms for 4 columns and two-edge groups.
 constexpr int GB = 1;
 
 template <int VW>
