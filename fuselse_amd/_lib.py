@@ -58,7 +58,7 @@ SIGNATURES = {
     "fl_sparse_csr_bwd_ws": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp,
                                     ctypes.c_size_t, _vp]),
     "fl_sparse_blocked_fwd": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _int, _vp]),
-    "fl_sparse_blocked_clear": (_int, [_vp, _vp, _i64, _i64, _i64, _vp]),
+    "fl_sparse_blocked_fwd_fresh": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _int, _vp]),
     "fl_sparse_blocked_bwd": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _int, _vp, _vp,
                                      _i64, _vp, _vp, _vp, _vp]),
     "fl_sparse_blocked_grad": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _int, _int, _vp,

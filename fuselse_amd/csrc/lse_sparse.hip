@@ -1764,22 +1764,6 @@ extern "C" int fl_sparse_csr_fwd(const float* child, const int64_t* offsets, con
     return launch_status(name);
 }
 
-extern "C" int fl_sparse_blocked_clear(float* node_mars, const int64_t* nids, int64_t num_nblocks, int64_t block_size,
-                                       int64_t batch, void* stream) {
-    const char* name = "fl_sparse_blocked_clear";
-    FL_CHECK(num_nblocks >= 0 && block_size >= 0 && batch >= 0, "%s: negative size", name);
-    if (num_nblocks == 0 || block_size == 0 || batch == 0) return ok();
-    FL_CHECK(node_mars && nids, "%s: NULL pointer argument", name);
-    // a wave per block up to 16384 waves, then a few blocks each
-    const int64_t share = (num_nblocks + 16383) / 16384;
-    const int per = (int)(share < 64 ? share : 64);
-    for_grid_chunks((num_nblocks + 4 * per - 1) / (4 * per), 256, [&](int64_t b0, int64_t n) {
-        sparse::block_clear_rows<<<dim3((unsigned)n), dim3(256), 0, reinterpret_cast<hipStream_t>(stream)>>>(
-            node_mars, nids, num_nblocks, block_size, batch, per, b0);
-    });
-    return launch_status(name);
-}
-
 extern "C" int fl_sparse_blocked_fwd(float* node_mars, const float* element_mars, const float* params,
                                      const int64_t* nids, const int64_t* cids, const int64_t* pids, int64_t num_nblocks,
                                      int64_t num_edges, int64_t block_size, int64_t batch, int q16, int params_are_log,
@@ -1806,4 +1790,23 @@ extern "C" int fl_sparse_blocked_fwd(float* node_mars, const float* element_mars
         else sparse::launch_block<false>(L, element_mars, items, st);
     }
     return launch_status(name);
+}
+
+extern "C" int fl_sparse_blocked_fwd_fresh(float* node_mars, const float* element_mars, const float* params,
+                                           const int64_t* nids, const int64_t* cids, const int64_t* pids,
+                                           int64_t num_nblocks, int64_t num_edges, int64_t block_size, int64_t batch,
+                                           int q16, int params_are_log, void* stream) {
+    // sizes and pointers that the forward refuses launch nothing
+    if (num_nblocks > 0 && num_edges >= 0 && block_size > 0 && batch > 0 && node_mars && element_mars && params && nids &&
+        (num_edges == 0 || (cids && pids))) {
+        // a wave per block up to 16384 waves, then a few blocks each
+        const int64_t share = (num_nblocks + 16383) / 16384;
+        const int per = (int)(share < 64 ? share : 64);
+        for_grid_chunks((num_nblocks + 4 * per - 1) / (4 * per), 256, [&](int64_t b0, int64_t n) {
+            sparse::block_clear_rows<<<dim3((unsigned)n), dim3(256), 0, reinterpret_cast<hipStream_t>(stream)>>>(
+                node_mars, nids, num_nblocks, block_size, batch, per, b0);
+        });
+    }
+    return fl_sparse_blocked_fwd(node_mars, element_mars, params, nids, cids, pids, num_nblocks, num_edges, block_size,
+                                 batch, q16, params_are_log, stream);
 }

@@ -521,31 +521,32 @@ def _sparse_blocked(node_mars, element_mars, params, nids, cids, pids, block_siz
     batch = node_mars.size(1)
     num_nblocks = nids.size(0)
     num_edges = cids.size(1)
-    if written_rows is not None:
-        _clear_unwritten(node_mars, nids, int(block_size), written_rows)
+    entry = "fl_sparse_blocked_fwd"
+    if written_rows is not None and _clear_unwritten(node_mars, num_nblocks * int(block_size), written_rows):
+        entry = "fl_sparse_blocked_fwd_fresh"
     if batch == 0 or num_nblocks == 0 or block_size == 0:
         return None
     with _on_device(node_mars):
-        _lib.call("fl_sparse_blocked_fwd", node_mars.data_ptr(), element_mars.data_ptr(), params.data_ptr(),
+        _lib.call(entry, node_mars.data_ptr(), element_mars.data_ptr(), params.data_ptr(),
                   nids.data_ptr(), cids.data_ptr(), pids.data_ptr(), num_nblocks, num_edges, int(block_size), batch,
                   int(q16), int(params_are_log), _stream(node_mars))
     return None
 
 
-def _clear_unwritten(node_mars, nids, block_size, written_rows):
-    """-inf into the rows that this layer's blocks will not write.
-    written_rows: a plan's word that they write the rows [0, written_rows) in
-    order (0: not known).  The plan may be another layer's, or older than a
-    change of nids, so these rows are left out only where this call's own sizes
-    and, on the device, its nids say the same."""
-    if not (written_rows == nids.size(0) * block_size <= node_mars.size(0)):
-        written_rows = 0
-    if written_rows < node_mars.size(0):
-        node_mars[written_rows:].fill_(float("-inf"))
-    if written_rows and node_mars.size(1):
-        with _on_device(node_mars):
-            _lib.call("fl_sparse_blocked_clear", node_mars.data_ptr(), nids.data_ptr(), nids.size(0), block_size,
-                      node_mars.size(1), _stream(node_mars))
+def _clear_unwritten(node_mars, rows, written_rows):
+    """-inf into the rows of an uninitialised node_mars that a layer of `rows`
+    rows in its blocks will not write; whether its launch has to be the one that
+    compares nids and clears the rest.  written_rows: a plan's word that the blocks
+    write the rows [0, written_rows) in order (0: not known).  The plan may be
+    another layer's, or older than a change of nids, so these rows are left out only
+    where this call's own sizes and, on the device, its nids say the same."""
+    total = node_mars.size(0)
+    if written_rows and written_rows == rows <= total:
+        if written_rows < total:
+            node_mars[written_rows:].fill_(float("-inf"))
+        return True
+    node_mars.fill_(float("-inf"))
+    return False
 
 
 def sparse_forward_float(node_mars, element_mars, params, nids, cids, pids, block_size, params_are_log=False):

@@ -235,14 +235,16 @@ int fl_sparse_blocked_fwd(float* node_mars, const float* element_mars, const flo
                           int64_t block_size, int64_t batch, int q16, int params_are_log, void* stream);
 
 /* ---------------------------------------------------------------------------
- * For a caller that hands fl_sparse_blocked_fwd rows it has not initialised:
- * -inf into the rows [j * block_size, (j + 1) * block_size) of every block j
- * with nids[j] != j * block_size.  Blocks that lie in order from row 0 on write
- * these rows in full; then nothing is written here.  node_mars holds at least
- * num_nblocks * block_size rows.
+ * fl_sparse_blocked_fwd for rows that hold anything: first -inf goes into the
+ * rows [j * block_size, (j + 1) * block_size) of every block j with
+ * nids[j] != j * block_size.  Blocks that lie in order from row 0 on write these
+ * rows in full, and nothing is cleared.  node_mars holds at least num_nblocks *
+ * block_size rows; rows past these are left alone.
  * ------------------------------------------------------------------------- */
-int fl_sparse_blocked_clear(float* node_mars, const int64_t* nids, int64_t num_nblocks, int64_t block_size,
-                            int64_t batch, void* stream);
+int fl_sparse_blocked_fwd_fresh(float* node_mars, const float* element_mars, const float* params,
+                                const int64_t* nids, const int64_t* cids, const int64_t* pids, int64_t num_nblocks,
+                                int64_t num_edges, int64_t block_size, int64_t batch, int q16, int params_are_log,
+                                void* stream);
 
 /* ---------------------------------------------------------------------------
  * Sparse CSR backward ("flows"; the reference has no backward for its sparse
